@@ -138,19 +138,39 @@ constexpr int kTrsvMaxWidth = 20;  // widest factor row the pipelined kernel tak
 
 struct DevTrsv {
   int nblocks = 0, nloc = 0, max_rows = 0, max_steps = 0, max_width = 0;
-  int window = 0;  // ring size when the packed columns are ring slots, else 0
-  int64_t nnz_padded = 0, nnz_real = 0, nrows_total = 0;
-  int64_t max_block_ent = 0, max_block_steps = 0;  // largest entry and step counts of one block
-  DevMem row0, step, stepU, ent0, ri0, desc, ent, ri;
-  // Half steps for the one-wave ring kernel (64 threads, 4 lanes per row, 16
-  // rows per pass) over the same ring packing: a step of more than 16 rows is
-  // walked as two consecutive half steps (rows 0-15, then 16-31).  Rows of a
-  // step are independent, and a half step reads and writes a subset of its
-  // step's positions, so the ring window still holds.
+  int window = 0;  // ring rows when the packed columns are ring slots, else 0
+  int64_t nnz_real = 0;
+  int64_t max_block_steps = 0;  // most steps of one block
+  DevMem row0, step, stepU, ri0;
+  // levels solved by the pipelined and direct kernels
+  DevMem ent0, desc, ent, ri;
+  // ring-packed levels: step boundaries, lane records, (slot, row id) pairs and
+  // 1/pivots by position (layouts at k_trsv_ring)
+  DevMem pos, rec, info, dinv;
+  int64_t positions = 0;
+  // half steps: a step of more than 16 rows walked as two consecutive ones (rows
+  // 0-15, then 16-31).  Rows of a step are independent, and a half step reads
+  // and writes a subset of its step's positions, so the window still holds.
   int64_t max_block_steps_h = 0;
-  DevMem step_h, stepU_h, desc_h;
+  DevMem step_h, stepU_h, pos_h;
 };
 
+// Step boundaries of every block (layout at k_trsv_ring) from the step
+// descriptors (desc: 4 per step, the first position at 0 and the rows at 2).
+std::vector<int> step_bounds(const std::vector<int>& desc, const std::vector<int>& blk_step) {
+  const int nb = (int)blk_step.size() - 1;
+  std::vector<int> pos((size_t)blk_step[nb] + nb);
+  for (int b = 0; b < nb; ++b) {
+    int* q = pos.data() + blk_step[b] + b;
+    int end = 0;
+    for (int s = blk_step[b]; s < blk_step[b + 1]; ++s) {
+      *q++ = desc[4 * s];
+      end = desc[4 * s] + desc[4 * s + 2];
+    }
+    *q = end;
+  }
+  return pos;
+}
 
 template <typename V, typename T>
 void upload_trsv(DevTrsv& d, const TrsvPack<T>& P, int64_t* counter) {
@@ -160,39 +180,68 @@ void upload_trsv(DevTrsv& d, const TrsvPack<T>& P, int64_t* counter) {
   d.max_steps = P.max_steps;
   d.max_width = P.max_width;
   d.window = P.window;
-  d.nnz_padded = (int64_t)P.col.size();
   d.nnz_real = P.nnz_real;
-  d.nrows_total = (int64_t)P.rows.size();
-  d.max_block_ent = d.max_block_steps = 0;
-  for (int b = 0; b < P.nblocks; ++b) {
-    d.max_block_ent = std::max<int64_t>(d.max_block_ent, P.blk_ent0[b + 1] - P.blk_ent0[b]);
+  d.max_block_steps = 0;
+  for (int b = 0; b < P.nblocks; ++b)
     d.max_block_steps = std::max<int64_t>(d.max_block_steps, P.blk_step[b + 1] - P.blk_step[b]);
-  }
   upload(d.row0, P.blk_row0, counter);
   upload(d.step, P.blk_step, counter);
   upload(d.stepU, P.blk_stepU, counter);
-  upload(d.ent0, P.blk_ent0, counter);
   upload(d.ri0, P.blk_ri0, counter);
-  upload(d.desc, P.desc, counter);
-  d.max_block_steps_h = 0;
-  int step_rows = 0;
-  for (size_t i = 2; i < P.desc.size(); i += 4) step_rows = std::max(step_rows, P.desc[i]);
-  if (P.window > 0 && step_rows <= 32) {
+  const int64_t nr = (int64_t)P.rows.size();
+  if (P.window > 0) {
+    upload(d.pos, step_bounds(P.desc, P.blk_step), counter);
     std::vector<int> dh, sh, suh;
     half_steps(P.desc, P.blk_step, P.blk_stepU, dh, sh, suh);
+    d.max_block_steps_h = 0;
     for (int b = 0; b < P.nblocks; ++b)
       d.max_block_steps_h = std::max<int64_t>(d.max_block_steps_h, sh[b + 1] - sh[b]);
-    upload(d.desc_h, dh, counter);
     upload(d.step_h, sh, counter);
     upload(d.stepU_h, suh, counter);
+    upload(d.pos_h, step_bounds(dh, sh), counter);
+    // the packed slots are positions modulo a power of two; the device's ring
+    // holds just the window's rows (a fifth less LDS at 128^3: room for more
+    // columns or stages): slot = position modulo the window
+    const int W = P.window, wn = std::max(P.window_needed, 1);
+    if (wn > 0xffff) throw std::runtime_error("sweep window too large for 16-bit slots");
+    d.window = wn;
+    d.positions = nr;
+    constexpr int RB = ring_row_bytes<V>();
+    std::vector<unsigned char> rec((size_t)nr * RB);
+    std::vector<int2> info((size_t)nr + 1);
+    info[nr] = int2{wn * (int)sizeof(V), kRingDummyRow};
+    parallel_for(P.nblocks, [&](int b) {
+      for (int s = P.blk_step[b]; s < P.blk_step[b + 1]; ++s) {
+        const int* d4 = &P.desc[4 * (size_t)s];
+        const int end = d4[0] + d4[2];  // a row the step reads is at most W positions before it
+        for (int t = 0; t < d4[2]; ++t) {
+          const int64_t q = P.blk_ri0[b] + d4[0] + t;
+          info[q] = int2{(d4[0] + t) % wn * (int)sizeof(V), P.rows[q]};
+          const int t0 = t / kRingGroup * kRingGroup;  // first row of t's group
+          unsigned char* g = rec.data() + (P.blk_ri0[b] + d4[0] + t0) * RB;
+          for (int j = 0; j < d4[3]; ++j) {
+            const int64_t e = P.blk_ent0[b] + d4[1] + (int64_t)t * d4[3] + j;
+            // (padded entries weigh zero, whatever row they name)
+            const int p = std::max(0, end - 1 - ((end - 1 - P.col[e]) & (W - 1)));
+            store_rec<V>(g, std::min(kRingGroup, d4[2] - t0), t - t0, j, hval<V>(P.val[e]), (unsigned)(p % wn));
+          }
+        }
+      }
+    });
+    upload(d.rec, rec, counter);
+    upload(d.info, info, counter);
+    upload(d.dinv, convert_vec<V>(P.dinv), counter);
+    return;
   }
+  upload(d.ent0, P.blk_ent0, counter);
+  upload(d.desc, P.desc, counter);
   std::vector<TPair<V>> ent(P.col.size() + 1), ri(P.rows.size() + 1);
   constexpr int64_t kChunk = 1 << 20;
-  const int64_t ne = (int64_t)P.col.size(), nr = (int64_t)P.rows.size();
+  const int64_t ne = (int64_t)P.col.size();
   parallel_for((int)((ne + kChunk - 1) / kChunk), [&](int c) {
     for (int64_t i = c * kChunk, i1 = std::min(ne, (c + 1) * kChunk); i < i1; ++i) {
       ent[i] = TPair<V>();
-      ent[i].col = P.window > 0 ? P.col[i] * ring_unit<V>() : P.col[i];  // ring slots as 4-column row offsets
+      ent[i].col = P.col[i];
       ent[i].val = hval<V>(P.val[i]);
     }
   });
@@ -232,19 +281,13 @@ struct pgs_dev_op_s {
   int is_complex = 0;
   int lds_max = 65536;
   int trsv_variant = 0;  // 0: pipelined kernels (ring when packed for it); 1: basic level-set kernel
-  // most right-hand-side columns per column group of the ring kernel; 0 =
-  // chosen per launch (4, or 8 for 4-byte values once 4 would give four or
-  // more workgroups per CU)
+  // most right-hand-side columns per workgroup of the ring kernel; 0 = chosen per
+  // launch
   int trsv_cg = 0;
-  int trsv_groups = 1;   // column groups per workgroup of the 128-thread ring kernel: 1, 2, or 0 = 2 when
-                         // the paired grid fills the device (measured slower at 128^3: kept selectable)
   int num_cus = 256;     // compute units of the device
   int trsv_nt = 128;     // threads of the pipelined kernel
   int trsv_lpr = 4;      // lanes per row (steps hold at most trsv_nt / trsv_lpr rows)
-  // ring kernel geometry: 0 = chosen per launch (128x4 or one-wave 64x4 on
-  // half steps); 128 / 64 with ring_lpr 4 or 2 force one geometry
-  int ring_nt = 0;
-  int ring_lpr = 4;
+  int ring_nt = 0;       // ring kernel on whole steps (128) or half steps (64): 0 = chosen per launch
   int lr_mfma = 1;          // low-rank term of FP32 blocks of 16, 32 or 64 columns on the matrix cores
   int usolve = 0;           // 1: the U variant of SolveLevel (no block L solve on the way down)
   int inner_maxits = 0;     // > 0: inner FGMRES on the level-0 Schur complement in every apply
@@ -463,117 +506,92 @@ void launch_trsv_pipe(int nt, int lpr, const DevTrsv& T, const V* rhs, V* x, int
   }
 }
 
-// Ring kernel geometries: rows of at most kRingWidth entries, LPR lanes per
-// row with kRingWidth / LPR slots each; 128 threads and 4 lanes per row (steps
-// of at most 32 rows), or one wave of 64 threads with 4 lanes (16 rows) or 2
-// lanes (32 rows) per row.
+// Ring kernel: rows of at most kRingWidth entries, steps of at most 32 rows.
 constexpr int kRingWidth = 20;
 
-// Stage depth of the ring kernel's register ring (steps whose entries are in
-// flight): the deepest ring whose registers stay within 256 VGPRs, so that
-// two waves fit on a SIMD and no stage is moved to AGPRs (a moved stage costs
-// register copies that wait for loads in flight).  With 4 lanes per row:
-// float 12 (8 for 8-column groups), 8-byte values 6, complex<double> 4; lane
-// pairs hold twice the slots per lane: 6 / 4 / 2.
-template <typename V, int CG, int LPR = 4>
+// Steps whose records are in LDS or on the way there: enough that a copy has
+// K - 2 steps to arrive (1 to 2 us), within the 63 copies that can be waited for
+// apart.  8 to 14 stages of 4-byte values and 6 to 10 of 8-byte ones measured
+// within 3 % of each other.
+template <typename V>
 constexpr int ring_depth() {
-  if constexpr (LPR == 2) return sizeof(V) == 4 ? 6 : sizeof(V) == 8 ? 4 : 2;
-  return sizeof(V) == 4 ? (CG == 8 ? 8 : 12) : sizeof(V) == 8 ? 6 : 4;
+  return sizeof(V) == 4 ? 10 : sizeof(V) == 8 ? 8 : 6;
 }
 
-template <typename V, int NT, int LPR, int CG, int G = 1>
-void launch_trsv_ring_cg(const DevTrsv& T, const V* rhs, V* x, int nrhs, hipStream_t s) {
-  constexpr int D = ring_depth<V, CG, LPR>();
-  auto kern = k_trsv_ring<V, NT, LPR, kRingWidth / LPR, D, CG, G>;  // LDS limit raised in set_kernel_attrs
-  const size_t lds = (size_t)(T.window + 1) * CG * G * sizeof(V);  // a ring + dummy slot per group
-  const unsigned grid = (unsigned)T.nblocks * (unsigned)(nrhs / (CG * G));
-  // 64 threads with 4 lanes per row take 16 rows per pass: they walk the half steps
-  const bool half = NT / LPR < 32;
-  const DevMem& step = half ? T.step_h : T.step;
-  const DevMem& stepU = half ? T.stepU_h : T.stepU;
-  const DevMem& desc = half ? T.desc_h : T.desc;
-  kern<<<grid, NT * G, lds, s>>>(T.nblocks, T.window - 1, T.row0.as<int>(), step.as<int>(), stepU.as<int>(),
-                                 T.ent0.as<int64_t>(), T.ri0.as<int64_t>(), desc.as<int4>(),
-                                 T.ent.as<TPair<V>>(), T.ri.as<TPair<V>>(), rhs, x, nrhs);
+template <typename V, int K, int CG, int NG, int NH>
+void launch_trsv_ring_k(const DevTrsv& T, const V* rhs, V* x, int nrhs, hipStream_t s) {
+  auto kern = k_trsv_ring<V, K, CG, NG, NH>;  // LDS limit raised in set_kernel_attrs
+  const size_t lds = RingLds<V, CG, NG, NH>::bytes(T.window, K);
+  const unsigned grid = (unsigned)T.nblocks * (unsigned)(nrhs / (CG * NG));
+  const DevMem& step = NH == 1 ? T.step_h : T.step;
+  const DevMem& stepU = NH == 1 ? T.stepU_h : T.stepU;
+  const DevMem& pos = NH == 1 ? T.pos_h : T.pos;
+  kern<<<grid, 64 * (NH * NG + 2), lds, s>>>(T.nblocks, T.window, T.row0.as<int>(), step.as<int>(), stepU.as<int>(),
+                                             T.ri0.as<int64_t>(), pos.as<int>(), T.rec.as<unsigned char>(),
+                                             T.info.as<int2>(), T.dinv.as<V>(), rhs, x, nrhs);
 }
 
 template <typename V>
 void launch_trsv_ring(pgs_dev_op_s* op, const DevTrsv& T, const V* rhs, V* x, int nrhs, hipStream_t s) {
-  // the kernel addresses a block's rows of all columns, its entries and its
-  // step descriptors with 32-bit byte offsets; lanes with nothing to store
-  // aim at offset 0x7ffffff0, which must stay past the block's vector; lanes
-  // past a step's rows read up to 32 rows' slabs beyond the step
-  if ((int64_t)T.max_rows * nrhs * (int64_t)sizeof(V) > (int64_t)0x7ffffff0 ||
-      (T.max_block_ent + 32 * kRingWidth + 1) * (int64_t)sizeof(TPair<V>) >= (int64_t)INT32_MAX ||
-      (std::max(T.max_block_steps, T.max_block_steps_h) + 64) * 16 >= (int64_t)INT32_MAX)
+  // the kernel addresses a block's rows of all columns, its records (two
+  // positions per row) and its step boundaries with 32-bit byte offsets; lanes
+  // with nothing to load or store aim at offset kRingOut, which must stay past
+  // each of them
+  if ((int64_t)T.max_rows * nrhs * (int64_t)sizeof(V) > (int64_t)kRingOut ||
+      2 * (int64_t)T.max_rows * ring_row_bytes<V>() > (int64_t)kRingOut || (T.positions + 1) * 8 > (int64_t)kRingOut ||
+      (T.max_block_steps + 64) * 4 > (int64_t)kRingOut)
     throw std::runtime_error("diagonal block too large for 32-bit offsets");
   if (nrhs <= 0 || (nrhs & (nrhs - 1)) != 0)
     throw std::runtime_error("the ring solve takes a power-of-two number of columns");
-  int cg = std::min(nrhs, op->trsv_cg > 0 ? op->trsv_cg : 4);
-  // Below one workgroup per CU each group's step chain is the bound, and a
-  // narrower group has shorter steps: spread the columns over as many groups
-  // as there are CUs (measured at 128^3 level 0, FP32: 4 RHS with 4 columns
-  // per group 0.93 ms, with 1 column per group on 256 workgroups ~0.75 ms).
+  constexpr int KB = ring_depth<V>();
+  constexpr int CMAX = sizeof(V) == 4 ? 16 : sizeof(V) == 8 ? 8 : 4;
+  // A workgroup takes as many columns as its rings and registers hold, since its
+  // columns share the records; but below one workgroup per CU the step chain is
+  // the bound and fewer columns have shorter steps, so the columns are spread
+  // over as many workgroups as there are CUs.
+  int c = std::min({nrhs, CMAX, op->trsv_cg > 0 ? op->trsv_cg : CMAX});
   if (op->trsv_cg == 0)
-    while (cg > 1 && (int64_t)T.nblocks * (nrhs / cg) * 2 <= (int64_t)op->num_cus) cg >>= 1;
-  // Eight columns per group halve the per-column loads, address arithmetic
-  // and reductions but lengthen each step.  They pay when four-column groups
-  // would put four or more one-wave workgroups on every CU, and at two per
-  // CU when the half steps make a block's chain half again as long as its
-  // whole steps (level sets of more than 16 rows), so that 8-column groups
-  // of 128 threads on whole steps shorten it.  Measured at 128^3, FP32, ms
-  // per launch: level 0 (6,300 half against 3,350 whole steps) at 32 RHS
-  // 1.19 with 8-column groups of 128 threads against 1.31 with 4-column
-  // one-wave groups, at 64 RHS 1.59 with 8-column one-wave groups against
-  // 3.14 with 4 (2.06 with 8 columns and 128 threads), at 16 RHS 0.85 with
-  // 4 columns against 1.18 with 8; level 1 (800 half against 700 whole
-  // steps) at 32 RHS 0.16 with 4-column one-wave groups against 0.24.
-  if (op->trsv_cg == 0 && sizeof(V) == 4 && nrhs >= 8) {
-    const int64_t g4 = (int64_t)T.nblocks * (nrhs / 4);
-    const bool long_halves = T.desc_h.p && 2 * (int64_t)T.max_block_steps_h >= 3 * (int64_t)T.max_block_steps;
-    if (g4 >= 4 * (int64_t)op->num_cus || (g4 >= 2 * (int64_t)op->num_cus && long_halves)) cg = 8;
+    while (c > 1 && (int64_t)T.nblocks * (nrhs / c) * 2 <= (int64_t)op->num_cus) c >>= 1;
+  // launches CG columns in each of NG groups with KB stages, or with 4 when LDS
+  // holds no more or when that lets the grid run in fewer rounds; false when LDS
+  // holds fewer than 4
+  auto go = [&](auto cg, auto ng, auto nh) {
+    constexpr int CG = decltype(cg)::value, NG = decltype(ng)::value, NH = decltype(nh)::value;
+    using L = RingLds<V, CG, NG, NH>;
+    const int64_t grid = (int64_t)T.nblocks * (nrhs / (CG * NG));
+    auto rounds = [&](int K) {
+      const int64_t at_once = (int64_t)op->num_cus * (op->lds_max / L::bytes(T.window, K));
+      return at_once > 0 ? (grid + at_once - 1) / at_once : INT64_MAX;
+    };
+    if (rounds(4) == INT64_MAX) return false;
+    if (rounds(KB) <= rounds(4)) launch_trsv_ring_k<V, KB, CG, NG, NH>(T, rhs, x, nrhs, s);
+    else launch_trsv_ring_k<V, 4, CG, NG, NH>(T, rhs, x, nrhs, s);
+    return true;
+  };
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I4 = std::integral_constant<int, 4>;
+  using I8 = std::integral_constant<int, 8>;
+  // Half steps have no idle wave where a level set rarely holds more than 16 rows:
+  // the solving waves are then all column groups.  Whole steps shorten the chain
+  // where it often does.  Measured, us per launch, half / whole steps: 64^3
+  // (62,914 against 60,888 steps) 8 FP64 columns 206 / 263, 64 FP32 306 / 424;
+  // 96^3 convection-diffusion (153,495 against 110,111) 8 FP64 columns 541 / 634;
+  // 128^3 (319,055 against 202,577) 8 FP32 columns 802 / 613, 8 FP64 940 / 806.
+  const bool half = op->ring_nt == 64 || (op->ring_nt == 0 && 2 * T.max_block_steps_h < 3 * T.max_block_steps);
+  if constexpr (CMAX >= 16) {
+    if (c == 16 && (half ? go(I4(), I4(), I1()) : go(I8(), I2(), I2()))) return;
+    if (c == 16) c = 8;
   }
-  if (op->ring_lpr == 2) cg = std::min(cg, 4);  // a lane pair finalizes at most two columns each
-  while (cg > 1 && (size_t)(T.window + 1) * cg * sizeof(V) > (size_t)op->lds_max) cg >>= 1;
-  // Per launch: at two or more workgroups per CU the CUs' issue and memory
-  // pipes bound the solve, and one-wave workgroups on half steps (no barrier
-  // per step) do the same work in less time; below that, 128 threads take the
-  // steps whole and halve the dependent chain.
-  int nt = op->ring_nt;
-  if (nt == 0)
-    nt = (T.desc_h.p && (int64_t)T.nblocks * (nrhs / cg) >= 2 * (int64_t)op->num_cus) ? 64 : 128;
-  if (nt == 64 && op->ring_lpr == 4 && !T.desc_h.p) nt = 128;
-  if (nt == 64 && op->ring_lpr == 2) {
-    if (cg >= 4) launch_trsv_ring_cg<V, 64, 2, 4>(T, rhs, x, nrhs, s);
-    else if (cg >= 2) launch_trsv_ring_cg<V, 64, 2, 2>(T, rhs, x, nrhs, s);
-    else launch_trsv_ring_cg<V, 64, 2, 1>(T, rhs, x, nrhs, s);
-  } else if (nt == 64) {
-    if constexpr (sizeof(V) == 4) {
-      if (cg >= 8) {
-        launch_trsv_ring_cg<V, 64, 4, 8>(T, rhs, x, nrhs, s);
-        return;
-      }
-    }
-    if (cg >= 4) launch_trsv_ring_cg<V, 64, 4, 4>(T, rhs, x, nrhs, s);
-    else if (cg == 2) launch_trsv_ring_cg<V, 64, 4, 2>(T, rhs, x, nrhs, s);
-    else launch_trsv_ring_cg<V, 64, 4, 1>(T, rhs, x, nrhs, s);
-  } else {
-    // two 4-column groups per workgroup when both rings fit in LDS and the
-    // paired grid still gives every CU a workgroup
-    const bool pair = cg >= 4 && op->trsv_groups != 1 && nrhs >= 8 &&
-                      (op->trsv_groups == 2 || (int64_t)T.nblocks * (nrhs / 8) >= op->num_cus) &&
-                      (size_t)(T.window + 1) * 8 * sizeof(V) <= (size_t)op->lds_max;
-    if constexpr (sizeof(V) == 4) {
-      if (cg >= 8) {
-        launch_trsv_ring_cg<V, 128, 4, 8>(T, rhs, x, nrhs, s);
-        return;
-      }
-    }
-    if (pair) launch_trsv_ring_cg<V, 128, 4, 4, 2>(T, rhs, x, nrhs, s);
-    else if (cg >= 4) launch_trsv_ring_cg<V, 128, 4, 4>(T, rhs, x, nrhs, s);
-    else if (cg == 2) launch_trsv_ring_cg<V, 128, 4, 2>(T, rhs, x, nrhs, s);
-    else launch_trsv_ring_cg<V, 128, 4, 1>(T, rhs, x, nrhs, s);
+  if constexpr (CMAX >= 8) {
+    if (c == 8 && (half ? go(I2(), I4(), I1()) : go(I4(), I2(), I2()))) return;
+    if (c == 8) c = 4;
   }
+  if (c == 4 && (half ? go(I2(), I2(), I1()) : go(I4(), I1(), I2()))) return;
+  if (c == 4) c = 2;
+  if (c == 2 && (half ? go(I1(), I2(), I1()) : go(I2(), I1(), I2()))) return;
+  // the largest rings leave room for fewer stages
+  if (!(half ? go(I1(), I1(), I1()) : go(I1(), I1(), I2()))) launch_trsv_ring_k<V, 2, 1, 1, 2>(T, rhs, x, nrhs, s);
 }
 
 template <typename V>
@@ -619,21 +637,29 @@ void set_ring_attrs(K kern, int lds_max) {
 
 template <typename V>
 void set_trsv_attrs(int lds_max) {
-  constexpr int D1 = ring_depth<V, 1>(), D2 = ring_depth<V, 2>(), D4 = ring_depth<V, 4>();
-  set_ring_attrs(k_trsv_ring<V, 128, 4, kRingWidth / 4, D1, 1, 1>, lds_max);
-  set_ring_attrs(k_trsv_ring<V, 128, 4, kRingWidth / 4, D2, 2, 1>, lds_max);
-  set_ring_attrs(k_trsv_ring<V, 128, 4, kRingWidth / 4, D4, 4, 1>, lds_max);
-  set_ring_attrs(k_trsv_ring<V, 128, 4, kRingWidth / 4, D4, 4, 2>, lds_max);
-  set_ring_attrs(k_trsv_ring<V, 64, 4, kRingWidth / 4, D1, 1, 1>, lds_max);
-  set_ring_attrs(k_trsv_ring<V, 64, 4, kRingWidth / 4, D2, 2, 1>, lds_max);
-  set_ring_attrs(k_trsv_ring<V, 64, 4, kRingWidth / 4, D4, 4, 1>, lds_max);
-  set_ring_attrs(k_trsv_ring<V, 64, 2, kRingWidth / 2, (ring_depth<V, 1, 2>()), 1, 1>, lds_max);
-  set_ring_attrs(k_trsv_ring<V, 64, 2, kRingWidth / 2, (ring_depth<V, 2, 2>()), 2, 1>, lds_max);
-  set_ring_attrs(k_trsv_ring<V, 64, 2, kRingWidth / 2, (ring_depth<V, 4, 2>()), 4, 1>, lds_max);
+  auto both = [&](auto cg, auto ng, auto nh) {  // both numbers of stages
+    constexpr int CG = decltype(cg)::value, NG = decltype(ng)::value, NH = decltype(nh)::value;
+    set_ring_attrs(k_trsv_ring<V, ring_depth<V>(), CG, NG, NH>, lds_max);
+    set_ring_attrs(k_trsv_ring<V, 4, CG, NG, NH>, lds_max);
+  };
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I4 = std::integral_constant<int, 4>;
+  using I8 = std::integral_constant<int, 8>;
+  set_ring_attrs(k_trsv_ring<V, 2, 1, 1, 2>, lds_max);
+  both(I1(), I1(), I2());
+  both(I1(), I1(), I1());
+  both(I2(), I1(), I2());
+  both(I1(), I2(), I1());
+  both(I4(), I1(), I2());
+  both(I2(), I2(), I1());
+  if constexpr (sizeof(V) <= 8) {
+    both(I4(), I2(), I2());
+    both(I2(), I4(), I1());
+  }
   if constexpr (sizeof(V) == 4) {
-    constexpr int D8 = ring_depth<V, 8>();
-    set_ring_attrs(k_trsv_ring<V, 128, 4, kRingWidth / 4, D8, 8, 1>, lds_max);
-    set_ring_attrs(k_trsv_ring<V, 64, 4, kRingWidth / 4, D8, 8, 1>, lds_max);
+    both(I8(), I2(), I2());
+    both(I4(), I4(), I1());
   }
   if constexpr (scalar_traits<V>::is_complex) return;  // no pipelined kernel for complex values
   constexpr int DL2 = sizeof(V) == 4 ? 5 : 4;  // the pipelined kernel's stage depths (launch_trsv_pipe_nt)
@@ -956,8 +982,8 @@ void upload_op(pgs_dev_op_s* op, const HostOp<T>& H, int prec_mask, bool all_c =
   // ring packing (ring kernel) unless another kernel geometry was asked for;
   // the ring holds at least one column of the operator's values
   const bool ring = op->trsv_variant == 0 && op->trsv_nt == 128 && op->trsv_lpr == 4;
-  // ring steps hold at most 32 rows: 128 threads x 4 lanes or 64 x 2 take a
-  // step whole, 64 x 4 takes it in two half steps
+  // ring steps hold at most 32 rows: 128 threads take a step whole, 64 take it
+  // in two half steps
   const int max_rows = ring ? 32 : op->trsv_nt / op->trsv_lpr;
   int max_window = 0;
   if (ring) {
@@ -1154,18 +1180,13 @@ int pgs_dev_op_create(pgs_gemslr_t hop, int device, int prec_mask, pgs_dev_op_t*
     if (op->trsv_lpr == 2 && op->trsv_nt == 256) op->trsv_nt = 128;
     if (op->trsv_lpr == 4 && op->trsv_nt == 64) op->trsv_nt = 128;
     if (const char* v = std::getenv("PGS_RING_GEOM")) {
-      // threads x lanes per row of the ring kernel: 128x4, 64x4 or 64x2
-      if (!std::strcmp(v, "64x4")) { op->ring_nt = 64; op->ring_lpr = 4; }
-      else if (!std::strcmp(v, "64x2")) { op->ring_nt = 64; op->ring_lpr = 2; }
-      else if (!std::strcmp(v, "128x4")) { op->ring_nt = 128; op->ring_lpr = 4; }
-    }
-    if (const char* v = std::getenv("PGS_TRSV_GROUPS")) {
-      const int g = std::atoi(v);
-      if (g >= 0 && g <= 2) op->trsv_groups = g;
+      // threads x lanes per row of one column group of the ring kernel: 128x4 or 64x4
+      if (!std::strcmp(v, "64x4")) op->ring_nt = 64;
+      else if (!std::strcmp(v, "128x4")) op->ring_nt = 128;
     }
     if (const char* v = std::getenv("PGS_TRSV_CG")) {
       const int cg = std::atoi(v);
-      if (cg == 1 || cg == 2 || cg == 4 || cg == 8) op->trsv_cg = cg;
+      if (cg == 1 || cg == 2 || cg == 4 || cg == 8 || cg == 16) op->trsv_cg = cg;
     }
     op->is_complex = h->is_complex;
     if (h->is_complex)

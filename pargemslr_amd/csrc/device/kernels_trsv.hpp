@@ -137,12 +137,6 @@ __device__ __forceinline__ TPair<cplx<double>> bload_pair(__amdgpu_buffer_rsrc_t
   p.col = (int)__builtin_amdgcn_raw_buffer_load_b32(r, off + 16, 0, 0);
   return p;
 }
-// The first three fields of a step descriptor (row offset, entry offset, rows).
-__device__ __forceinline__ int3 bload_i3(__amdgpu_buffer_rsrc_t r, int off) {
-  auto v = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
-  return make_int3((int)v[0], (int)v[1], (int)v[2]);
-}
-
 // Sum over the 4 lanes of a quad with DPP quad permutations (xor 1, xor 2).
 __device__ __forceinline__ float quad_sum(float v) {
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
@@ -152,11 +146,11 @@ __device__ __forceinline__ float quad_sum(float v) {
 __device__ __forceinline__ double quad_perm_f64(double v, int ctrl_sel) {
   int lo = __double2loint(v), hi = __double2hiint(v);
   if (ctrl_sel == 1) {
-    lo = __builtin_amdgcn_update_dpp(0, lo, 0xB1, 0xF, 0xF, false);
-    hi = __builtin_amdgcn_update_dpp(0, hi, 0xB1, 0xF, 0xF, false);
+    lo = __builtin_amdgcn_mov_dpp(lo, 0xB1, 0xF, 0xF, true);
+    hi = __builtin_amdgcn_mov_dpp(hi, 0xB1, 0xF, 0xF, true);
   } else {
-    lo = __builtin_amdgcn_update_dpp(0, lo, 0x4E, 0xF, 0xF, false);
-    hi = __builtin_amdgcn_update_dpp(0, hi, 0x4E, 0xF, 0xF, false);
+    lo = __builtin_amdgcn_mov_dpp(lo, 0x4E, 0xF, 0xF, true);
+    hi = __builtin_amdgcn_mov_dpp(hi, 0x4E, 0xF, 0xF, true);
   }
   return __hiloint2double(hi, lo);
 }
@@ -347,47 +341,39 @@ __global__ __launch_bounds__(NT) void k_trsv_pipe(int nblocks, const int* __rest
   }
 }
 
-// Ring kernel: one workgroup per (diagonal block, group of CG right-hand-side
+// Ring kernel: one workgroup per (diagonal block, C = CG * NG right-hand-side
 // columns); grid index = group * nblocks + block (all groups of a block on one
 // XCD, as above).  The packed columns are ring slots: the value of the row
-// stored at pair index p lives in LDS slot p & wmask (CG values per slot)
-// from its step until its last reader, so the LDS footprint is the sweep
-// window, not the block.  The L sweep reads rhs and writes y to x in global
-// memory; the U sweep reads y back from x and overwrites it with the solution
-// (a row's y is read by the lanes that later write that row).  Rows are
-// prefetched D steps ahead (descriptor, row pair, slots); the right-hand side
-// of a step, whose address depends on the row pair, is loaded D/2 steps ahead.
-// Lane q of a row's LPR lanes finalizes columns q, q + LPR, ...  Lanes past
-// a step's rows gather and write nothing.  With 8- and 16-byte values they
-// re-read the step's last row (cache lines already fetched); with 4-byte
-// values they read the following rows' pairs and slabs (valid ring slots, or
-// zeros past the block from the bounded buffers), which saves the clamp's
-// instructions in a loop bound by instruction issue.
+// stored at position p lives in LDS slot p % rows (CG values per slot, one ring
+// per column group) from its step until its last reader, so the LDS footprint
+// is the sweep window, not the block.  The L sweep reads rhs and writes y to x in
+// global memory; the U sweep reads y back from x and overwrites it with the
+// solution (a row's y is read before that row is written).
+//
+// What bounds it: a block is a chain of dependent steps (3,350 at 128^3), and a
+// step is LDS gathers -> multiply-adds -> quad reduction -> LDS write -> barrier,
+// about 230 clocks of latency, plus the instructions around it at 4 to 6 clocks
+// each, since a SIMD issues one instruction of a wave at a time.  So the work is
+// split over waves, one per SIMD for one column: NH * NG solving waves (NH = 2:
+// the rows 0-15 and 16-31 of a step, NH = 1: half steps of at most 16 rows; NG
+// groups of CG columns) do nothing but the chain, one wave copies the factor
+// records to LDS and one the row data, both K steps ahead and straight from
+// memory to LDS.  Four lanes solve a row with five entries each; lane q of a row
+// finalizes columns q, q + 4, ...  When every wave did everything (5 entry loads, a
+// row pair, a descriptor and a right-hand side per step: about 51 instructions
+// for one FP32 column, 69 for FP64, against 35 and 42 in a solving wave now),
+// level 0 took, us per launch at 128^3, FP32 / FP64, before -> now: 1 column 652 /
+// 970 -> 517 / 664; 8 columns 740 / 1013 -> 611 / 807; 64 columns 1586 / 3699 ->
+// 1452 / 2869; 64^3, 1 column: 219 / 255 -> 145 / 172; 1023 x 1021, 8 columns: 790 /
+// 1020 -> 592 / 685.
 template <typename V, int CG>
 struct alignas(CG * sizeof(V) < 16 ? CG * sizeof(V) : 16) RingRow {
   V v[CG];
 };
 
-// Ring-packed entries hold their ring slot times ring_unit<V>(): the byte
-// offset of the slot in a ring of 4-column rows, so that 4-column groups (the
-// default) gather without scaling the slot and the others scale it by one
-// shift.
-template <typename V>
-constexpr int ring_unit() {
-  return 4 * (int)sizeof(V);
-}
-template <typename V, int CG>
-__device__ __forceinline__ unsigned ring_byte(int c) {
-  constexpr int RB = CG * (int)sizeof(V), U = ring_unit<V>();
-  if constexpr (RB >= U) return (unsigned)c * (RB / U);
-  else return (unsigned)c / (unsigned)(U / RB);
-}
-
 // A ring row read through its LDS byte address.  The ring kernel has no
 // static LDS, so its dynamic LDS starts at address 0 (checked on the host
-// when the kernels are set up): the address is the slot's byte offset plus
-// the group's ring offset, and with one group the gather takes the entry's
-// column as its address unchanged.
+// when the kernels are set up): the address is the slot's byte offset.
 template <typename T>
 __device__ __forceinline__ T lds_read(unsigned addr) {
   constexpr int N = (int)sizeof(T) / 4;
@@ -399,27 +385,12 @@ __device__ __forceinline__ T lds_read(unsigned addr) {
   }
 }
 
-__device__ __forceinline__ float bload_val(__amdgpu_buffer_rsrc_t r, int off, float) {
-  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
-}
-__device__ __forceinline__ double bload_val(__amdgpu_buffer_rsrc_t r, int off, double) {
-  auto v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
-  return __hiloint2double((int)v[1], (int)v[0]);
-}
 // Buffer stores (vector memory): writes outside the resource are dropped.
 __device__ __forceinline__ void bstore_val(__amdgpu_buffer_rsrc_t r, int off, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, off, 0, 0);
 }
 __device__ __forceinline__ void bstore_val(__amdgpu_buffer_rsrc_t r, int off, double v) {
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, v), r, off, 0, 0);
-}
-__device__ __forceinline__ cplx<float> bload_val(__amdgpu_buffer_rsrc_t r, int off, cplx<float>) {
-  auto v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
-  return cplx<float>(__uint_as_float(v[0]), __uint_as_float(v[1]));
-}
-__device__ __forceinline__ cplx<double> bload_val(__amdgpu_buffer_rsrc_t r, int off, cplx<double>) {
-  auto v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
-  return cplx<double>(__hiloint2double((int)v[1], (int)v[0]), __hiloint2double((int)v[3], (int)v[2]));
 }
 __device__ __forceinline__ void bstore_val(__amdgpu_buffer_rsrc_t r, int off, cplx<float> v) {
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, v), r, off, 0, 0);
@@ -429,19 +400,6 @@ __device__ __forceinline__ void bstore_val(__amdgpu_buffer_rsrc_t r, int off, cp
 }
 
 // Two consecutive values in one buffer access (8-byte and smaller values).
-template <typename V>
-__device__ __forceinline__ RingRow<V, 2> bload_val2(__amdgpu_buffer_rsrc_t r, int off) {
-  static_assert(sizeof(V) <= 8, "two values in one access");
-  RingRow<V, 2> o;
-  if constexpr (sizeof(V) == 4) {
-    auto v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
-    o = __builtin_bit_cast(RingRow<V, 2>, v);
-  } else {
-    auto v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
-    o = __builtin_bit_cast(RingRow<V, 2>, v);
-  }
-  return o;
-}
 template <typename V>
 __device__ __forceinline__ void bstore_val2(__amdgpu_buffer_rsrc_t r, int off, const RingRow<V, 2>& o) {
   static_assert(sizeof(V) <= 8, "two values in one access");
@@ -454,164 +412,378 @@ __device__ __forceinline__ void bstore_val2(__amdgpu_buffer_rsrc_t r, int off, c
 // An empty asm that takes a value as read and rewritten: the value must have
 // arrived, and it counts as produced here rather than by its load.
 __device__ __forceinline__ void pin_reg(int& v) { __asm__ __volatile__("" : "+v"(v)); }
-__device__ __forceinline__ void pin_reg(float& v) { __asm__ __volatile__("" : "+v"(v)); }
-__device__ __forceinline__ void pin_reg(double& v) { __asm__ __volatile__("" : "+v"(v)); }
-template <typename R>
-__device__ __forceinline__ void pin_reg(cplx<R>& v) {
-  pin_reg(v.re);
-  pin_reg(v.im);
-}
+
+// Factor entries of the ring kernel.  A row takes four lanes, a lane five
+// entries: entry j of the row is entry j / 4 of lane j % 4.  A lane's record is
+// its five values and five 16-bit ring slots, cut into pieces of at most 16
+// bytes:
+//   4-byte values   [v0 v1 v2 v3] [v4 s01 s23 s4]
+//   8-byte values   [v0 v1] [v2 v3] [v4 s01 s23] [s4]
+//   16-byte values  [v0] [v1] [v2] [v3] [v4] [s01 s23 s4 -]
+// (s01: slots 0 and 1 in one word).  The rows of a step are cut into groups of
+// 16 (the rows of one wave); a group of n rows at position p starts at byte
+// p * ring_row_bytes<V>() of its block and holds piece 0 of its 4 n lanes, then
+// piece 1, ...: every copy of a wave is one contiguous run of memory at a
+// wave-uniform base, and lands in LDS as the solving lanes read it.
 template <typename V>
-__device__ __forceinline__ void pin_reg(TPair<V>& p) {
-  pin_reg(p.col);
-  pin_reg(p.val);
+__host__ __device__ constexpr int ring_row_bytes() {
+  return 4 * (5 * (int)sizeof(V) + (sizeof(V) == 16 ? 16 : 12));
 }
-__device__ __forceinline__ void pin_reg(int3& d) {
-  pin_reg(d.x);
-  pin_reg(d.y);
-  pin_reg(d.z);
-}
+constexpr int kRingGroup = 16;  // rows of a group
 
-template <typename V, int NT, int LPR, int EPL, int D, int CG, bool UPPER, int G>
-__device__ __forceinline__ void ring_sweep(int s_begin, int s_end, int sbeg, int wmask, int nrhs, int c0,
-                                           __amdgpu_buffer_rsrc_t rs_desc, __amdgpu_buffer_rsrc_t rs_ri,
-                                           __amdgpu_buffer_rsrc_t rs_ent, __amdgpu_buffer_rsrc_t rs_src, V* xs,
-                                           unsigned xsb,
-                                           __amdgpu_buffer_rsrc_t rs_dst) {
-  constexpr int PS = (int)sizeof(TPair<V>);
-  constexpr int VS = (int)sizeof(V);
-  constexpr int RW = LPR * EPL;  // slab width of every ring-packed step
-  static_assert(D % 2 == 0, "stage depth must be even");
-  static_assert((LPR == 4 && (CG == 1 || CG == 2 || CG == 4 || CG == 8)) ||
-                    (LPR == 2 && (CG == 1 || CG == 2 || CG == 4)),
-                "quad lanes with 1, 2, 4 or 8 columns, or lane pairs with 1, 2 or 4 columns");
-  constexpr int NCL = CG == 2 * LPR ? 2 : 1;  // columns finalized per lane
-  // a lane's two columns are adjacent: one access for both (8-byte and
-  // smaller values)
-  constexpr bool kPairIO = NCL == 2 && sizeof(V) <= 8;
-  const int tid = threadIdx.x % NT;  // thread within this column group
-  const int q = tid % LPR;
-  const int t0 = tid / LPR;
-  // after the reduction lane q holds column q % CG (lanes q < CG write it), or
-  // with two columns per lane (8 columns on quads, 4 on lane pairs) columns
-  // 2q and 2q + 1
-  int cl[NCL];
-  if constexpr (NCL == 2) {
-    cl[0] = 2 * q;
-    cl[1] = 2 * q + 1;
+template <typename V>
+struct LaneRec {
+  V val[5];
+  unsigned s01, s23, s4;
+};
+
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// Writes (on the host) entry j of row t of the group of n rows
+// whose bytes start at g.
+template <typename V>
+inline void store_rec(unsigned char* g, int n, int t, int j, const V& v, unsigned slot) {
+  const int lane = 4 * t + j % 4, e = j / 4;
+  auto put = [](unsigned char* q, const void* x, int b) { __builtin_memcpy(q, x, (size_t)b); };
+  const uint16_t s16 = (uint16_t)slot;
+  unsigned char* sl;  // the word of slots 0 and 1; slot 4's word
+  unsigned char* s4;
+  if constexpr (sizeof(V) == 4) {
+    unsigned char* b = g + n * 64 + lane * 16;
+    put(e < 4 ? g + lane * 16 + e * 4 : b, &v, 4);
+    sl = b + 4;
+    s4 = b + 12;
+  } else if constexpr (sizeof(V) == 8) {
+    put(g + (e / 2) * n * 64 + lane * 16 + (e % 2) * 8, &v, 8);
+    sl = g + n * 128 + lane * 16 + 8;
+    s4 = g + n * 192 + lane * 4;
   } else {
-    cl[0] = q % CG;
+    put(g + e * n * 64 + lane * 16, &v, 16);
+    sl = g + n * 320 + lane * 16;
+    s4 = sl + 8;
   }
-  const bool writer = q < CG;
-  const int dummy = (wmask + 1) * CG;  // LDS slot written by lanes with nothing to write
-  // row * nrhs as a shift: the launch admits power-of-two column counts only
-  // (a 32-bit multiply is a quarter-rate instruction, two per step otherwise)
-  const int csh = __builtin_ctz((unsigned)nrhs);
-  constexpr bool kClampRows = sizeof(V) > 4;
-  // Gathers through LDS byte addresses and the prologue's register pinning
-  // (below) make every geometry faster (level 0 at 128^3: 1 to 64 RHS 3-12 %
-  // less time) except one: the one-wave FP32 kernel with 4-column groups
-  // (the 32-RHS launch) runs 12 % slower with them (1.47 against 1.31 ms on
-  // one device), with or without the other, and at ring depths 8 and 10 as
-  // well.  That kernel keeps the generic gather and the plain prologue.
-  constexpr bool kLdsPath = !(NT == 64 && LPR == 4 && CG == 4 && sizeof(V) == 4);
+  put(e < 4 ? sl + 2 * e : s4, &s16, 2);
+}
 
-  TPair<V> pe[D][EPL];
-  TPair<V> pr[D];
-  V xr[D][NCL];
-  int sw[D];   // ring slot of this lane's row in the step held by stage k, -1 past the step's rows
-  int3 dn[D];  // descriptor of the step stage k loads next
+// LDS byte address of a ring row: base + slot * RS with the slot in the low or
+// high half of w, one instruction.
+template <int RS, bool HIGH>
+__device__ __forceinline__ unsigned slot_addr(unsigned w, unsigned base) {
+  unsigned a;
+  if constexpr (HIGH) __asm__("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(a) : "v"(w), "s"(RS), "v"(base));
+  else __asm__("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(a) : "v"(w), "s"(RS), "v"(base));
+  return a;
+}
 
-#define PGS_RING_PAIR(K, DESC)                                                  \
-  do {                                                                          \
-    const int3 d_ = (DESC);                                                     \
-    const int tt_ = kClampRows ? min(t0, max(d_.z - 1, 0)) : t0;                \
-    const int r_ = d_.x + tt_;                                                  \
-    sw[K] = t0 < d_.z ? (r_ & wmask) : -1;                                      \
-    pr[K] = bload_pair(rs_ri, r_ * PS, V(0));                                   \
-  } while (0)
-#define PGS_RING_ENT(K, DESC)                                                   \
-  do {                                                                          \
-    const int3 d_ = (DESC);                                                     \
-    const int tt_ = kClampRows ? min(t0, max(d_.z - 1, 0)) : t0;                \
-    const int eb_ = (d_.y + tt_ * RW + q) * PS;                                 \
-    _Pragma("unroll") for (int e_ = 0; e_ < EPL; ++e_)                          \
-      pe[K][e_] = bload_pair(rs_ent, eb_ + e_ * LPR * PS, V(0));                \
-  } while (0)
-#define PGS_RING_STAGE(K, DESC) \
-  do {                          \
-    const int3 ds_ = (DESC);    \
-    PGS_RING_PAIR(K, ds_);      \
-    PGS_RING_ENT(K, ds_);       \
-  } while (0)
-#define PGS_RING_RHS(K)                                                           \
-  do {                                                                            \
-    if constexpr (kPairIO) {                                                      \
-      const RingRow<V, 2> t_ = bload_val2<V>(rs_src, ((pr[K].col << csh) + c0 + cl[0]) * VS); \
-      xr[K][0] = t_.v[0];                                                         \
-      xr[K][1] = t_.v[1];                                                         \
-    } else {                                                                      \
-      _Pragma("unroll") for (int j_ = 0; j_ < NCL; ++j_) xr[K][j_] =              \
-          bload_val(rs_src, ((pr[K].col << csh) + c0 + cl[j_]) * VS, V(0));       \
-    }                                                                             \
-  } while (0)
-
-  const int rel = s_begin - sbeg;
-#pragma unroll
-  for (int k = 0; k < D; ++k) {
-    PGS_RING_STAGE(k, bload_i3(rs_desc, (rel + k) * 16));
-    dn[k] = bload_i3(rs_desc, (rel + k + D) * 16);
+// A value written through its LDS byte address.
+template <typename T>
+__device__ __forceinline__ void lds_write(unsigned addr, const T& v) {
+  constexpr int N = (int)sizeof(T) / 4;
+  if constexpr (N == 1) {
+    *reinterpret_cast<__attribute__((address_space(3))) unsigned*>((size_t)addr) = __builtin_bit_cast(unsigned, v);
+  } else {
+    using W = unsigned __attribute__((ext_vector_type(N)));
+    *reinterpret_cast<__attribute__((address_space(3))) W*>((size_t)addr) = __builtin_bit_cast(W, v);
   }
+}
+
+constexpr int kRingOut = 0x7ffffff0;  // a byte offset past every resource of the ring kernel
+
+// Pieces of a lane's record: loads (and direct-to-LDS copies) per wave and step.
+template <typename V>
+constexpr int ring_pieces() {
+  return sizeof(V) == 4 ? 2 : sizeof(V) == 8 ? 4 : 6;
+}
+// Bytes of one wave's records in LDS: piece i at i * 1024, 16 bytes per lane (the
+// last piece of 8-byte values: 4).
+template <typename V>
+constexpr int ring_stage_bytes() {
+  return 16 * ring_row_bytes<V>();
+}
+
+// A right-hand side row of C values in pieces that direct-to-LDS copies can move
+// (4 or 16 bytes per lane): U bytes each, ND copies for the 16 NH rows of a step.
+template <typename V, int C, int NH>
+struct RingRhs {
+  static constexpr int row = C * (int)sizeof(V);
+  static constexpr int U = row < 16 ? 4 : 16;
+  static constexpr int ND = (16 * NH * row / U + 63) / 64;
+};
+
+// LDS of the ring kernel in bytes, by offset: NG rings of CG columns (each with
+// its dummy row), then K stages of {records of 16 NH rows; 32 pairs (ring slot
+// times sizeof(V), row id); 32 pivots; the rows' right-hand sides}.  A copy moves
+// a piece of every lane, so a part holds at least 64 pieces.
+template <typename V, int CG, int NG, int NH>
+struct RingLds {
+  using R = RingRhs<V, CG * NG, NH>;
+  static constexpr int rec = NH * ring_stage_bytes<V>();
+  static constexpr int info = 64 * 4, piv = 64 * (sizeof(V) == 16 ? 16 : 4), rhs = R::ND * 64 * R::U;
+  static constexpr int stage = rec + info + piv + rhs;
+  __host__ __device__ static int ring(int rows) { return ((rows + 1) * CG * (int)sizeof(V) + 15) & ~15; }
+  __host__ __device__ static int bytes(int rows, int K) { return NG * ring(rows) + K * stage; }
+};
+
+// Sweep of the wave that moves the records.  Between the barriers of steps s - 1
+// and s it starts the copy of the records of step s + K into the stage that the
+// solving waves have just taken step s from, and waits until the records of step
+// s + 2 have arrived.
+template <typename V, int K, int CG, int NG, int NH>
+__device__ __forceinline__ void ring_copy_sweep(int nsteps, const int* pos, int rows, __amdgpu_buffer_rsrc_t rs_ent) {
+  constexpr int RB = ring_row_bytes<V>(), PB = ring_stage_bytes<V>(), NP = ring_pieces<V>();
+  using L = RingLds<V, CG, NG, NH>;
+  static_assert(2 * K + 2 <= 64, "step boundaries of a pass and its look-ahead in one register");
+  constexpr int kWait = K > 2 ? (K - 2) * NH * NP : 0;  // the copies of the K - 2 steps after s + 2
+  static_assert(kWait <= 60, "outstanding copies");
+  const int lane = threadIdx.x & 63;
+  const unsigned stage0 = (unsigned)(NG * L::ring(rows));
+  const __amdgpu_buffer_rsrc_t rs_pos = make_rsrc(pos, (int64_t)(nsteps + 1) * 4);
+  int pv = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_pos, min(lane, nsteps) * 4, 0, 0);
+  const int l16 = lane * 16;
+  auto copy_group = [&](unsigned a, int p, int n) {
+    // lanes past a group's rows copy zeros (no memory traffic)
+    using LP = __attribute__((address_space(3))) void*;
+    const bool in = lane < 4 * n;
+    const int vo16 = in ? l16 : kRingOut;
+    const int base = p * RB, pc = n * 64;
+    constexpr int N16 = sizeof(V) == 8 ? 3 : NP;
 #pragma unroll
-  for (int k = 0; k < D / 2; ++k) PGS_RING_RHS(k);
-  // The compiler gives the loop's first steps the load waits of the worst
-  // path into them, and the path from here is the worst: the prologue's last
-  // loads are right-hand sides and slabs of the first steps, and every
-  // iteration would wait for nearly all loads in flight once per 2 D steps.
-  // Taking the prologue's registers as redefined here (one wait for its
-  // loads, once per sweep) leaves the loop the waits of its own back edge.
+    for (int j = 0; j < N16; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_ent, (LP)(size_t)(a + j * 1024), 16, vo16, base + j * pc, 0, 0);
+    if constexpr (sizeof(V) == 8)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_ent, (LP)(size_t)(a + 3 * 1024), 4, in ? lane * 4 : kRingOut, base + 3 * pc,
+                                               0, 0);
+  };
+  auto copy_step = [&](int stage, int i) {  // step i of the pass
+    const int p0 = __builtin_amdgcn_readlane(pv, i), n = __builtin_amdgcn_readlane(pv, i + 1) - p0;
+    const int n0 = min(n, kRingGroup);
+    const unsigned a = stage0 + stage * L::stage;
+    copy_group(a, p0, n0);
+    if constexpr (NH == 2) copy_group(a + PB, p0 + n0, n - n0);
+  };
 #pragma unroll
-  for (int k = 0; k < (kLdsPath ? D : 0); ++k) {
-    if (k < D / 2) {
+  for (int k = 0; k < K; ++k) copy_step(k, k);
+  __builtin_amdgcn_sched_barrier(0);
+  __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  // the solving waves take step 0 here, before its stage is used again
+  __builtin_amdgcn_s_barrier();
+  __asm__ __volatile__("" ::: "memory");
+  for (int base = 0; base < nsteps; base += K) {
+    const int pvn = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_pos, min(base + K + lane, nsteps) * 4, 0, 0);
 #pragma unroll
-      for (int j = 0; j < NCL; ++j) pin_reg(xr[k][j]);
+    for (int kk = 0; kk < K; ++kk) {
+      copy_step(kk, kk + K);
+      __builtin_amdgcn_sched_barrier(0);
+      __asm__ __volatile__("s_waitcnt vmcnt(%0)" ::"n"(kWait) : "memory");
+      __builtin_amdgcn_s_barrier();
+      __asm__ __volatile__("" ::: "memory");
     }
-    pin_reg(pr[k]);
-    pin_reg(dn[k]);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) pin_reg(pe[k][e]);
+    pv = pvn;
   }
+  // nothing may still be on its way to LDS when the stages are used again or
+  // the workgroup ends
+  __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory");
+}
 
-  for (int base = s_begin; base < s_end; base += 2 * D) {
+// The row id of the dummy row: shifted by 2 to 10 bits it is a byte offset past
+// every resource.
+constexpr int kRingDummyRow = 0x3fe00000;
+
+// Sweep of the wave that moves the row data (right-hand sides, pivots, ring slots
+// and row ids), as ring_copy_sweep the records; the row ids that the right-hand
+// sides' addresses need are loaded K steps before them.
+template <typename V, int K, int CG, int NG, int NH, bool UPPER>
+__device__ __forceinline__ void ring_row_sweep(int nsteps, const int* pos, int rows, int nrhs, int c0, int dummy,
+                                               __amdgpu_buffer_rsrc_t rs_info, __amdgpu_buffer_rsrc_t rs_dinv,
+                                               __amdgpu_buffer_rsrc_t rs_src) {
+  constexpr int VS = (int)sizeof(V);
+  using L = RingLds<V, CG, NG, NH>;
+  using R = typename L::R;
+  constexpr int ND = R::ND, U = R::U;
+  constexpr int OPS = 2 * ND + (UPPER ? 2 : 1);
+  constexpr int kWait = K > 2 ? (K - 2) * OPS : 0;
+  static_assert(kWait <= 60, "outstanding loads");
+  static_assert(3 * K + 2 <= 64, "step boundaries of a pass and its look-ahead in one register");
+  const int lane = threadIdx.x & 63;
+  const int csh = __builtin_ctz((unsigned)nrhs);
+  const unsigned stage0 = (unsigned)(NG * L::ring(rows));
+  using LP = __attribute__((address_space(3))) void*;
+  int rl[ND], rb[ND];  // this lane's row of the step and byte of the row, per copy
 #pragma unroll
-    for (int kk = 0; kk < 2 * D; ++kk) {
-      const int k = kk % D;
-      const int s = base + kk;
-      // gather this step's slots from the ring and take what the arithmetic
-      // needs out of the stage registers
-      RingRow<V, CG> xv[EPL];
-      V wgt[EPL];
+  for (int j = 0; j < ND; ++j) {
+    rl[j] = (j * 64 + lane) * U / R::row;
+    rb[j] = c0 * VS + (j * 64 + lane) * U % R::row;
+  }
+  int rowr[K][ND];
+
+  const __amdgpu_buffer_rsrc_t rs_pos = make_rsrc(pos, (int64_t)(nsteps + 1) * 4);
+  int pv = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_pos, min(lane, nsteps) * 4, 0, 0);
+  auto bnd = [&](int i) { return __builtin_amdgcn_readlane(pv, i); };
+  auto load_row = [&](int k, int i) {
+    const int p = bnd(i), n = bnd(i + 1) - p;
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        if constexpr (kLdsPath)
-          xv[e] = lds_read<RingRow<V, CG>>(xsb + ring_byte<V, CG>(pe[k][e].col));
-        else
-          xv[e] = *reinterpret_cast<const RingRow<V, CG>*>(reinterpret_cast<const unsigned char*>(xs) +
-                                                            ring_byte<V, CG>(pe[k][e].col));
-        wgt[e] = pe[k][e].val;  // padded slots weigh zero
+    for (int j = 0; j < ND; ++j)
+      rowr[k][j] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_info, rl[j] < n ? rl[j] * 8 + 4 : kRingOut, p * 8, 0);
+  };
+  // row data of step i of the pass into stage k, its row ids in rowr[k].  Lanes
+  // past the step's rows copy the dummy row's pair and, for the rest, zeros (no
+  // memory traffic).
+  auto copy_step = [&](int k, int i) {
+    const int p = bnd(i), n = bnd(i + 1) - p;
+    const unsigned a = stage0 + k * L::stage + L::rec;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_info, (LP)(size_t)a, 4,
+                                             lane < 2 * n ? lane * 4 : dummy - p * 8 + (lane & 1) * 4, p * 8, 0, 0);
+    if constexpr (UPPER) {
+      if constexpr (VS == 16)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_dinv, (LP)(size_t)(a + L::info), 16, lane < n ? lane * 16 : kRingOut,
+                                                 p * VS, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_dinv, (LP)(size_t)(a + L::info), 4,
+                                                 lane < n * (VS / 4) ? lane * 4 : kRingOut, p * VS, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < ND; ++j) {
+      const int o = (int)((unsigned)rowr[k][j] << csh) * VS + rb[j];
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_src, (LP)(size_t)(a + L::info + L::piv + j * 64 * U), U,
+                                               rl[j] < n ? o : kRingOut, 0, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < K; ++k) load_row(k, k);
+#pragma unroll
+  for (int k = 0; k < K; ++k) copy_step(k, k);
+#pragma unroll
+  for (int k = 0; k < K; ++k) load_row(k, K + k);
+  // The compiler gives the loop's first steps the load waits of the worst
+  // path into them.  Taking the prologue's registers as redefined here (one
+  // wait for its loads, once per sweep) leaves the loop the waits of its own
+  // back edge.
+  __builtin_amdgcn_sched_barrier(0);
+  __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+#pragma unroll
+    for (int j = 0; j < ND; ++j) pin_reg(rowr[k][j]);
+  __builtin_amdgcn_s_barrier();
+  // the solving waves take step 0 here, before its stage is used again
+  __builtin_amdgcn_s_barrier();
+  __asm__ __volatile__("" ::: "memory");
+  for (int base = 0; base < nsteps; base += K) {
+    const int pvn = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_pos, min(base + K + lane, nsteps) * 4, 0, 0);
+#pragma unroll
+    for (int kk = 0; kk < K; ++kk) {
+      copy_step(kk, kk + K);
+      load_row(kk, kk + 2 * K);
+      __builtin_amdgcn_sched_barrier(0);
+      __asm__ __volatile__("s_waitcnt vmcnt(%0)" ::"n"(kWait) : "memory");
+      __builtin_amdgcn_s_barrier();
+      __asm__ __volatile__("" ::: "memory");
+    }
+    pv = pvn;
+  }
+  __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// Sweep of the solving waves: wave g * 2 + h of the group g of CG columns takes
+// rows 16 h .. 16 h + 15 of each step.
+template <typename V, int K, int CG, int NG, int NH, bool UPPER>
+__device__ __forceinline__ void ring_solve_sweep(int h, int g, int nsteps, int rows, int nrhs, int c0,
+                                                 __amdgpu_buffer_rsrc_t rs_dst) {
+  constexpr int VS = (int)sizeof(V);
+  constexpr int PB = ring_stage_bytes<V>();
+  using L = RingLds<V, CG, NG, NH>;
+  constexpr int NCL = CG == 8 ? 2 : 1;  // columns finalized per lane: adjacent ones, one access for both
+  static_assert(CG == 1 || CG == 2 || CG == 4 || (CG == 8 && VS == 4), "columns per group");
+  const int lane = threadIdx.x & 63;
+  const int q = lane % 4;
+  const int t = 16 * h + lane / 4;                      // this lane's row of the step
+  const int cq = CG == 8 ? 2 * q : q % CG;              // after the reduction the lane holds column cq (and cq + 1 of 8)
+  const unsigned gat = g * (unsigned)L::ring(rows);     // this group's ring
+  const unsigned wad = gat + cq * VS;                   // this lane's column of its row 0
+  const int cl = g * CG + cq;
+  const int sh = __builtin_ctz((unsigned)nrhs * (unsigned)VS);
+  const unsigned coff = (unsigned)((c0 + cl) * VS);
+  const unsigned ring_end = NG * (unsigned)L::ring(rows);
+  const unsigned st_a = ring_end + h * PB + lane * 16;
+  const unsigned st_x = ring_end + h * PB + 3 * 1024 + lane * 4;
+  const unsigned info_a = ring_end + L::rec + t * 8;
+  const unsigned piv_a = ring_end + L::rec + L::info + t * VS;
+  const unsigned rhs_a = ring_end + L::rec + L::info + L::piv + (t * CG * NG + cl) * VS;
+
+  LaneRec<V> rec;
+  u32x2 info;
+  V xin[NCL], dv = V(0);
+  auto take = [&](int stage) {  // the records and row data of a step
+    const unsigned a = st_a + stage * L::stage;
+    if constexpr (sizeof(V) == 4) {
+      const u32x4 v0 = lds_read<u32x4>(a), v1 = lds_read<u32x4>(a + 1024);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rec.val[e] = __uint_as_float(v0[e]);
+      rec.val[4] = __uint_as_float(v1[0]);
+      rec.s01 = v1[1];
+      rec.s23 = v1[2];
+      rec.s4 = v1[3];
+    } else if constexpr (sizeof(V) == 8) {
+      const u32x4 v0 = lds_read<u32x4>(a), v1 = lds_read<u32x4>(a + 1024), v2 = lds_read<u32x4>(a + 2048);
+      rec.s4 = lds_read<unsigned>(st_x + stage * L::stage);
+      rec.val[0] = __builtin_bit_cast(V, u32x2{v0[0], v0[1]});
+      rec.val[1] = __builtin_bit_cast(V, u32x2{v0[2], v0[3]});
+      rec.val[2] = __builtin_bit_cast(V, u32x2{v1[0], v1[1]});
+      rec.val[3] = __builtin_bit_cast(V, u32x2{v1[2], v1[3]});
+      rec.val[4] = __builtin_bit_cast(V, u32x2{v2[0], v2[1]});
+      rec.s01 = v2[2];
+      rec.s23 = v2[3];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 5; ++e) rec.val[e] = __builtin_bit_cast(V, lds_read<u32x4>(a + e * 1024));
+      const u32x4 x = lds_read<u32x4>(a + 5 * 1024);
+      rec.s01 = x[0];
+      rec.s23 = x[1];
+      rec.s4 = x[2];
+    }
+    const unsigned d = stage * L::stage;
+    info = lds_read<u32x2>(info_a + d);
+    if constexpr (NCL == 2) {
+      const RingRow<V, 2> r = lds_read<RingRow<V, 2>>(rhs_a + d);
+      xin[0] = r.v[0];
+      xin[1] = r.v[1];
+    } else {
+      xin[0] = lds_read<V>(rhs_a + d);
+    }
+    if constexpr (UPPER) dv = lds_read<V>(piv_a + d);
+  };
+
+  __syncthreads();  // the loading waves have filled the first stages
+  take(0);
+  __syncthreads();  // step 0 is taken: its stage may be used again
+  for (int base = 0; base < nsteps; base += K) {
+#pragma unroll
+    for (int kk = 0; kk < K; ++kk) {
+      const unsigned sa[5] = {slot_addr<CG * VS, false>(rec.s01, gat), slot_addr<CG * VS, true>(rec.s01, gat),
+                              slot_addr<CG * VS, false>(rec.s23, gat), slot_addr<CG * VS, true>(rec.s23, gat),
+                              slot_addr<CG * VS, false>(rec.s4, gat)};
+      RingRow<V, CG> xv[5];
+      V wgt[5];
+#pragma unroll
+      for (int e = 0; e < 5; ++e) {
+        xv[e] = lds_read<RingRow<V, CG>>(sa[e]);
+        wgt[e] = rec.val[e];  // padded slots weigh zero
       }
-      const int slot = sw[k];
-      const int row = pr[k].col;
-      const V dv = pr[k].val;
-      const bool wr = s < s_end && slot >= 0 && writer;
-      V xin[NCL];
+      const unsigned wa = CG * NG == 1 ? info[0] : info[0] * CG + wad;
+      const int off = (int)((info[1] << sh) + coff);
+      V x0[NCL];
 #pragma unroll
-      for (int j = 0; j < NCL; ++j) xin[j] = xr[k][j];
+      for (int j = 0; j < NCL; ++j) x0[j] = xin[j];
+      const V d0 = dv;
+      // the next step's records and row data follow the gathers in the LDS queue
+      take((kk + 1) % K);
       V acc[CG];
 #pragma unroll
       for (int c = 0; c < CG; ++c) acc[c] = 0;
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) {
+      for (int e = 0; e < 5; ++e) {
 #pragma unroll
         for (int c = 0; c < CG; ++c) acc[c] += wgt[e] * xv[e].v[c];
       }
@@ -621,24 +793,12 @@ __device__ __forceinline__ void ring_sweep(int s_begin, int s_end, int sbeg, int
       if constexpr (CG == 8) {
         // xor 2: keep columns 0-3 (q bit 1 clear) or 4-7, send the other half
         const bool b0 = q & 1, b1 = q & 2;
-        V h[4];
+        V hh[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) h[c] = (b1 ? acc[c + 4] : acc[c]) + dpp_xor2(b1 ? acc[c] : acc[c + 4]);
+        for (int c = 0; c < 4; ++c) hh[c] = (b1 ? acc[c + 4] : acc[c]) + dpp_xor2(b1 ? acc[c] : acc[c + 4]);
         // xor 1: keep columns 0-1 of the half (q bit 0 clear) or 2-3
 #pragma unroll
-        for (int c = 0; c < 2; ++c) a[c] = (b0 ? h[c + 2] : h[c]) + dpp_xor1(b0 ? h[c] : h[c + 2]);
-      } else if constexpr (LPR == 2 && CG == 4) {
-        // xor 1: keep columns 0-1 (q = 0) or 2-3 (q = 1), send the other pair
-        const bool b0 = q & 1;
-#pragma unroll
-        for (int c = 0; c < 2; ++c) a[c] = (b0 ? acc[c + 2] : acc[c]) + dpp_xor1(b0 ? acc[c] : acc[c + 2]);
-      } else if constexpr (LPR == 2) {
-        if constexpr (CG == 2) {
-          const bool b0 = q & 1;
-          a[0] = (b0 ? acc[1] : acc[0]) + dpp_xor1(b0 ? acc[0] : acc[1]);
-        } else {
-          a[0] = pair_sum(acc[0]);
-        }
+        for (int c = 0; c < 2; ++c) a[c] = (b0 ? hh[c + 2] : hh[c]) + dpp_xor1(b0 ? hh[c] : hh[c + 2]);
       } else if constexpr (CG == 4) {
         // xor 1: keep columns with bit 0 = q bit 0, send the other two
         const bool b0 = q & 1, b1 = q & 2;
@@ -653,87 +813,79 @@ __device__ __forceinline__ void ring_sweep(int s_begin, int s_end, int sbeg, int
       } else {
         a[0] = quad_sum(acc[0]);
       }
-      // lanes with nothing to write store to the dummy LDS slot and out of
+      // with fewer than four columns several lanes hold and write the same
+      // value; lanes past the step's rows write the dummy ring row and past
       // the buffer's range (dropped): no branch
-      if constexpr (kPairIO) {
+      if constexpr (NCL == 2) {
         RingRow<V, 2> o;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          o.v[j] = xin[j] - a[j];
-          if (UPPER) o.v[j] *= dv;
+          o.v[j] = x0[j] - a[j];
+          if (UPPER) o.v[j] *= d0;
         }
-        *reinterpret_cast<RingRow<V, 2>*>(xs + (wr ? slot * CG + cl[0] : dummy)) = o;
-        bstore_val2<V>(rs_dst, wr ? ((row << csh) + c0 + cl[0]) * VS : 0x7ffffff0, o);
+        lds_write(wa, o);
+        bstore_val2<V>(rs_dst, off, o);
       } else {
-#pragma unroll
-        for (int j = 0; j < NCL; ++j) {
-          V v = xin[j] - a[j];
-          if (UPPER) v *= dv;
-          xs[wr ? slot * CG + cl[j] : dummy] = v;
-          bstore_val(rs_dst, wr ? ((row << csh) + c0 + cl[j]) * VS : 0x7ffffff0, v);
-        }
+        V v = x0[0] - a[0];
+        if (UPPER) v *= d0;
+        lds_write(wa, v);
+        bstore_val(rs_dst, off, v);
       }
-      // refill this stage with step s + D and load the right-hand side of
-      // step s + D/2, whose row pair arrived D/2 steps ago.  The refill
-      // follows the last use of the stage's registers, so the old and the
-      // new contents are never live together: the loop needs no register
-      // copies at its back edge, and no copy waits for a load in flight.
-      __builtin_amdgcn_sched_barrier(0);
-      PGS_RING_STAGE(k, dn[k]);
-      dn[k] = bload_i3(rs_desc, (s - sbeg + 2 * D) * 16);
-      PGS_RING_RHS((k + D / 2) % D);
-      if constexpr (NT == 64 && G == 1) {
-        // one wave: its LDS operations complete in issue order, so the next
-        // step's gathers see this step's writes without a wait or barrier;
-        // only the compiler must keep the order
-        __builtin_amdgcn_wave_barrier();
-        __asm__ __volatile__("" ::: "memory");
-      } else {
-        __syncthreads();
-      }
+      __syncthreads();
     }
   }
-#undef PGS_RING_STAGE
-#undef PGS_RING_PAIR
-#undef PGS_RING_ENT
-#undef PGS_RING_RHS
 }
 
-// G column groups of CG columns each share a workgroup of G * NT threads: the
-// groups walk the same steps in lockstep (one barrier per step), so their
-// identical loads of the block's entries and row pairs are served once by the
-// CU's L1 instead of each group streaming them from L2; each group has its own
-// ring in LDS.
-template <typename V, int NT, int LPR, int EPL, int D, int CG, int G>
-__global__ __launch_bounds__(NT * G) void k_trsv_ring(int nblocks, int wmask, const int* __restrict__ blk_row0,
-                                                  const int* __restrict__ blk_step, const int* __restrict__ blk_stepU,
-                                                  const int64_t* __restrict__ blk_ent0,
-                                                  const int64_t* __restrict__ blk_ri0, const int4* __restrict__ desc,
-                                                  const TPair<V>* __restrict__ ent, const TPair<V>* __restrict__ ri,
-                                                  const V* __restrict__ rhs, V* __restrict__ x, int nrhs) {
+// pos: per block b the boundaries of its steps (blk_step[b + 1] - blk_step[b] + 1
+// values from blk_step[b] + b; the first of them is 0, sU's the block's
+// rows).  info, dinv: per position the pair (ring slot times sizeof(V),
+// block-local row id) and 1/pivot, from blk_ri0[b], and the dummy row's pair
+// after the last block's; ent: the block's records, from blk_ri0[b] *
+// ring_row_bytes<V>().
+template <typename V, int K, int CG, int NG, int NH>
+__global__ __launch_bounds__(64 * (NH * NG + 2)) void k_trsv_ring(
+    int nblocks, int rows, const int* __restrict__ blk_row0, const int* __restrict__ blk_step,
+    const int* __restrict__ blk_stepU, const int64_t* __restrict__ blk_ri0, const int* __restrict__ pos,
+    const unsigned char* __restrict__ ent, const int2* __restrict__ info, const V* __restrict__ dinv,
+    const V* __restrict__ rhs, V* __restrict__ x, int nrhs) {
   extern __shared__ unsigned char smem_raw[];
-  const int grp = threadIdx.x / NT;
-  V* xs = reinterpret_cast<V*>(smem_raw) + grp * (wmask + 2) * CG;
-  const unsigned xsb = (unsigned)(grp * (wmask + 2) * CG * (int)sizeof(V));  // xs as an LDS byte address
   const int b = blockIdx.x % nblocks;
-  const int c0 = (blockIdx.x / nblocks) * CG * G + grp * CG;
+  const int c0 = (blockIdx.x / nblocks) * CG * NG;
   const int r0 = blk_row0[b], nb = blk_row0[b + 1] - r0;
   const int sbeg = blk_step[b], send = blk_step[b + 1], sU = blk_stepU[b];
-  const int64_t e0 = blk_ent0[b], e1 = blk_ent0[b + 1];
-  const int64_t q0 = blk_ri0[b], q1 = blk_ri0[b + 1];
-  const __amdgpu_buffer_rsrc_t rs_ent = make_rsrc(ent + e0, (e1 - e0) * (int64_t)sizeof(TPair<V>));
-  const __amdgpu_buffer_rsrc_t rs_ri = make_rsrc(ri + q0, (q1 - q0) * (int64_t)sizeof(TPair<V>));
-  const __amdgpu_buffer_rsrc_t rs_desc = make_rsrc(desc + sbeg, (int64_t)(send - sbeg) * 16);
+  const int64_t q0 = blk_ri0[b], np = blk_ri0[b + 1] - q0, nd = blk_ri0[nblocks] - q0;
+  const int* pb = pos + sbeg + b;
   const int64_t vbytes = (int64_t)nb * nrhs * (int64_t)sizeof(V);
   V* xb = x + (int64_t)r0 * nrhs;
-  V* xall = reinterpret_cast<V*>(smem_raw);
-  for (int i = threadIdx.x; i < (wmask + 2) * CG * G; i += NT * G) xall[i] = 0;  // rings + dummy slots
+  const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(xb, vbytes);
+  // rings, dummy rows and stages start as zeros: a record that is not there reads
+  // slot 0 with weight zero
+  uint4* lds4 = reinterpret_cast<uint4*>(smem_raw);
+  for (int i = threadIdx.x; i < RingLds<V, CG, NG, NH>::bytes(rows, K) / 16; i += 64 * (NH * NG + 2)) lds4[i] = uint4{0, 0, 0, 0};
   __syncthreads();
-  ring_sweep<V, NT, LPR, EPL, D, CG, false, G>(sbeg, sU, sbeg, wmask, nrhs, c0, rs_desc, rs_ri, rs_ent,
-                                               make_rsrc(rhs + (int64_t)r0 * nrhs, vbytes), xs, xsb,
-                                               make_rsrc(xb, vbytes));
-  ring_sweep<V, NT, LPR, EPL, D, CG, true, G>(sU, send, sbeg, wmask, nrhs, c0, rs_desc, rs_ri, rs_ent,
-                                              make_rsrc(xb, vbytes), xs, xsb, make_rsrc(xb, vbytes));
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (w < NH * NG) {
+    const int h = NH == 1 ? 0 : w % 2, g = NG == 1 ? 0 : w / NH;
+    ring_solve_sweep<V, K, CG, NG, NH, false>(h, g, sU - sbeg, rows, nrhs, c0, rs_x);
+    // y of every row has reached memory before the row data's wave reads it back (a
+    // barrier alone orders LDS, not one wave's stores before another's copies)
+    __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    ring_solve_sweep<V, K, CG, NG, NH, true>(h, g, send - sU, rows, nrhs, c0, rs_x);
+  } else if (w == NH * NG) {
+    const __amdgpu_buffer_rsrc_t rs_ent = make_rsrc(ent + q0 * ring_row_bytes<V>(), np * ring_row_bytes<V>());
+    ring_copy_sweep<V, K, CG, NG, NH>(sU - sbeg, pb, rows, rs_ent);
+    __syncthreads();
+    ring_copy_sweep<V, K, CG, NG, NH>(send - sU, pb + (sU - sbeg), rows, rs_ent);
+  } else {
+    const __amdgpu_buffer_rsrc_t rs_info = make_rsrc(info + q0, (nd + 1) * 8);
+    const __amdgpu_buffer_rsrc_t rs_dinv = make_rsrc(dinv + q0, np * (int64_t)sizeof(V));
+    const int dummy = (int)(nd * 8);
+    ring_row_sweep<V, K, CG, NG, NH, false>(sU - sbeg, pb, rows, nrhs, c0, dummy, rs_info, rs_dinv,
+                                        make_rsrc(rhs + (int64_t)r0 * nrhs, vbytes));
+    __syncthreads();
+    ring_row_sweep<V, K, CG, NG, NH, true>(send - sU, pb + (sU - sbeg), rows, nrhs, c0, dummy, rs_info, rs_dinv, rs_x);
+  }
 }
 
 }  // namespace dev
