@@ -309,13 +309,13 @@ struct pgs_ws_s {
   DevMem r0, x0, lrpart, lrt;
   std::vector<std::unique_ptr<DevMem>> zlev;
   // Krylov
-  DevMem V, Z, part, hbuf, h2buf, t2, H, cs, sn, rs, coef, upd, st, zflag, nb2, nr2, flag;
+  DevMem V, Z, part, hbuf, h2buf, H, cs, sn, rs, coef, upd, st, zflag, nb2, nr2;
   DevMem dc_d, dc_coef;  // delayed CGS2: the step's dot table and update coefficients
   DevMem dc_R;           // delayed CGS2: final basis in terms of the raw slots, (kdim+1)^2 per column
   DevMem dc_vscale;      // delayed CGS2: pending normalization of the newest basis vector, per column
   // inner Schur iteration: basis, preconditioned basis, temporaries (vectors
   // in the apply's precision) and its Hessenberg / Givens state per column
-  DevMem in_V, in_Z, in_T, in_U, in_Y, in_h, in_t2, in_H, in_cs, in_sn, in_rs, in_coef, in_upd, in_st, in_flag,
+  DevMem in_V, in_Z, in_T, in_U, in_Y, in_h, in_H, in_cs, in_sn, in_rs, in_coef, in_upd, in_st, in_flag,
       in_nb2;
   int* flag_host = nullptr;
   int part_blocks = 0;
@@ -356,7 +356,7 @@ constexpr int kPMAX = 128;  // Krylov dimension + 1 limit of the shared-memory c
 constexpr int kLrBlocks = 1024;  // most workgroups (partial sums) of the low-rank stage 1
 constexpr int kBasisNT = 256;
 constexpr int kBasisPM = 64;  // most basis vectors k_basis_reg takes
-constexpr int kPartRowsDcgs2 = 2 * 32 + 2;  // outputs per column of one k_dcgs2_dots chunk
+constexpr int kFixNT = 1024;  // threads of k_dcgs2_fix
 
 template <typename V>
 DevPrec<V>& prec_of(pgs_dev_op_s* op);
@@ -691,18 +691,9 @@ void set_kernel_attrs(int lds_max) {
     set_lds_limit(k_basis_reg<kBasisNT, 32, 0, 2>, lds_max);
     set_lds_limit(k_basis_reg<kBasisNT, 32, 1, 2>, lds_max);
     // coefficient tables of up to 127 x 64 values in LDS
-    set_lds_limit(k_dcgs2_update<double, kBasisNT, 8, 1>, lds_max);
-    set_lds_limit(k_dcgs2_update<double, kBasisNT, 16, 1>, lds_max);
-    set_lds_limit(k_dcgs2_update<double, kBasisNT, 32, 1>, lds_max);
-    set_lds_limit(k_dcgs2_update<double, kBasisNT, 32, 2>, lds_max);
-    set_lds_limit(k_dcgs2_update<double, kBasisNT, 64, 2>, lds_max);
+    set_lds_limit(k_dcgs2_update<double, kBasisNT, false>, lds_max);
     using Z = cplx<double>;
-    set_lds_limit(k_dcgs2_update<Z, kBasisNT, 8, 1>, lds_max);
-    set_lds_limit(k_dcgs2_update<Z, kBasisNT, 16, 1>, lds_max);
-    set_lds_limit(k_dcgs2_update<Z, kBasisNT, 16, 2>, lds_max);
-    set_lds_limit(k_dcgs2_update<Z, kBasisNT, 32, 2>, lds_max);
-    set_lds_limit(k_dcgs2_dots<Z, kBasisNT, 8, 1>, lds_max);
-    set_lds_limit(k_dcgs2_dots<Z, kBasisNT, 8, 2>, lds_max);
+    set_lds_limit(k_dcgs2_update<Z, kBasisNT, false>, lds_max);
     set_lds_limit(k_multi_axpy_norm<double, double, kNT>, lds_max);
     set_lds_limit(k_multi_axpy_norm<cplx<double>, cplx<double>, kNT>, lds_max);
     set_lds_limit(k_update_x<double, double>, lds_max);
@@ -800,18 +791,27 @@ void colnorm2(pgs_ws_s* ws, int64_t n, int nrhs, const S* x, double* out, hipStr
   HIPCHK(hipGetLastError());
 }
 
-// w -= V(:, 0:p) h; with t2, t2[c] = ||w(:, c)||^2 of the result.  V, w in
-// VV, h and the arithmetic in S.
+// w -= V(:, 0:p) h; with `norm`, partial sums of ||w(:, c)||^2 of the result
+// in ws->part.  V, w in VV, h and the arithmetic in S.  Returns the number of
+// workgroups.
 template <typename VV, typename S = VV>
-void multi_axpy(pgs_ws_s* ws, int64_t n, int nrhs, int p, const VV* V, int64_t ldv, const S* h, VV* w, double* t2,
-                hipStream_t s) {
+int multi_axpy(pgs_ws_s* ws, int64_t n, int nrhs, int p, const VV* V, int64_t ldv, const S* h, VV* w, bool norm,
+               hipStream_t s) {
   // enough workgroups to keep every CU busy on the streaming update
   const int nblk = (int)std::min<int64_t>(4096, std::max<int64_t>(1, (n * nrhs + kNT - 1) / kNT));
   const size_t shm = sizeof(S) * (size_t)p * nrhs + sizeof(double) * (kNT / 64) * nrhs;
   k_multi_axpy_norm<VV, S, kNT><<<nblk, kNT, shm, s>>>(n, nrhs, p, V, ldv, h, w,
-                                                       t2 ? ws->part.as<double>() : nullptr);
-  if (t2) k_dot_final_wave<<<(nrhs + 3) / 4, 256, 0, s>>>(nblk, 1, nrhs, ws->part.as<double>(), t2, 0);
+                                                       norm ? ws->part.as<double>() : nullptr);
   HIPCHK(hipGetLastError());
+  return nblk;
+}
+
+// k_givens after step i (1-based) of a cycle of m vectors, ||w||^2 in nblk partials
+template <typename S>
+void launch_givens(pgs_ws_s* ws, int nblk, int nrhs, int m, int i, int maxits, const S* h, const S* hadd, S* H, S* cs,
+                   S* sn, S* rs, KState* st, int* flag, hipStream_t s) {
+  k_givens<S><<<nrhs, kTailNT, sizeof(S) * 3 * i, s>>>(nblk, nrhs, m, i, maxits, h, hadd, ws->part.as<double>(), H,
+                                                       cs, sn, rs, st, flag);
 }
 
 template <typename V>
@@ -852,14 +852,13 @@ void inner_schur(pgs_dev_op_s* op, pgs_ws_s* ws, DevPrec<V>& P, const V* b, V* x
   V* U = ws->in_U.as<V>();
   V* Y = ws->in_Y.as<V>();
   S* h = ws->in_h.as<S>();
-  double* t2 = ws->in_t2.as<double>();
   S* H = ws->in_H.as<S>();
   S* rs = ws->in_rs.as<S>();
   KState* st = ws->in_st.as<KState>();
   // ||b||; x0 = 0, so the residual is b and normr = normb
   colnorm2<V>(ws, m, nrhs, b, ws->in_nb2.as<double>(), s);
-  k_fgmres_init<<<1, 64, 0, s>>>(nrhs, ws->in_nb2.as<double>(), ws->in_nb2.as<double>(), op->inner_tol, 0, st,
-                                 ws->in_flag.as<double>());
+  k_fgmres_init<<<1, 64, 0, s>>>(nrhs, ws->in_nb2.as<double>(), ws->in_nb2.as<double>(), op->inner_tol, 0, K, st,
+                                 ws->in_flag.as<double>(), nullptr);
   k_fill_zero<V><<<nb, kNT, 0, s>>>(ldv, x);
   // v0 = b / normb
   k_copy_conv<V, V><<<nb, kNT, 0, s>>>(ldv, b, Vb);
@@ -880,17 +879,17 @@ void inner_schur(pgs_dev_op_s* op, pgs_ws_s* ws, DevPrec<V>& P, const V* b, V* x
     launch_spmv<V, V, V, V>(L0.E, Y, w, (const V*)nullptr, V(-1.0), V(0.0), 0, nrhs, s);
     launch_spmv<V, V, V, V>(L0.C, zc, w, (const V*)nullptr, V(1.0), V(1.0), 0, nrhs, s);
     // modified Gram-Schmidt against v_0..v_{i-1}; ||w||^2 with the last update
+    int nblk = 0;
     for (int j = 0; j < i; ++j) {
       multidot<V, V, S>(ws, m, nrhs, 1, Vb + (int64_t)j * ldv, ldv, w, h + (int64_t)j * nrhs, 0, s);
-      multi_axpy<V, S>(ws, m, nrhs, 1, Vb + (int64_t)j * ldv, ldv, h + (int64_t)j * nrhs, w,
-                       j == i - 1 ? t2 : nullptr, s);
+      nblk = multi_axpy<V, S>(ws, m, nrhs, 1, Vb + (int64_t)j * ldv, ldv, h + (int64_t)j * nrhs, w, j == i - 1, s);
     }
-    k_givens<S><<<1, 64, 0, s>>>(nrhs, K, i, K, h, t2, H, ws->in_cs.as<S>(), ws->in_sn.as<S>(), rs, st);
+    launch_givens<S>(ws, nblk, nrhs, K, i, K, h, nullptr, H, ws->in_cs.as<S>(), ws->in_sn.as<S>(), rs, st, nullptr, s);
     k_scale_cols<V><<<nb, kNT, 0, s>>>(m, nrhs, st, w);
     HIPCHK(hipGetLastError());
   }
   // x = Z y over each column's steps
-  k_backsolve<S><<<1, 64, 0, s>>>(nrhs, K, H, rs, st, ws->in_coef.as<S>(), ws->in_upd.as<int>());
+  k_backsolve<S><<<nrhs, kWave, 0, s>>>(nrhs, K, H, rs, st, ws->in_coef.as<S>(), ws->in_upd.as<int>());
   k_update_x<V, S, V><<<nb, kNT, sizeof(S) * K * nrhs, s>>>(m, nrhs, K, Zb, ldv, ws->in_coef.as<S>(),
                                                             ws->in_upd.as<int>(), x);
   HIPCHK(hipGetLastError());
@@ -1050,6 +1049,10 @@ struct WsSizes {
 // multi-dots and norms use (level temporaries, partial sums, the low-rank
 // term's partials); no Krylov bases, Hessenberg state or inner-iteration
 // buffers.
+// partial sums per workgroup and column: kdim + 1 dots, or the 2 p + 2 of a
+// delayed-CGS2 step (66: the norms of an update by up to 4096 workgroups)
+size_t part_rows(int kdim) { return (size_t)std::max(2 * kdim + 2, 66); }
+
 WsSizes ws_sizes(const pgs_dev_op_s* op, int nr, int kdim, bool lowrank_build = false) {
   WsSizes z;
   const int64_t n = op->n;
@@ -1072,8 +1075,7 @@ WsSizes ws_sizes(const pgs_dev_op_s* op, int nr, int kdim, bool lowrank_build = 
   if (lowrank_build) {
     add(&pgs_ws_s::lrpart, (size_t)std::max(1, (kLrBlocks + 1) * maxrank * nr) * es);
     add(&pgs_ws_s::lrt, (size_t)std::max(1, maxrank * nr) * es);
-    add(&pgs_ws_s::part, (size_t)z.part_blocks * std::max(kdim + 1, kPartRowsDcgs2) * nr * es);
-    add(&pgs_ws_s::flag, 16);
+    add(&pgs_ws_s::part, (size_t)z.part_blocks * part_rows(kdim) * nr * es);
     return z;
   }
   add(&pgs_ws_s::r0, vb);
@@ -1082,11 +1084,9 @@ WsSizes ws_sizes(const pgs_dev_op_s* op, int nr, int kdim, bool lowrank_build = 
   add(&pgs_ws_s::lrt, (size_t)std::max(1, maxrank * nr) * es);
   add(&pgs_ws_s::V, (ik + 1) * (vb + kBasisPad * es));
   add(&pgs_ws_s::Z, ik * (vb + kBasisPad * es));
-  // partial rows per workgroup: kdim + 1 dots, or 2 * 32 + 2 of a delayed-CGS2 dot chunk
-  add(&pgs_ws_s::part, (size_t)z.part_blocks * std::max(kdim + 1, kPartRowsDcgs2) * nr * es);
+  add(&pgs_ws_s::part, (size_t)z.part_blocks * part_rows(kdim) * nr * es);
   add(&pgs_ws_s::hbuf, (ik + 1) * nr * es);
   add(&pgs_ws_s::h2buf, (ik + 1) * nr * es);
-  add(&pgs_ws_s::t2, (size_t)nr * sizeof(double));
   add(&pgs_ws_s::H, (size_t)nr * (ik + 1) * ik * es);
   add(&pgs_ws_s::cs, (size_t)nr * ik * es);
   add(&pgs_ws_s::sn, (size_t)nr * ik * es);
@@ -1101,7 +1101,6 @@ WsSizes ws_sizes(const pgs_dev_op_s* op, int nr, int kdim, bool lowrank_build = 
   add(&pgs_ws_s::zflag, (size_t)nr * sizeof(double));
   add(&pgs_ws_s::nb2, (size_t)nr * sizeof(double));
   add(&pgs_ws_s::nr2, (size_t)nr * sizeof(double));
-  add(&pgs_ws_s::flag, 16);
   if (op->inner_maxits > 0) {
     // inner Schur iteration: basis, preconditioned basis and temporaries of
     // the level-0 remainder (m0) and of level 0 (nl0); its scalars are
@@ -1114,7 +1113,6 @@ WsSizes ws_sizes(const pgs_dev_op_s* op, int nr, int kdim, bool lowrank_build = 
     add(&pgs_ws_s::in_U, nl0 * nr * es);
     add(&pgs_ws_s::in_Y, nl0 * nr * es);
     add(&pgs_ws_s::in_h, K * nr * es);
-    add(&pgs_ws_s::in_t2, (size_t)nr * sizeof(double));
     add(&pgs_ws_s::in_H, (size_t)nr * (K + 1) * K * es);
     add(&pgs_ws_s::in_cs, (size_t)nr * K * es);
     add(&pgs_ws_s::in_sn, (size_t)nr * K * es);
@@ -1259,7 +1257,7 @@ int ws_create(pgs_dev_op_s* op, int max_nrhs, int kdim, bool lowrank_build, pgs_
       ws->zlev.push_back(std::move(m));
     }
     for (const auto& e : z.bufs) (ws.get()->*(e.first)).alloc(e.second);
-    HIPCHK(hipHostMalloc((void**)&ws->flag_host, 16, hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void**)&ws->flag_host, sizeof(int) * nr, hipHostMallocCoherent));
   } catch (const HipError& e) {
     return set_err(e);
   }
@@ -1379,11 +1377,12 @@ bool basis_fits(const pgs_ws_s* ws, int p, int nrhs) {
 
 // One sweep of k_basis_reg over V_0..V_{p-1} (basis_fits must hold): mode 0
 // out[j, c] = V_j^T w; mode 1 w -= V h, then out[j, c] = V_j^T w; mode 2
-// w -= V h, then out[c] = ||w(:, c)||^2.  Past 32 vectors the dot sweeps
+// w -= V h, the partial sums of ||w(:, c)||^2 left in ws->part.  Returns the
+// number of workgroups.  Past 32 vectors the dot sweeps
 // spread an element over two lanes (32 basis values each) to keep register
 // use, and with it occupancy, at the level of the 32-vector case.
-void basis_reg(pgs_ws_s* ws, int64_t n, int nrhs, int p, const double* V, int64_t ldv, const double* h, double* w,
-               double* out, int mode, hipStream_t s) {
+int basis_reg(pgs_ws_s* ws, int64_t n, int nrhs, int p, const double* V, int64_t ldv, const double* h, double* w,
+              double* out, int mode, hipStream_t s) {
   const int q = mode == 2 ? 1 : p;
   const size_t lds = basis_lds(p, nrhs, mode);
   const int lds_max = ws->op->lds_max;
@@ -1403,8 +1402,9 @@ void basis_reg(pgs_ws_s* ws, int64_t n, int nrhs, int p, const double* V, int64_
   else if (two) PGS_BASIS(32, 2);
   else PGS_BASIS(64, 1);
 #undef PGS_BASIS
-  k_dot_final_wave<<<(q * nrhs + 3) / 4, 256, 0, s>>>(nblk, q, nrhs, part, out, 0);
+  if (mode != 2) k_dot_final_wave<<<(q * nrhs + 3) / 4, 256, 0, s>>>(nblk, q, nrhs, part, out, 0);
   HIPCHK(hipGetLastError());
+  return nblk;
 }
 
 // apply arithmetic of the two preconditioner precisions for Krylov scalar S
@@ -1421,69 +1421,61 @@ struct PrecTypes<cplx<double>> {
 
 // FGMRES (FlexGmresClass::Solve, fgmres.hpp:300-540) on nrhs columns at once:
 // Krylov scalar S (double or complex<double>), preconditioned basis Z in VZ.
-// Delayed CGS2, dots of step p: d = [s (p rows) | a (p rows) | q.q | q.w]
+// Delayed CGS2, dots of step p: the table [s (p rows) | a (p rows) | q.q | q.w]
 // with s = V_{0..p-1}^H q, a = V_{0..p-1}^H w, q = basis slot p; with w ==
-// nullptr (the closing pass of a cycle) d = [s | q.q].  The basis is read in
-// chunks of 16 vectors per lane for real values, 8 for complex ones (two
-// lanes per element up to 32 columns).
+// nullptr (the closing pass of a cycle) [s | q.q].  Returns the number of
+// partial tables left in ws->part for k_dcgs2_fix to sum, or 0 with their sum
+// in d: the fix reads them with one workgroup per column, which beats a launch
+// of its own (4 to 5 us) while they are few (at 128, 4 complex columns, about
+// 3 us more of the fix; at 1024 it would be a CU's 10 us and more).
+constexpr int kFixPartials = 128;
+
 template <typename S>
-void dcgs2_dots(pgs_ws_s* ws, int64_t n, int nrhs, int p, const S* V, int64_t ldv, const S* w, S* d,
-                hipStream_t s) {
-  constexpr int PM = scalar_traits<S>::is_complex ? 8 : 16;
+int dcgs2_dots(pgs_ws_s* ws, int64_t n, int nrhs, int p, const S* V, int64_t ldv, const S* w, S* d,
+               hipStream_t s) {
   const S* q = V + (int64_t)p * ldv;
-  // two lanes per element up to 32 columns; at 64 columns one lane per
-  // element runs faster although its chunks of 16 vectors read q and w twice
-  // as often (128^3, 64 columns: 478 against 500 ms of dots per two solves)
-  const int lpe = nrhs <= 32 ? 2 : 1;
-  const int chunk = PM * lpe;
-  const int64_t nthr = (n * nrhs * lpe + kBasisNT - 1) / kBasisNT;
+  constexpr int E = 16 / (int)sizeof(S);
+  const int64_t nthr = (n * nrhs + kWave * E - 1) / (kWave * E);
   const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(ws->part_blocks, nthr));
-  const int hw = w != nullptr;
+  // equal chunks: a short last one would leave too few loads in flight
+  const int nch = std::max(1, (p + kDotsChunk - 1) / kDotsChunk);
+  const int chunk = (p + nch - 1) / nch;
+  const dim3 grid(nblk, nch);
+  const int nout = w != nullptr ? 2 * p + 2 : p + 1;
   S* part = ws->part.as<S>();
-  for (int j0 = 0; j0 == 0 || j0 < p; j0 += chunk) {
-    const int cnt = std::min(chunk, p - j0);
-    const int first = j0 == 0;
-    const int nout = (hw ? 2 * cnt : cnt) + (first ? (hw ? 2 : 1) : 0);
-    const size_t lds = sizeof(S) * (size_t)nout * nrhs;
-    if (lpe == 2)
-      k_dcgs2_dots<S, kBasisNT, PM, 2><<<nblk, kBasisNT, lds, s>>>(n, nrhs, j0, cnt, V, ldv, q, w, first, part);
-    else
-      k_dcgs2_dots<S, kBasisNT, PM, 1><<<nblk, kBasisNT, lds, s>>>(n, nrhs, j0, cnt, V, ldv, q, w, first, part);
-    k_dcgs2_final<S><<<(nout * nrhs + 3) / 4, 256, 0, s>>>(nblk, nout, cnt, nrhs, hw, p, j0, part, d);
-  }
+  if (E == 2 && nrhs == 1) k_dcgs2_dots<S, E == 2><<<grid, kDotsNT, 0, s>>>(n, nrhs, p, chunk, V, ldv, q, w, part);
+  else k_dcgs2_dots<S, false><<<grid, kDotsNT, 0, s>>>(n, nrhs, p, chunk, V, ldv, q, w, part);
+  if (nblk > kFixPartials) dot_final<S>(nblk, nout, nrhs, part, d, 0, s);
+  HIPCHK(hipGetLastError());
+  return nblk > kFixPartials ? 0 : nblk;
+}
+
+// Delayed CGS2, k_dcgs2_fix after the dots of step p (nblk as dcgs2_dots returned it)
+template <typename S>
+void dcgs2_fix(pgs_ws_s* ws, int nrhs, int m, int p, int maxits, bool final_pass, int nblk, const double* vscale,
+               int* flag, hipStream_t s) {
+  k_dcgs2_fix<S, kFixNT><<<nrhs, kFixNT, sizeof(S) * fix_lds(p, kFixNT), s>>>(
+      nrhs, m, p, maxits, final_pass ? 1 : 0, nblk, nblk > 0 ? ws->part.as<S>() : ws->dc_d.as<S>(), ws->H.as<S>(),
+      ws->cs.as<S>(), ws->sn.as<S>(), ws->rs.as<S>(), ws->st.as<KState>(), ws->dc_coef.as<S>(), vscale,
+      ws->dc_R.as<S>(), flag);
   HIPCHK(hipGetLastError());
 }
 
 // Delayed CGS2, update of step p (k_dcgs2_update: w minus its projection on
-// the final basis v_0..v_p, in terms of the raw slots 0..p), then
-// t2[c] = ||w(:, c)||^2.
-// Real values: one lane per element up to 32 vectors, then two (the one-lane
-// 64-vector kernel needs more than 256 VGPRs); complex values (twice the
-// registers per vector): one lane up to 16 vectors, then two, at most 64.
+// the final basis v_0..v_p, in terms of the raw slots 0..p); returns the
+// number of partial sums of ||w(:, c)||^2 left in ws->part.
 template <typename S>
-void dcgs2_update(pgs_ws_s* ws, int64_t n, int nrhs, int p, const S* V, int64_t ldv, const S* q, S* w,
-                  const S* coef, double* t2, hipStream_t s) {
-  constexpr bool cx = scalar_traits<S>::is_complex;
-  const bool two = cx ? p > 16 : p > 32;
-  const int64_t nthr = (n * nrhs * (two ? 2 : 1) + kBasisNT - 1) / kBasisNT;
+int dcgs2_update(pgs_ws_s* ws, int64_t n, int nrhs, int p, const S* V, int64_t ldv, const S* q, S* w,
+                 const S* coef, hipStream_t s) {
+  constexpr int E = 16 / (int)sizeof(S);
+  const int64_t nthr = (n * nrhs + kBasisNT * E - 1) / (kBasisNT * E);
   const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(ws->part_blocks, nthr));
-  const size_t lds = sizeof(S) * (size_t)(p + 1) * nrhs + sizeof(double) * (size_t)(kBasisNT / kWave) * nrhs;
+  const size_t lds = sizeof(S) * (size_t)(p + 1) * nrhs + sizeof(double) * ((size_t)(kBasisNT / kWave) * nrhs + 1);
   double* part = ws->part.as<double>();
-  if constexpr (cx) {
-    if (p <= 8) k_dcgs2_update<S, kBasisNT, 8, 1><<<nblk, kBasisNT, lds, s>>>(n, nrhs, p, V, ldv, q, w, coef, part);
-    else if (p <= 16) k_dcgs2_update<S, kBasisNT, 16, 1><<<nblk, kBasisNT, lds, s>>>(n, nrhs, p, V, ldv, q, w, coef, part);
-    else if (p <= 32) k_dcgs2_update<S, kBasisNT, 16, 2><<<nblk, kBasisNT, lds, s>>>(n, nrhs, p, V, ldv, q, w, coef, part);
-    else if (p <= 64) k_dcgs2_update<S, kBasisNT, 32, 2><<<nblk, kBasisNT, lds, s>>>(n, nrhs, p, V, ldv, q, w, coef, part);
-    else throw std::runtime_error("delayed CGS2: complex bases hold at most 64 vectors");
-  } else {
-    if (p <= 8) k_dcgs2_update<S, kBasisNT, 8, 1><<<nblk, kBasisNT, lds, s>>>(n, nrhs, p, V, ldv, q, w, coef, part);
-    else if (p <= 16) k_dcgs2_update<S, kBasisNT, 16, 1><<<nblk, kBasisNT, lds, s>>>(n, nrhs, p, V, ldv, q, w, coef, part);
-    else if (p <= 32) k_dcgs2_update<S, kBasisNT, 32, 1><<<nblk, kBasisNT, lds, s>>>(n, nrhs, p, V, ldv, q, w, coef, part);
-    else if (p <= 64) k_dcgs2_update<S, kBasisNT, 32, 2><<<nblk, kBasisNT, lds, s>>>(n, nrhs, p, V, ldv, q, w, coef, part);
-    else k_dcgs2_update<S, kBasisNT, 64, 2><<<nblk, kBasisNT, lds, s>>>(n, nrhs, p, V, ldv, q, w, coef, part);
-  }
-  k_dot_final_wave<<<(nrhs + 3) / 4, 256, 0, s>>>(nblk, 1, nrhs, part, t2, 0);
+  if (nrhs == 1) k_dcgs2_update<S, kBasisNT, true><<<nblk, kBasisNT, lds, s>>>(n, nrhs, p, V, ldv, q, w, coef, part);
+  else k_dcgs2_update<S, kBasisNT, false><<<nblk, kBasisNT, lds, s>>>(n, nrhs, p, V, ldv, q, w, coef, part);
   HIPCHK(hipGetLastError());
+  return nblk;
 }
 
 template <typename S, typename VZ>
@@ -1509,20 +1501,19 @@ int fgmres_impl(pgs_dev_op_s* op, pgs_ws_s* ws, const S* b, S* x, int nrhs, cons
   timed(ws, s, PGS_PROF_SPMV_A, spmv_bytes<S, S, S>(op->A, nrhs, true),
         [&] { launch_spmv<S, S, S, S>(op->A, x, V, b, S(1.0), S(0.0), 1, nrhs, s); });
   colnorm2<S>(ws, n, nrhs, V, ws->nr2.as<double>(), s);
-  k_fgmres_init<<<1, 64, 0, s>>>(nrhs, ws->nb2.as<double>(), ws->nr2.as<double>(), o.tol, o.absolute_tol, st,
-                                 ws->zflag.as<double>());
+  k_fgmres_init<<<1, 64, 0, s>>>(nrhs, ws->nb2.as<double>(), ws->nr2.as<double>(), o.tol, o.absolute_tol,
+                                 maxits, st, ws->zflag.as<double>(), ws->flag_host);
   k_zero_cols<S><<<nb, kNT, 0, s>>>(n, nrhs, ws->zflag.as<double>(), x);
   HIPCHK(hipGetLastError());
-  int* hflag = ws->flag_host;
-  // number of running (restartable) or active columns, read back through pinned memory
-  auto read_flag = [&](bool running) -> int {
-    if (running)
-      k_count_running<<<1, 1, 0, s>>>(nrhs, st, maxits, ws->flag.as<int>());
-    else
-      k_count_active<<<1, 1, 0, s>>>(nrhs, st, ws->flag.as<int>());
-    HIPCHK(hipMemcpyAsync(hflag, ws->flag.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    return hflag[0];
+  // number of columns with a state bit set, once the launches so far are done
+  // (each step's last kernel writes its columns' states into host memory);
+  // no wait when the last one read is still the newest
+  auto columns = [&](int bit, bool wait = true) -> int {
+    if (wait) HIPCHK(hipStreamSynchronize(s));
+    const volatile int* f = ws->flag_host;
+    int cnt = 0;
+    for (int c = 0; c < nrhs; ++c) cnt += (f[c] & bit) != 0;
+    return cnt;
   };
   // inner step i of a cycle: z = M^{-1} v_{i-1}, w = A z, orthogonalize w
   // against v_0..v_{i-1}, Givens update, v_i = w / ||w||; every launch on
@@ -1548,28 +1539,29 @@ int fgmres_impl(pgs_dev_op_s* op, pgs_ws_s* ws, const S* b, S* x, int nrhs, cons
           [&] { launch_spmv<S, VZ, S, S>(op->A, zc, w, (const S*)nullptr, S(1.0), S(0.0), 0, nrhs, ss); });
     S* h = ws->hbuf.as<S>();
     S* h2 = ws->h2buf.as<S>();
-    double* t2 = ws->t2.as<double>();
     if (dcgs2) {
       // delayed CGS2: finalize v_{i-1} (and Hessenberg column i-2, with its
       // Givens update) from the dots of this sweep, then project w once.
       // The slots keep the raw vectors; the final basis is carried by R
       // (k_dcgs2_fix), so the update writes w alone
       const int p = i - 1;
-      S* d = ws->dc_d.as<S>();
       S* coef = ws->dc_coef.as<S>();
       const double vb = (double)n * nrhs * sizeof(S);
-      timed(ws, ss, PGS_PROF_ORTH_DOTS, (p + 2.0) * vb, [&] { dcgs2_dots<S>(ws, n, nrhs, p, V, ldv, w, d, ss); });
-      timed(ws, ss, PGS_PROF_STATE, 0.0, [&] {
-        k_dcgs2_fix<S><<<nrhs, kWave, sizeof(S) * 2 * std::max(p, 1), ss>>>(
-            nrhs, m, p, maxits, 0, d, H, ws->cs.as<S>(), ws->sn.as<S>(), rs, st, coef, vsc, ws->dc_R.as<S>());
-      });
+      int nblk = 0;
+      timed(ws, ss, PGS_PROF_ORTH_DOTS, (p + 2.0) * vb,
+            [&] { nblk = dcgs2_dots<S>(ws, n, nrhs, p, V, ldv, w, ws->dc_d.as<S>(), ss); });
+      timed(ws, ss, PGS_PROF_STATE, 0.0, [&] { dcgs2_fix<S>(ws, nrhs, m, p, maxits, false, nblk, vsc, nullptr, ss); });
       timed(ws, ss, PGS_PROF_ORTH_UPDATE, (p + 3.0) * vb,
-            [&] { dcgs2_update<S>(ws, n, nrhs, p, V, ldv, vprev, w, coef, t2, ss); });
-      timed(ws, ss, PGS_PROF_STATE, 0.0,
-            [&] { k_dcgs2_norm<S><<<1, 64, 0, ss>>>(nrhs, m, p, t2, H, st, ws->dc_vscale.as<double>()); });
+            [&] { nblk = dcgs2_update<S>(ws, n, nrhs, p, V, ldv, vprev, w, coef, ss); });
+      timed(ws, ss, PGS_PROF_STATE, 0.0, [&] {
+        k_dcgs2_norm<S><<<nrhs, kTailNT, 0, ss>>>(nblk, nrhs, m, p, maxits, ws->part.as<double>(), H, st,
+                                                  ws->dc_vscale.as<double>(), ws->flag_host);
+      });
       HIPCHK(hipGetLastError());
       return;
     }
+    int nblk = 0;           // partials of ||w||^2
+    const S* hadd = nullptr;  // the second pass's coefficients
     if (o.orth == PGS_ORTH_CGS2 || o.orth == PGS_ORTH_DCGS2) {
       // PargemslrCgs2 (matrixops.cpp:10588-10709): two projection passes, the
       // norm of the result accumulated by the second update.  Three sweeps
@@ -1583,18 +1575,18 @@ int fgmres_impl(pgs_dev_op_s* op, pgs_ws_s* ws, const S* b, S* x, int nrhs, cons
           timed(ws, ss, PGS_PROF_ORTH_UPDATE, (i + 2.0) * vb,
                 [&] { basis_reg(ws, n, nrhs, i, V, ldv, h, w, h2, 1, ss); });
           timed(ws, ss, PGS_PROF_ORTH_UPDATE, (i + 2.0) * vb,
-                [&] { basis_reg(ws, n, nrhs, i, V, ldv, h2, w, t2, 2, ss); });
+                [&] { nblk = basis_reg(ws, n, nrhs, i, V, ldv, h2, w, nullptr, 2, ss); });
           fused = true;
         }
       }
       if (!fused) {
         const double vb = (double)n * nrhs * sizeof(S);
         timed(ws, ss, PGS_PROF_ORTH_DOTS, (i + 1.0) * vb, [&] { multidot<S, S, S>(ws, n, nrhs, i, V, ldv, w, h, 0, ss); });
-        timed(ws, ss, PGS_PROF_ORTH_UPDATE, (i + 2.0) * vb, [&] { multi_axpy<S>(ws, n, nrhs, i, V, ldv, h, w, nullptr, ss); });
+        timed(ws, ss, PGS_PROF_ORTH_UPDATE, (i + 2.0) * vb, [&] { multi_axpy<S>(ws, n, nrhs, i, V, ldv, h, w, false, ss); });
         timed(ws, ss, PGS_PROF_ORTH_DOTS, (i + 1.0) * vb, [&] { multidot<S, S, S>(ws, n, nrhs, i, V, ldv, w, h2, 0, ss); });
-        timed(ws, ss, PGS_PROF_ORTH_UPDATE, (i + 2.0) * vb, [&] { multi_axpy<S>(ws, n, nrhs, i, V, ldv, h2, w, t2, ss); });
+        timed(ws, ss, PGS_PROF_ORTH_UPDATE, (i + 2.0) * vb, [&] { nblk = multi_axpy<S>(ws, n, nrhs, i, V, ldv, h2, w, true, ss); });
       }
-      dot_final<S>(1, i, nrhs, h2, h, 1, ss);
+      hadd = h2;
     } else {
       // PargemslrMgs (matrixops.cpp:10728-10807): one (dot, axpy) pair per basis vector
       const double vb = (double)n * nrhs * sizeof(S);
@@ -1603,14 +1595,13 @@ int fgmres_impl(pgs_dev_op_s* op, pgs_ws_s* ws, const S* b, S* x, int nrhs, cons
           multidot<S, S, S>(ws, n, nrhs, 1, V + (int64_t)j * ldv, ldv, w, h + (int64_t)j * nrhs, 0, ss);
         });
         timed(ws, ss, PGS_PROF_ORTH_UPDATE, 3.0 * vb, [&] {
-          multi_axpy<S>(ws, n, nrhs, 1, V + (int64_t)j * ldv, ldv, h + (int64_t)j * nrhs, w,
-                        j == i - 1 ? t2 : nullptr, ss);
+          nblk = multi_axpy<S>(ws, n, nrhs, 1, V + (int64_t)j * ldv, ldv, h + (int64_t)j * nrhs, w, j == i - 1, ss);
         });
       }
     }
     timed(ws, ss, PGS_PROF_STATE, 0.0, [&] {
-      k_givens<S><<<1, 64, 0, ss>>>(nrhs, m, i, maxits, h, ws->t2.as<double>(), H, ws->cs.as<S>(), ws->sn.as<S>(),
-                                    rs, st);
+      launch_givens<S>(ws, nblk, nrhs, m, i, maxits, h, hadd, H, ws->cs.as<S>(), ws->sn.as<S>(), rs, st,
+                       ws->flag_host, ss);
     });
     timed(ws, ss, PGS_PROF_SCALE, 2.0 * (double)n * nrhs * sizeof(S),
           [&] { k_scale_cols<S><<<nb, kNT, 0, ss>>>(n, nrhs, st, w); });
@@ -1630,8 +1621,8 @@ int fgmres_impl(pgs_dev_op_s* op, pgs_ws_s* ws, const S* b, S* x, int nrhs, cons
     }
   }
   int iters_host = 0;
-  while (true) {
-    if (read_flag(true) == 0) break;
+  bool more = columns(kStateRunning) > 0;
+  while (more) {
     k_cycle_start<S><<<1, 64, 0, s>>>(nrhs, m, st, rs, dcgs2 ? ws->dc_vscale.as<double>() : nullptr);
     k_scale_cols<S><<<nb, kNT, 0, s>>>(n, nrhs, st, V);
     int i = 0;
@@ -1665,35 +1656,34 @@ int fgmres_impl(pgs_dev_op_s* op, pgs_ws_s* ws, const S* b, S* x, int nrhs, cons
         inner_step(i, s);
       }
       if (i % check == 0 || i == m) {
-        if (read_flag(false) == 0) {
+        if (columns(kStateActive) == 0) {
           none_active = true;
           break;
         }
       }
     }
-    if (dcgs2 && !none_active) {
+    const bool closing = dcgs2 && !none_active;
+    if (closing) {
       // close the cycle: finalize the last basis vector and Hessenberg
       // column of the columns still running (one more dot sweep)
-      S* d = ws->dc_d.as<S>();
+      int nblk = 0;
       timed(ws, s, PGS_PROF_ORTH_DOTS, (i + 1.0) * (double)n * nrhs * sizeof(S),
-            [&] { dcgs2_dots<S>(ws, n, nrhs, i, V, ldv, nullptr, d, s); });
+            [&] { nblk = dcgs2_dots<S>(ws, n, nrhs, i, V, ldv, nullptr, ws->dc_d.as<S>(), s); });
       timed(ws, s, PGS_PROF_STATE, 0.0, [&] {
-        k_dcgs2_fix<S><<<nrhs, kWave, sizeof(S) * 2 * std::max(i, 1), s>>>(
-            nrhs, m, i, maxits, 1, d, H, ws->cs.as<S>(), ws->sn.as<S>(), rs, st, ws->dc_coef.as<S>(),
-            ws->dc_vscale.as<double>(), ws->dc_R.as<S>());
+        dcgs2_fix<S>(ws, nrhs, m, i, maxits, true, nblk, ws->dc_vscale.as<double>(), ws->flag_host, s);
       });
-      HIPCHK(hipGetLastError());
     }
     // x += Z y
     timed(ws, s, PGS_PROF_STATE, 0.0,
-          [&] { k_backsolve<S><<<1, 64, 0, s>>>(nrhs, m, H, rs, st, ws->coef.as<S>(), ws->upd.as<int>()); });
+          [&] { k_backsolve<S><<<nrhs, kWave, 0, s>>>(nrhs, m, H, rs, st, ws->coef.as<S>(), ws->upd.as<int>()); });
     timed(ws, s, PGS_PROF_UPDATE_X, (double)n * nrhs * ((double)i * sizeof(VZ) + 2.0 * sizeof(S)), [&] {
       k_update_x<VZ, S><<<nb, kNT, sizeof(S) * std::max(1, i) * nrhs, s>>>(n, nrhs, i, Z, ldv, ws->coef.as<S>(),
                                                                           ws->upd.as<int>(), x);
     });
     HIPCHK(hipGetLastError());
     if (iters_host >= maxits) break;
-    if (read_flag(true) == 0) break;
+    more = columns(kStateRunning, closing) > 0;
+    if (!more) break;
     // restart: v0 = b - A x (fgmres.hpp:500-514); normr keeps the Givens estimate
     timed(ws, s, PGS_PROF_SPMV_A, spmv_bytes<S, S, S>(op->A, nrhs, true),
           [&] { launch_spmv<S, S, S, S>(op->A, x, V, b, S(1.0), S(0.0), 1, nrhs, s); });
@@ -2252,7 +2242,7 @@ struct DevLrBackend final : LrBackend<T> {
     HIPCHK(hipMemcpy(hd.p, h, sizeof(V) * (size_t)(j + 1), hipMemcpyHostToDevice));
     for (int q0 = 0; q0 <= j; q0 += kChunk) {
       const int pc = std::min(kChunk, j + 1 - q0);
-      multi_axpy<V, V>(ws, m, 1, pc, col(q0), m, hd.as<V>() + q0, col(j + 1), nullptr, s);
+      multi_axpy<V, V>(ws, m, 1, pc, col(q0), m, hd.as<V>() + q0, col(j + 1), false, s);
     }
   }
   double norm(int j) override {

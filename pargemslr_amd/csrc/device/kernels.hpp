@@ -24,6 +24,72 @@ __device__ __forceinline__ cplx<R> shfl_xor_v(cplx<R> v, int m, int width = kWav
   return cplx<R>(__shfl_xor(v.re, m, width), __shfl_xor(v.im, m, width));
 }
 
+// One step of a sum over lanes: v plus the value of lane ^ M, by lane
+// permutes of the vector unit (a ds_bpermute shuffle of a double is two LDS
+// round trips).  M = 4 rotates a row of 16 lanes by 4, which is the same once
+// the M = 8 step has made the row repeat after 8 lanes: the steps are taken
+// from M = 32 down.
+template <int M>
+__device__ __forceinline__ double lane_step(double v) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)u, hi = (unsigned)(u >> 32);
+  if constexpr (M >= 16) {
+    auto swap = [](unsigned x) {
+      if constexpr (M == 32) return __builtin_amdgcn_permlane32_swap(x, x, false, false);
+      else return __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    };
+    const auto l = swap(lo);
+    const auto h = swap(hi);
+    const unsigned l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1];
+    return __builtin_bit_cast(double, (unsigned long long)h0 << 32 | l0) +
+           __builtin_bit_cast(double, (unsigned long long)h1 << 32 | l1);
+  } else {
+    constexpr int ctrl = M == 8 ? 0x128 : M == 4 ? 0x124 : M == 2 ? 0x4E : 0xB1;  // row_ror, quad_perm
+    const unsigned l = (unsigned)__builtin_amdgcn_mov_dpp((int)lo, ctrl, 0xF, 0xF, true);
+    const unsigned h = (unsigned)__builtin_amdgcn_mov_dpp((int)hi, ctrl, 0xF, 0xF, true);
+    return v + __builtin_bit_cast(double, (unsigned long long)h << 32 | l);
+  }
+}
+template <int M, typename R>
+__device__ __forceinline__ cplx<R> lane_step(cplx<R> v) {
+  return cplx<R>(lane_step<M>(v.re), lane_step<M>(v.im));
+}
+
+// Sums each of the K values over the lanes that share lane % nl (nl a power
+// of two, at most 64); every lane gets its class's sum.
+template <int K, typename V>
+__device__ __forceinline__ void lane_class_sums(V (&a)[K], int nl) {
+#define PGS_LANE_STEP(M)                                \
+  if (M >= nl) {                                        \
+    _Pragma("unroll") for (int u = 0; u < K; ++u) a[u] = lane_step<M>(a[u]); \
+  }
+  PGS_LANE_STEP(32)
+  PGS_LANE_STEP(16)
+  PGS_LANE_STEP(8)
+  PGS_LANE_STEP(4)
+  PGS_LANE_STEP(2)
+  PGS_LANE_STEP(1)
+#undef PGS_LANE_STEP
+}
+template <typename V>
+__device__ __forceinline__ V lane_class_sum(V v, int nl) {
+  V a[1] = {v};
+  lane_class_sums<1>(a, nl);
+  return a[0];
+}
+
+// the value of lane `src` (the same in all lanes)
+__device__ __forceinline__ double lane_value(double v, int src) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)u, src);
+  const unsigned hi = __builtin_amdgcn_readlane((unsigned)(u >> 32), src);
+  return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+template <typename R>
+__device__ __forceinline__ cplx<R> lane_value(cplx<R> v, int src) {
+  return cplx<R>(lane_value(v.re, src), lane_value(v.im, src));
+}
+
 template <typename To, typename From>
 __device__ __forceinline__ To cvt(From v) { return (To)v; }
 
@@ -476,6 +542,45 @@ struct KState {
   int icur;     // inner steps of the current cycle
 };
 
+// A column's state for the host: kStateActive while it runs in the current
+// cycle, kStateRunning while it may go on in another one.  The kernel that
+// settles a step's state writes it for its column straight into host memory.
+constexpr int kStateActive = 1, kStateRunning = 2;
+__device__ __forceinline__ int state_bits(const KState& s, int maxits) {
+  return (s.active ? kStateActive : 0) | (s.status == 0 && s.iters < maxits ? kStateRunning : 0);
+}
+
+// The first p - 1 rotations applied to h_0..h_{p-1}: writes the finished
+// entries 0..p-2 to `out` (global memory, so that the reads of h and of the
+// rotations in LDS need not wait for the writes), returns entry p-1.
+template <typename S>
+__device__ __forceinline__ S rotate_column(int p, const S* h, const S* cl, const S* sl, S* out) {
+  S hi = h[0];
+#pragma unroll 4
+  for (int j = 1; j < p; ++j) {
+    const S hj = h[j], cj = cl[j - 1], sj = sl[j - 1];
+    out[j - 1] = sconj(cj) * hi + sj * hj;
+    hi = -sj * hi + cj * hj;
+  }
+  return hi;
+}
+
+constexpr int kTailNT = 256;  // threads of the kernels that close a step, one workgroup per column
+
+// Sum of part[b * nrhs + c] over b < nblk in a fixed order (all kTailNT
+// threads of a workgroup; red holds one value per wave).
+__device__ __forceinline__ double column_sum(int nblk, int nrhs, int c, const double* __restrict__ part, double* red) {
+  double t = 0.0;
+#pragma unroll 4
+  for (int b = threadIdx.x; b < nblk; b += kTailNT) t += part[(int64_t)b * nrhs + c];
+  t = lane_class_sum(t, 1);
+  if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = t;
+  __syncthreads();
+  t = red[0];
+  for (int k = 1; k < kTailNT / kWave; ++k) t += red[k];
+  return t;
+}
+
 // partial dot products d[j, c] = sum_rows conj(V_j[r, c]) * w[r, c] for j < p
 // (w may be one of the V_j), accumulated in S.  One partial per workgroup.
 template <typename VV, typename VW, typename S, int NT>
@@ -679,152 +784,228 @@ __global__ __launch_bounds__(NT) void k_basis_reg(int64_t n, int nrhs, int p, co
 // instead of three times.  Basis slots 0..p-1 are final, q is tentative.
 // ---------------------------------------------------------------------------
 
-// Dots of the basis chunk V_{j0..j0+cnt-1} with q and with w (w may be null):
-// per workgroup partials part[blk * nout * nrhs + o * nrhs + c] for
-//   o < cnt:             V_{j0+o} . q
-//   cnt <= o < 2 cnt:    V_{j0+o-cnt} . w          (w != null)
-//   o = 2 cnt, 2 cnt+1:  q . q and q . w           (first chunk, w != null)
-//   o = cnt:             q . q                     (first chunk, w == null)
-// nout = 2 cnt + 2 (w != null, first), 2 cnt (w != null), cnt + 1 / cnt
-// (w == null, first / not).  LPE lanes share an element, lane `sub` holds
-// V_{j0 + u LPE + sub}, u < ceil(cnt / LPE) <= PM; every lane walks the
-// elements with a grid stride; reductions over lanes, then over waves in a
-// fixed order (one LDS table of nout * nrhs doubles, the waves add in turn).
-// With nrhs * LPE > 64 a wave covers only part of a row's columns, and each
-// of its lanes adds its own sums (no lane reduction).
-template <typename S, int NT, int PM, int LPE>
-__global__ __launch_bounds__(NT) void k_dcgs2_dots(int64_t n, int nrhs, int j0, int cnt, const S* __restrict__ V,
-                                                   int64_t ldv, const S* __restrict__ q, const S* __restrict__ w,
-                                                   int first, S* __restrict__ part) {
-  extern __shared__ unsigned char dd_raw[];
-  S* dd_sm = reinterpret_cast<S*>(dd_raw);
+// 16 bytes of consecutive values as one load or store; the address need only
+// be aligned for a value
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef f64x2 f64x2_a8 __attribute__((aligned(8)));
+
+__device__ __forceinline__ f64x2 load16(const void* x) { return *reinterpret_cast<const f64x2_a8*>(x); }
+__device__ __forceinline__ f64x2 stream16(const void* x) {  // as ld_stream
+  return __builtin_nontemporal_load(reinterpret_cast<const f64x2_a8*>(x));
+}
+
+// Dots of the basis V_0..V_{p-1} with q and with w (w may be null), in chunks
+// of `chunk` <= kDotsChunk vectors (blockIdx.y): per workgroup partials
+// part[blockIdx.x * nout * nrhs + o * nrhs + c] for
+//   o < p:             V_o . q
+//   p <= o < 2 p:      V_{o-p} . w       (w != null)
+//   o = 2 p, 2 p + 1:  q . q and q . w   (w != null)
+//   o = p:             q . q             (w == null)
+// A stream over the basis, bound by HBM.  The waves of a workgroup walk the
+// same elements (their reads of q and w meet in the cache of the CU) and
+// share out the chunk's vectors: wave k takes j0 + k, j0 + k + NW, ..., at most
+// kDotsPM of them, 16 bytes of each per lane (two real values or a complex
+// one), and keeps their sums, so that the sums are only reduced over a wave's
+// lanes.  ONE: a single real column.
+// Before, a lane (or a pair) took 8 bytes of 16 (32) vectors and the waves
+// summed up in turn: 96^3 x 16 columns, 17 vectors on average, 440 -> 380 us;
+// 128^3, one column 89 -> 66 us; 64^2 rows 10.8 -> 4.6 us; 128^3 x 64 columns
+// 4.45 -> 4.6 ms (6 TB/s, the rate of a large read; two vectors a step more
+// were read before).  Tried: 128 threads (4.69 ms, 375 us), 512 with 4 or 8
+// vectors per wave (5.3 and 4.8 ms, 410 us), 4 KB of a vector per workgroup
+// (4.75 ms, 419 us).
+constexpr int kDotsPM = 8;
+constexpr int kDotsNT = 256;
+constexpr int kDotsChunk = kDotsPM * (kDotsNT / kWave);
+
+template <typename S, bool ONE>
+__global__ __launch_bounds__(kDotsNT) void k_dcgs2_dots(int64_t n, int nrhs, int p, int chunk, const S* __restrict__ V,
+                                                        int64_t ldv, const S* __restrict__ q,
+                                                        const S* __restrict__ w, S* __restrict__ part) {
+  constexpr int E = 16 / (int)sizeof(S), NW = kDotsNT / kWave, PM = kDotsPM;
   const bool hw = w != nullptr;
-  const int nout = (hw ? 2 * cnt : cnt) + (first ? (hw ? 2 : 1) : 0);
-  const int tid = threadIdx.x;
-  const int sub = tid % LPE;
-  const int cth = (tid / LPE) % nrhs;  // the lane's column (the grid stride keeps it)
-  const int pu = (cnt + LPE - 1) / LPE;
-  const S* Vl = V + (int64_t)(j0 + sub) * ldv;
-  S aq[PM], aw[PM];
-  S aa = S(0.0), ab = S(0.0);
+  const int lane = threadIdx.x % kWave;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int j0 = blockIdx.y * chunk + wid;  // the wave's first vector
+  const int j1 = min(p, (int)(blockIdx.y + 1) * chunk);
+  const int pu = j0 < j1 ? (j1 - j0 + NW - 1) / NW : 0;
+  const bool own = blockIdx.y == 0 && wid == NW - 1;  // takes q.q and q.w too
+  if (pu == 0 && !own) return;
+  f64x2 aq[PM], aw[PM], ab[2];
 #pragma unroll
-  for (int u = 0; u < PM; ++u) {
-    aq[u] = S(0.0);
-    aw[u] = S(0.0);
-  }
+  for (int u = 0; u < PM; ++u) aq[u] = aw[u] = f64x2{0.0, 0.0};
+  ab[0] = ab[1] = f64x2{0.0, 0.0};
+  // acc += conj(x) y for the lane's value or values
+  auto add = [](f64x2& acc, f64x2 x, f64x2 y) {
+    if constexpr (E == 2) {
+      acc += x * y;
+    } else {
+      acc.x += x.x * y.x + x.y * y.y;
+      acc.y += x.x * y.y - x.y * y.x;
+    }
+  };
   const int64_t total = n * nrhs;
-  const int64_t stride = (int64_t)gridDim.x * (NT / LPE);
-  for (int64_t g = ((int64_t)blockIdx.x * NT + tid) / LPE; g < total; g += stride) {
-    const S qv = q[g];
-    const S wv = hw ? w[g] : S(0.0);
-    S v[PM];
+  const int64_t stride = (int64_t)gridDim.x * kWave * E;
+  const S* Vw = V + (int64_t)j0 * ldv;
+  int64_t g = ((int64_t)blockIdx.x * kWave + lane) * E;
+  for (; g + E <= total; g += stride) {
+    const f64x2 qv = load16(q + g);
+    const f64x2 wv = hw ? load16(w + g) : f64x2{0.0, 0.0};
+    f64x2 v[PM];
 #pragma unroll
     for (int u = 0; u < PM; ++u)
-      if (u < pu && u * LPE + sub < cnt) v[u] = ld_stream(Vl + (int64_t)(u * LPE) * ldv + g);
-      else v[u] = S(0.0);
-    // dots conjugate the basis (x^H y)
+      if (u < pu) v[u] = stream16(Vw + (int64_t)(u * NW) * ldv + g);
 #pragma unroll
     for (int u = 0; u < PM; ++u)
       if (u < pu) {
-        const S vc = sconj(v[u]);
-        aq[u] += vc * qv;
-        aw[u] += vc * wv;
+        add(aq[u], v[u], qv);
+        add(aw[u], v[u], wv);
       }
-    if (sub == 0) {
-      aa += sconj(qv) * qv;
-      ab += sconj(qv) * wv;
+    if (own) {
+      add(ab[0], qv, qv);
+      add(ab[1], qv, wv);
     }
   }
-  // reduce over the lanes of a column (lanes c LPE + sub keep the sums)
+  if constexpr (ONE) {
+    if (g < total) {  // the last value of an odd length
+      const double qv = q[g], wv = hw ? w[g] : 0.0;
 #pragma unroll
-  for (int u = 0; u < PM; ++u) {
-    if (u < pu) {
-      for (int mm = kWave / 2; mm >= nrhs * LPE; mm >>= 1) {
-        aq[u] += shfl_xor_v(aq[u], mm);
-        aw[u] += shfl_xor_v(aw[u], mm);
-      }
-    }
-  }
-  for (int mm = kWave / 2; mm >= nrhs * LPE; mm >>= 1) {
-    aa += shfl_xor_v(aa, mm);
-    ab += shfl_xor_v(ab, mm);
-  }
-  for (int t = tid; t < nout * nrhs; t += NT) dd_sm[t] = S(0.0);
-  __syncthreads();
-  // the waves add their sums to the table in turn (a fixed order)
-  const int wid = tid / kWave, lane = tid % kWave;
-  for (int k = 0; k < NT / kWave; ++k) {
-    if (wid == k && lane < nrhs * LPE) {
-#pragma unroll
-      for (int u = 0; u < PM; ++u) {
-        const int j = u * LPE + sub;
-        if (u < pu && j < cnt) {
-          dd_sm[j * nrhs + cth] += aq[u];
-          if (hw) dd_sm[(cnt + j) * nrhs + cth] += aw[u];
+      for (int u = 0; u < PM; ++u)
+        if (u < pu) {
+          const double v = Vw[(int64_t)(u * NW) * ldv + g];
+          aq[u].x += v * qv;
+          aw[u].x += v * wv;
         }
-      }
-      if (first && lane % LPE == 0) {
-        const int o = hw ? 2 * cnt : cnt;
-        dd_sm[o * nrhs + cth] += aa;
-        if (hw) dd_sm[(o + 1) * nrhs + cth] += ab;
+      ab[0].x += qv * qv;
+      ab[1].x += qv * wv;
+    }
+  }
+  // the rows of the step's table: V.q, then V.w, then q.q and q.w
+  const int nl = ONE ? 1 : nrhs / E;  // lanes l and l + nl hold the same columns
+  double* out = reinterpret_cast<double*>(part + (int64_t)blockIdx.x * ((hw ? 2 * p : p) + (hw ? 2 : 1)) * nrhs);
+  auto put = [&](int row, f64x2 a) {
+    if (lane >= nl) return;
+    if constexpr (ONE) out[row] = a.x;
+    else *reinterpret_cast<f64x2*>(out + ((int64_t)row * (nrhs / E) + lane) * 2) = a;
+  };
+  auto sum = [&](auto& a) {
+    constexpr int K = sizeof(a) / sizeof(a[0]);
+    double t[ONE ? K : 2 * K];
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+      if constexpr (ONE) {
+        t[u] = a[u].x + a[u].y;
+      } else {
+        t[2 * u] = a[u].x;
+        t[2 * u + 1] = a[u].y;
       }
     }
-    __syncthreads();
+    lane_class_sums(t, nl);
+#pragma unroll
+    for (int u = 0; u < K; ++u) a[u] = ONE ? f64x2{t[u], 0.0} : f64x2{t[ONE ? u : 2 * u], t[ONE ? u : 2 * u + 1]};
+  };
+  sum(aq);
+  if (hw) sum(aw);
+#pragma unroll
+  for (int u = 0; u < PM; ++u)
+    if (u < pu) {
+      put(j0 + u * NW, aq[u]);
+      if (hw) put(p + j0 + u * NW, aw[u]);
+    }
+  if (own) {
+    sum(ab);
+    put(hw ? 2 * p : p, ab[0]);
+    if (hw) put(2 * p + 1, ab[1]);
   }
-  for (int t = tid; t < nout * nrhs; t += NT) part[(int64_t)blockIdx.x * nout * nrhs + t] = dd_sm[t];
 }
 
 // w <- w - sum_{j<p} V_j e_j - e_p q: the projection of w on the final
 // basis v_0..v_p, written in terms of the raw basis slots 0..p (q = slot p,
 // which stays as it is), with per-workgroup partials of |w|^2 in
 // part[blk * nrhs + c].  coef = [e_0..e_{p-1} (p x nrhs) | e_p (nrhs)],
-// copied to LDS.  Element layout as k_basis_reg (LPE lanes per element, lane
-// sub holds V_{u LPE + sub}).
-template <typename S, int NT, int PM, int LPE>
+// copied to LDS.
+// A stream over p + 2 vectors, bound by HBM: a lane takes 16 bytes of every
+// vector (two real values or a complex one), 8 vectors' loads in flight, one
+// running sum, so that any p runs at the same occupancy.  Before, a lane held
+// all p values of an element (two lanes past 32 vectors, 208 VGPRs, 4.5 TB/s):
+// 128^3 x 64 columns, 24 vectors on average, 5.9 -> 5.15 ms (5.5 TB/s with its
+// write); 96^3 x 16, 17 vectors, 390 -> 370 us; 32^3 x 4 complex columns,
+// 24 vectors, 24 -> 15 us.  ONE: a single column (a lane's two values share
+// their coefficients).
+template <typename S, int NT, bool ONE>
 __global__ __launch_bounds__(NT) void k_dcgs2_update(int64_t n, int nrhs, int p, const S* __restrict__ V,
                                                      int64_t ldv, const S* __restrict__ q, S* __restrict__ w,
                                                      const S* __restrict__ coef, double* __restrict__ part) {
-  extern __shared__ unsigned char du_raw[];
+  constexpr int E = 16 / (int)sizeof(S);  // values per lane
+  constexpr int U = 8;                    // vectors in flight
+  extern __shared__ __align__(16) unsigned char du_raw[];
   const int nc = (p + 1) * nrhs;
-  S* cs = reinterpret_cast<S*>(du_raw);
-  double* red = reinterpret_cast<double*>(cs + nc);
+  double* red = reinterpret_cast<double*>(du_raw);
+  S* cs = reinterpret_cast<S*>(red + (NT / kWave) * nrhs + ((NT / kWave) * nrhs) % 2);
   const int tid = threadIdx.x;
   for (int t = tid; t < nc; t += NT) cs[t] = coef[t];
-  // a wave covers 64 / LPE elements: all columns when nrhs * LPE <= 64, else
-  // half of them, and the other half of its row of the table stays zero
-  for (int t = tid; t < (NT / kWave) * nrhs; t += NT) red[t] = 0.0;
   __syncthreads();
-  const S* gc = cs;
-  const S* gam = cs + p * nrhs;
-  const int sub = tid % LPE;
-  const int c = (tid / LPE) % nrhs;
-  const int pu = (p + LPE - 1) / LPE;
-  const S* Vl = V + (int64_t)sub * ldv;
-  double acc = 0.0;
+  const int c = ONE ? 0 : (tid * E) % nrhs;  // the lane's first column (the grid stride keeps it)
+  // sum += v * e of vector j
+  auto add = [&](f64x2& sum, f64x2 v, int j) {
+    if constexpr (E == 1) {
+      const S e = cs[j * nrhs + c];
+      sum.x += v.x * e.re - v.y * e.im;
+      sum.y += v.x * e.im + v.y * e.re;
+    } else if constexpr (ONE) {
+      sum += v * cs[j];
+    } else {
+      sum += v * *reinterpret_cast<const f64x2*>(cs + j * nrhs + c);
+    }
+  };
+  f64x2 acc = {0.0, 0.0};
   const int64_t total = n * nrhs;
-  const int64_t stride = (int64_t)gridDim.x * (NT / LPE);
-  for (int64_t g = ((int64_t)blockIdx.x * NT + tid) / LPE; g < total; g += stride) {
-    S v[PM];
+  const int64_t stride = (int64_t)gridDim.x * NT * E;
+  int64_t g = ((int64_t)blockIdx.x * NT + tid) * E;
+  for (; g + E <= total; g += stride) {
+    f64x2 wv = load16(w + g), sum = {0.0, 0.0}, v[U];
+    const f64x2 qv = load16(q + g);
+    const S* x = V + g;
+    int j = 0;
+    for (; j + U <= p; j += U, x += U * ldv) {
 #pragma unroll
-    for (int u = 0; u < PM; ++u)
-      if (u < pu) v[u] = (u * LPE + sub < p) ? ld_stream(Vl + (int64_t)(u * LPE) * ldv + g) : S(0.0);
-    S gv = S(0.0);
+      for (int u = 0; u < U; ++u) v[u] = stream16(x + u * ldv);
 #pragma unroll
-    for (int u = 0; u < PM; ++u)
-      if (u < pu) {
-        const int j = u * LPE + sub;
-        gv += v[u] * (j < p ? gc[j * nrhs + c] : S(0.0));
-      }
-    if constexpr (LPE == 2) gv += shfl_xor_v(gv, 1);
-    if (sub == 0) {
-      const S un = w[g] - gv - gam[c] * q[g];
+      for (int u = 0; u < U; ++u) add(sum, v[u], j + u);
+    }
+#pragma unroll
+    for (int u = 0; u < U - 1; ++u)
+      if (j + u < p) v[u] = stream16(x + u * ldv);
+#pragma unroll
+    for (int u = 0; u < U - 1; ++u)
+      if (j + u < p) add(sum, v[u], j + u);
+    f64x2 gq = {0.0, 0.0};
+    add(gq, qv, p);
+    wv = wv - sum - gq;
+    *reinterpret_cast<f64x2_a8*>(w + g) = wv;
+    acc += wv * wv;
+  }
+  if constexpr (ONE && E == 2) {
+    if (g < total) {  // the last value of an odd length
+      double sum = 0.0;
+      for (int j = 0; j < p; ++j) sum += V[j * ldv + g] * cs[j];
+      const double un = w[g] - sum - q[g] * cs[p];
       w[g] = un;
-      acc += (double)sabs2(un);
+      acc.x += un * un;
     }
   }
   const int wid = tid / kWave, lane = tid % kWave;
-  for (int mm = kWave / 2; mm >= nrhs * LPE; mm >>= 1) acc += __shfl_xor(acc, mm);
-  if (lane < nrhs * LPE && lane % LPE == 0) red[wid * nrhs + c] = acc;
+  if constexpr (ONE || E == 1) {
+    const double s2 = lane_class_sum(acc.x + acc.y, nrhs);
+    if (lane < nrhs) red[wid * nrhs + lane] = s2;
+  } else {
+    double a[2] = {acc.x, acc.y};
+    lane_class_sums<2>(a, nrhs / 2);
+    if (lane < nrhs / 2) {
+      red[wid * nrhs + 2 * lane] = a[0];
+      red[wid * nrhs + 2 * lane + 1] = a[1];
+    }
+  }
   __syncthreads();
   for (int t = tid; t < nrhs; t += NT) {
     double s2 = 0.0;
@@ -850,51 +1031,122 @@ __global__ __launch_bounds__(NT) void k_dcgs2_update(int64_t n, int nrhs, int p,
 // slot_i e_i with e_i = (R (a - gm s))_i for i < p, e_p = sg gm, gm = c_p / nu:
 // coef = [e_0..e_p] (rows of nrhs) for k_dcgs2_update, zero for columns that
 // are not active.  p = 0: q is the exact v0 (nu = 1, no column to finalize).
-// Dynamic LDS: 2 p values of S.
-template <typename S>
-__global__ __launch_bounds__(64) void k_dcgs2_fix(int nrhs, int m, int p, int maxits, int final_pass,
+// With nblk > 0, d holds nblk partial tables of the dots (part of
+// k_dcgs2_dots), summed here in a fixed order.  flag (final pass, may be
+// null): the column's state for the host (state_bits).
+// Lanes take the basis indices, waves share the sums; only the Givens
+// recurrence runs on one lane, from LDS (it was one lane reading memory all
+// through: 10 -> 6.6 us at 15 vectors, 21 -> 9 at 24, 29 -> 14 at 24 complex
+// ones, and the launch that summed the partials is gone).
+// Dynamic LDS: fix_lds(p, NT) values of S.
+__host__ __device__ inline int fix_lds(int p, int nt) { return (2 * p + 2) * (1 + nt / kWave) + 5 * p + 1; }
+
+template <typename S, int NT>
+__global__ __launch_bounds__(NT) void k_dcgs2_fix(int nrhs, int m, int p, int maxits, int final_pass, int nblk,
                                                   const S* __restrict__ d, S* __restrict__ H, S* __restrict__ cs,
                                                   S* __restrict__ sn, S* __restrict__ rs, KState* __restrict__ st,
                                                   S* __restrict__ coef, const double* __restrict__ vscale,
-                                                  S* __restrict__ R) {
+                                                  S* __restrict__ R, int* __restrict__ flag) {
+  constexpr int NW = NT / kWave;
   extern __shared__ unsigned char fx_raw[];
-  S* sv = reinterpret_cast<S*>(fx_raw);  // s_j
-  S* av = sv + p;                        // a_j (not final)
+  S* dt = reinterpret_cast<S*>(fx_raw);  // the dot table, later [s_j | a_j]
+  S* red = dt + 2 * p + 2;               // NW rows of sums
+  S* cl = red + NW * (2 * p + 2);        // earlier rotations
+  S* sl = cl + p;
+  S* h = sl + p;    // the tentative Hessenberg column, p + 1 values
+  S* sv = h + p + 1;
+  S* av = sv + p;
   __shared__ int go_sh;
   __shared__ double in_sh;
   __shared__ S gm_sh;
   const int c = blockIdx.x;
-  const int lane = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid % kWave, wid = tid / kWave;
   const int64_t ldr = m + 1;
   S* Rc = R + (int64_t)c * ldr * ldr;
+  S* Hc = H + (int64_t)c * (m + 1) * m;
+  S* csc = cs + (int64_t)c * m;
+  S* snc = sn + (int64_t)c * m;
+  const int col = p - 1;
   const double sg = vscale ? vscale[c] : 1.0;
-  const bool was_active = st[c].active != 0;
-  // s and a on the final basis (lanes over j, rows of R read along j)
-  if (was_active) {
+  KState s = st[c];
+  bool go = s.active != 0;  // the same in every thread
+  if (go) {
+    const int no = final_pass ? p + 1 : 2 * p + 2;
+    if (nblk > 0) {
+      for (int o = lane; o < no; o += kWave) {
+        S acc = S(0.0);
+#pragma unroll 8
+        for (int b = wid; b < nblk; b += NW) acc += d[((int64_t)b * no + o) * nrhs + c];
+        red[wid * no + o] = acc;
+      }
+      __syncthreads();
+      for (int o = tid; o < no; o += NT) {
+        S acc = red[o];
+        for (int k = 1; k < NW; ++k) acc += red[k * no + o];
+        dt[o] = acc;
+      }
+    } else {
+      for (int o = tid; o < no; o += NT) dt[o] = d[(int64_t)o * nrhs + c];
+    }
+    for (int j = tid; j + 1 < p; j += NT) {
+      cl[j] = csc[j];
+      sl[j] = snc[j];
+    }
+    if (p > 0)
+      for (int j = tid; j <= p; j += NT) h[j] = Hc[j + col * (m + 1)];
+    __syncthreads();
+    // s and a on the final basis (lanes over j, rows of R read along j, the
+    // rows dealt to the waves)
     for (int j = lane; j < p; j += kWave) {
       S ts = S(0.0), ta = S(0.0);
-      for (int i = 0; i <= j; ++i) {
+#pragma unroll 4
+      for (int i = wid; i <= j; i += NW) {
         const S r = sconj(Rc[i * ldr + j]);
-        ts += r * d[i * nrhs + c];
-        if (!final_pass) ta += r * d[(p + i) * nrhs + c];
+        ts += r * dt[i];
+        if (!final_pass) ta += r * dt[p + i];
+      }
+      red[wid * 2 * p + j] = ts;
+      red[wid * 2 * p + p + j] = ta;
+    }
+    __syncthreads();
+    for (int j = tid; j < p; j += NT) {
+      S ts = red[j], ta = red[p + j];
+      for (int k = 1; k < NW; ++k) {
+        ts += red[k * 2 * p + j];
+        ta += red[k * 2 * p + p + j];
       }
       sv[j] = S(sg) * ts;
-      if (!final_pass) av[j] = ta;
+      av[j] = ta;
+    }
+    __syncthreads();
+  }
+  // d rows: slot_j^H q (j < p), then slot_j^H w (j < p), then q.q, q.w
+  // (final: slot_j^H q, q.q)
+  double qq = 0.0, nu = 1.0, ss = 0.0;
+  S qw = S(0.0), sa = S(0.0);
+  if (go) {
+    qq = sg * sg * (double)sreal(final_pass ? dt[p] : dt[2 * p]);
+    if (!final_pass) qw = S(sg) * dt[2 * p + 1];
+    for (int j = lane; j < p; j += kWave) {
+      ss += (double)sabs2(sv[j]);
+      if (!final_pass) sa += sconj(sv[j]) * av[j];
+    }
+    ss = lane_class_sum(ss, 1);
+    sa = lane_class_sum(sa, 1);
+    nu = p > 0 ? sqrt(fmax(qq - ss, 0.0)) : 1.0;
+    if (p > 0) {
+      const S hq = h[p];
+      __syncthreads();
+      for (int j = tid; j < p; j += NT) h[j] += hq * sv[j];
+      if (tid == 0) h[p] = hq * S(nu);
+      __syncthreads();
     }
   }
-  __syncthreads();
-  if (lane == 0) {
+  if (tid == 0) {
     // the column's scalar part; returns whether w gets coefficients
     auto scalar_part = [&]() -> bool {
-      KState s = st[c];
-      if (!s.active) return false;
+      if (!go) return false;
       const double eps = 2.220446049250313e-16;
-      // d rows: slot_j^H q (j < p), then slot_j^H w (j < p), then q.q, q.w
-      // (final: slot_j^H q, q.q)
-      const double qq = sg * sg * (double)sreal(final_pass ? d[p * nrhs + c] : d[2 * p * nrhs + c]);
-      const S qw = final_pass ? S(0.0) : S(sg) * d[(2 * p + 1) * nrhs + c];
-      double nu = 1.0;
-      S* Hc = H + (int64_t)c * (m + 1) * m;
       auto retire = [&](int status) {
         s.status = status;
         s.active = 0;
@@ -912,34 +1164,20 @@ __global__ __launch_bounds__(64) void k_dcgs2_fix(int nrhs, int m, int p, int ma
       // nu * h is negligible there, a lucky breakdown) and restarts from its
       // true residual instead of continuing on a basis vector that is not
       // orthogonal
-      bool dependent = false;
       if (p > 0) {
-        double ss = 0.0;
-        for (int j = 0; j < p; ++j) ss += (double)sabs2(sv[j]);
         if (!isfinite(ss)) {
           retire(5);
           return false;
         }
-        dependent = !(qq - ss > kDcgs2DependentTol * qq);
-        nu = sqrt(fmax(qq - ss, 0.0));
-        const int col = p - 1;
-        const S hq = Hc[p + col * (m + 1)];
-        for (int j = 0; j < p; ++j) Hc[j + col * (m + 1)] += hq * sv[j];
-        Hc[p + col * (m + 1)] = hq * S(nu);
+        const bool dependent = !(qq - ss > kDcgs2DependentTol * qq);
         // Givens update of column col, as k_givens (fgmres.hpp:428-461)
-        S* csc = cs + (int64_t)c * m;
-        S* snc = sn + (int64_t)c * m;
         S* rsc = rs + (int64_t)c * (m + 1);
+        S* hc = Hc + (int64_t)col * (m + 1);
         s.iters += 1;
         s.icur = p;
-        for (int j = 1; j < p; ++j) {
-          const S hii = Hc[(j - 1) + col * (m + 1)];
-          const S hj = Hc[j + col * (m + 1)];
-          Hc[(j - 1) + col * (m + 1)] = sconj(csc[j - 1]) * hii + snc[j - 1] * hj;
-          Hc[j + col * (m + 1)] = -snc[j - 1] * hii + csc[j - 1] * hj;
-        }
-        const S hii = Hc[(p - 1) + col * (m + 1)];
-        const S hii1 = Hc[p + col * (m + 1)];
+        const S hii = rotate_column(p, h, cl, sl, hc);
+        const S hii1 = h[p];
+        hc[p] = hii1;
         const double g = sqrt((double)sabs2(hii) + (double)sabs2(hii1));
         if (!isfinite(g)) {
           retire(5);
@@ -949,12 +1187,14 @@ __global__ __launch_bounds__(64) void k_dcgs2_fix(int nrhs, int m, int p, int ma
           retire(2);
           return false;
         }
-        csc[p - 1] = hii / S(g);
-        snc[p - 1] = hii1 / S(g);
-        rsc[p] = -snc[p - 1] * rsc[p - 1];
-        rsc[p - 1] = sconj(csc[p - 1]) * rsc[p - 1];
-        Hc[(p - 1) + col * (m + 1)] = sconj(csc[p - 1]) * hii + snc[p - 1] * hii1;
-        s.normr = sabs_d(rsc[p]);
+        const S cn = hii / S(g), sn1 = hii1 / S(g);
+        const S r0 = rsc[p - 1];
+        csc[p - 1] = cn;
+        snc[p - 1] = sn1;
+        rsc[p] = -sn1 * r0;
+        rsc[p - 1] = sconj(cn) * r0;
+        hc[p - 1] = sconj(cn) * hii + sn1 * hii1;
+        s.normr = sabs_d(-sn1 * r0);
         if (s.normr <= s.tolr) {
           s.status = 1;
           s.active = 0;
@@ -967,86 +1207,77 @@ __global__ __launch_bounds__(64) void k_dcgs2_fix(int nrhs, int m, int p, int ma
       if (final_pass) return false;
       const double in = nu > 0.0 ? 1.0 / nu : 0.0;
       // coefficient of w on the final v_p: (q - V s)^H w / nu = (q.w - s^H a) / nu
-      S sa = S(0.0);
-      for (int j = 0; j < p; ++j) sa += sconj(sv[j]) * av[j];
       const S cp = (qw - sa) * S(in);
-      for (int j = 0; j < p; ++j) Hc[j + p * (m + 1)] = av[j];
-      Hc[p + p * (m + 1)] = cp;
+      Hc[p + (int64_t)p * (m + 1)] = cp;
       in_sh = in;
       gm_sh = cp * S(in);
       return true;
     };
     go_sh = scalar_part() ? 1 : 0;
+    if (flag) flag[c] = state_bits(s, maxits);
   }
-  __syncthreads();
   if (final_pass) return;
+  __syncthreads();
   if (!go_sh) {
-    for (int j = lane; j <= p; j += kWave) coef[(int64_t)j * nrhs + c] = S(0.0);
+    for (int j = tid; j <= p; j += NT) coef[(int64_t)j * nrhs + c] = S(0.0);
     return;
   }
   const double in = in_sh;
   const S gm = gm_sh;
-  // R's column p and the update's coefficients (lanes over rows of R)
-  for (int i = lane; i < p; i += kWave) {
+  for (int j = tid; j < p; j += NT) Hc[j + (int64_t)p * (m + 1)] = av[j];
+  // R's column p and the update's coefficients (16 lanes to a row of R)
+  for (int i0 = 0; i0 < p; i0 += NT / 16) {
+    const int i = i0 + tid / 16;
     S rsv = S(0.0), rg = S(0.0);
-    for (int j = i; j < p; ++j) {
-      const S r = Rc[i * ldr + j];
-      rsv += r * sv[j];
-      rg += r * (av[j] - gm * sv[j]);
+    if (i < p) {
+#pragma unroll 4
+      for (int j = i + tid % 16; j < p; j += 16) {
+        const S r = Rc[i * ldr + j];
+        rsv += r * sv[j];
+        rg += r * (av[j] - gm * sv[j]);
+      }
     }
-    Rc[i * ldr + p] = -rsv * S(in);
-    coef[(int64_t)i * nrhs + c] = rg;
+    rsv = lane_step<1>(lane_step<2>(lane_step<4>(lane_step<8>(rsv))));
+    rg = lane_step<1>(lane_step<2>(lane_step<4>(lane_step<8>(rg))));
+    if (i < p && tid % 16 == 0) {
+      Rc[i * ldr + p] = -rsv * S(in);
+      coef[(int64_t)i * nrhs + c] = rg;
+    }
   }
-  if (lane == 0) {
+  if (tid == 0) {
     Rc[p * ldr + p] = S(sg * in);
     coef[(int64_t)p * nrhs + c] = S(sg) * gm;
   }
 }
 
-// Sums the nblk partials of one k_dcgs2_dots launch into the rows of the
-// step's dot table d (rows: s_j, then a_j, then q.q and q.w; or s_j, q.q
-// without w), one wave per output, in a fixed order.
+// After k_dcgs2_update of step p, per column (blockIdx.x): ||w|| from the
+// nblk partials of ||w||^2, the tentative H[p+1, p] = ||w|| and the scale that
+// normalizes w (zero for columns that are not active); the column's state for
+// the host in flag.
 template <typename S>
-__global__ __launch_bounds__(256) void k_dcgs2_final(int nblk, int nout, int cnt, int nrhs, int hw, int p, int j0,
-                                                     const S* __restrict__ part, S* __restrict__ d) {
-  const int g = blockIdx.x * 4 + threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
-  const int total = nout * nrhs;
-  if (g >= total) return;  // whole wave exits together
-  S s = S(0.0);
-  for (int b = lane; b < nblk; b += kWave) s += part[(int64_t)b * total + g];
-#pragma unroll
-  for (int mm = kWave / 2; mm > 0; mm >>= 1) s += shfl_xor_v(s, mm);
-  if (lane != 0) return;
-  const int o = g / nrhs, c = g % nrhs;
-  int row;
-  if (o < cnt) row = j0 + o;
-  else if (hw && o < 2 * cnt) row = p + j0 + (o - cnt);
-  else row = (hw ? 2 * p : p) + (o - (hw ? 2 * cnt : cnt));
-  d[row * nrhs + c] = s;
-}
-
-// After k_dcgs2_update of step p: the tentative H[p+1, p] = ||w|| and the
-// scale that normalizes w (zero for columns that are not active).
-template <typename S>
-__global__ void k_dcgs2_norm(int nrhs, int m, int p, const double* __restrict__ t2, S* __restrict__ H,
-                             KState* __restrict__ st, double* __restrict__ vscale) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nrhs) return;
+__global__ __launch_bounds__(kTailNT) void k_dcgs2_norm(int nblk, int nrhs, int m, int p, int maxits,
+                                                        const double* __restrict__ part, S* __restrict__ H,
+                                                        KState* __restrict__ st, double* __restrict__ vscale,
+                                                        int* __restrict__ flag) {
+  __shared__ double red[kTailNT / kWave];
+  const int c = blockIdx.x;
+  const double t2 = column_sum(nblk, nrhs, c, part, red);
+  if (threadIdx.x != 0) return;
   KState s = st[c];
   if (!s.active) {
     s.scale = 0.0;
-  } else if (!isfinite(t2[c])) {
+  } else if (!isfinite(t2)) {
     s.status = 5;
     s.active = 0;
     s.scale = 0.0;
   } else {
-    const double t = sqrt(t2[c]);
+    const double t = sqrt(t2);
     H[(int64_t)c * (m + 1) * m + (p + 1) + p * (m + 1)] = S(t);
     s.scale = t > 0.0 ? 1.0 / t : 0.0;
   }
   st[c] = s;
-  if (vscale) vscale[c] = s.scale;  // w stays as it is; its readers apply the scale
+  vscale[c] = s.scale;  // w stays as it is; its readers apply the scale
+  if (flag) flag[c] = state_bits(s, maxits);
 }
 
 // v[r, c] *= s[c]   (s from KState.scale)
@@ -1059,7 +1290,8 @@ __global__ void k_scale_cols(int64_t n, int nrhs, const KState* __restrict__ st,
 
 // FGMRES start (fgmres.hpp:318-359): normb, normr from squared norms.
 __global__ void k_fgmres_init(int nrhs, const double* __restrict__ nb2, const double* __restrict__ nr2, double tol,
-                              int absolute, KState* __restrict__ st, double* __restrict__ x_zero_flag) {
+                              int absolute, int maxits, KState* __restrict__ st,
+                              double* __restrict__ x_zero_flag, int* __restrict__ flag) {
   int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= nrhs) return;
   const double eps = 2.220446049250313e-16;
@@ -1084,6 +1316,7 @@ __global__ void k_fgmres_init(int nrhs, const double* __restrict__ nb2, const do
     s.active = 1;
   }
   st[c] = s;
+  if (flag) flag[c] = state_bits(s, maxits);
 }
 
 // x[r, c] = 0 where flag[c] != 0
@@ -1117,89 +1350,111 @@ __global__ void k_cycle_start(int nrhs, int m, KState* __restrict__ st, S* __res
 // Hessenberg column + Givens update for inner step i (1-based), fgmres.hpp:424-461
 // (complex: c = h_ii / gamma and s = h_i+1,i / gamma, rotations applied with
 // conj(c) as the reference does).  hcol[j*nrhs + c], j <= i-1 : orthogonalization
-// coefficients; t2[c] = ||w||^2.
+// coefficients (plus those of hadd, a second projection pass, when not null);
+// ||w||^2 from nblk partials.  One workgroup per column: the column and the
+// earlier rotations go through LDS, one lane runs the recurrence; the
+// column's state for the host in flag (may be null).
+// Dynamic LDS: 3 i values of S.
 template <typename S>
-__global__ void k_givens(int nrhs, int m, int i, int maxits, const S* __restrict__ hcol,
-                         const double* __restrict__ t2, S* __restrict__ H, S* __restrict__ cs,
-                         S* __restrict__ sn, S* __restrict__ rs, KState* __restrict__ st) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nrhs) return;
+__global__ __launch_bounds__(kTailNT) void k_givens(int nblk, int nrhs, int m, int i, int maxits,
+                                                    const S* __restrict__ hcol, const S* __restrict__ hadd,
+                                                    const double* __restrict__ part, S* __restrict__ H,
+                                                    S* __restrict__ cs, S* __restrict__ sn, S* __restrict__ rs,
+                                                    KState* __restrict__ st, int* __restrict__ flag) {
+  extern __shared__ unsigned char gv_raw[];
+  S* h = reinterpret_cast<S*>(gv_raw);
+  S* cl = h + i;
+  S* sl = cl + i;
+  __shared__ double red[kTailNT / kWave];
+  const int c = blockIdx.x;
+  S* csc = cs + (int64_t)c * m;
+  S* snc = sn + (int64_t)c * m;
+  for (int j = threadIdx.x; j < i; j += kTailNT) {
+    h[j] = hadd ? hcol[j * nrhs + c] + hadd[j * nrhs + c] : hcol[j * nrhs + c];
+    if (j + 1 < i) {
+      cl[j] = csc[j];
+      sl[j] = snc[j];
+    }
+  }
+  const double t = sqrt(column_sum(nblk, nrhs, c, part, red));  // its barrier also covers h, cl, sl
+  if (threadIdx.x != 0) return;
   KState s = st[c];
-  if (!s.active) {
-    s.scale = 0.0;
+  auto settle = [&](int status, int active, double scale) {
+    s.status = status;
+    s.active = active;
+    s.scale = scale;
     st[c] = s;
+    if (flag) flag[c] = state_bits(s, maxits);
+  };
+  if (!s.active) {
+    settle(s.status, 0, 0.0);
     return;
   }
   const double eps = 2.220446049250313e-16;
-  S* Hc = H + (int64_t)c * (m + 1) * m;
-  S* csc = cs + (int64_t)c * m;
-  S* snc = sn + (int64_t)c * m;
   S* rsc = rs + (int64_t)c * (m + 1);
-  const int col = i - 1;
-  for (int j = 0; j < i; ++j) Hc[j + col * (m + 1)] = hcol[j * nrhs + c];
-  const double t = sqrt(t2[c]);
-  Hc[i + col * (m + 1)] = S(t);
+  S* hc = H + (int64_t)c * (m + 1) * m + (int64_t)(i - 1) * (m + 1);
   s.iters += 1;
   s.icur = i;
-  for (int j = 1; j < i; ++j) {
-    const S hii = Hc[(j - 1) + col * (m + 1)];
-    const S hj = Hc[j + col * (m + 1)];
-    Hc[(j - 1) + col * (m + 1)] = sconj(csc[j - 1]) * hii + snc[j - 1] * hj;
-    Hc[j + col * (m + 1)] = -snc[j - 1] * hii + csc[j - 1] * hj;
-  }
-  const S hii = Hc[(i - 1) + col * (m + 1)];
-  const S hii1 = Hc[i + col * (m + 1)];
+  const S hii = rotate_column(i, h, cl, sl, hc);
+  const S hii1 = S(t);
+  hc[i] = hii1;
   const double gam = sqrt((double)sabs2(hii) + (double)sabs2(hii1));
   if (!isfinite(gam) || !isfinite(t)) {  // NaN or Inf from the apply or the matrix product
-    s.status = 5;
-    s.active = 0;
-    s.scale = 0.0;
-    st[c] = s;
+    settle(5, 0, 0.0);
     return;
   }
   if (fabs(gam) < eps) {  // breakdown: the reference leaves x untouched (fgmres.hpp:440-443)
-    s.status = 2;
-    s.active = 0;
-    s.scale = 0.0;
-    st[c] = s;
+    settle(2, 0, 0.0);
     return;
   }
-  csc[i - 1] = hii / S(gam);
-  snc[i - 1] = hii1 / S(gam);
-  rsc[i] = -snc[i - 1] * rsc[i - 1];
-  rsc[i - 1] = sconj(csc[i - 1]) * rsc[i - 1];
-  Hc[(i - 1) + col * (m + 1)] = sconj(csc[i - 1]) * hii + snc[i - 1] * hii1;
-  s.normr = sabs_d(rsc[i]);
-  s.scale = (t > 0.0) ? 1.0 / t : 0.0;
-  if (s.normr <= s.tolr) {
-    s.status = 1;
-    s.active = 0;
-  } else if (i >= m || s.iters >= maxits) {
-    s.active = 0;  // cycle ends for this column
-  }
-  st[c] = s;
+  const S cn = hii / S(gam), sn1 = hii1 / S(gam);
+  const S r0 = rsc[i - 1];
+  csc[i - 1] = cn;
+  snc[i - 1] = sn1;
+  rsc[i] = -sn1 * r0;
+  rsc[i - 1] = sconj(cn) * r0;
+  hc[i - 1] = sconj(cn) * hii + sn1 * hii1;
+  s.normr = sabs_d(-sn1 * r0);
+  const double scale = (t > 0.0) ? 1.0 / t : 0.0;
+  if (s.normr <= s.tolr) settle(1, 0, scale);
+  else settle(s.status, i >= m || s.iters >= maxits ? 0 : s.active, scale);  // the cycle may end for this column
 }
 
 // Back substitution on the triangularized H (fgmres.hpp:471-480); coef[j*nrhs+c].
+// One wave per column; lane j of round r holds y_{64 r + j}, and each solved
+// value is taken out of the rest by the column of H that it multiplies (one
+// lane reading H along its rows took 62 us for 30 vectors and 268 for 50
+// complex ones, now 9 and 30).  m < 128.
 template <typename S>
-__global__ void k_backsolve(int nrhs, int m, const S* __restrict__ H, S* __restrict__ rs,
-                            const KState* __restrict__ st, S* __restrict__ coef, int* __restrict__ upd) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nrhs) return;
-  KState s = st[c];
-  for (int j = 0; j < m; ++j) coef[j * nrhs + c] = S(0.0);
-  upd[c] = 0;
-  if (s.status == 2 || s.status == 4 || s.status == 5 || s.icur == 0) return;
+__global__ __launch_bounds__(kWave) void k_backsolve(int nrhs, int m, const S* __restrict__ H,
+                                                     const S* __restrict__ rs, const KState* __restrict__ st,
+                                                     S* __restrict__ coef, int* __restrict__ upd) {
+  const int c = blockIdx.x;
+  const int lane = threadIdx.x;
+  const KState s = st[c];
+  const bool use = !(s.status == 2 || s.status == 4 || s.status == 5 || s.icur == 0);
+  const int i = use ? s.icur : 0;
+  if (lane == 0) upd[c] = use ? 1 : 0;
   const S* Hc = H + (int64_t)c * (m + 1) * m;
-  S* rsc = rs + (int64_t)c * (m + 1);
-  const int i = s.icur;
-  rsc[i - 1] /= Hc[(i - 1) + (i - 1) * (m + 1)];
-  for (int k = i - 2; k >= 0; --k) {
-    for (int j = k + 1; j < i; ++j) rsc[k] -= Hc[k + j * (m + 1)] * rsc[j];
-    rsc[k] /= Hc[k + k * (m + 1)];
+  const S* rsc = rs + (int64_t)c * (m + 1);
+  S y[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) y[r] = r * kWave + lane < i ? rsc[r * kWave + lane] : S(0.0);
+#pragma unroll
+  for (int r = 1; r >= 0; --r) {
+#pragma unroll 4
+    for (int k = min(i, (r + 1) * kWave) - 1; k >= r * kWave; --k) {
+      const S* hk = Hc + (int64_t)k * (m + 1);
+      const S yk = lane_value(y[r], k % kWave) / hk[k];
+      const int row = r * kWave + lane;
+      if (row == k) y[r] = yk;
+      else if (row < k) y[r] -= hk[row] * yk;
+      if (r == 1) y[0] -= hk[lane] * yk;
+    }
   }
-  for (int j = 0; j < i; ++j) coef[j * nrhs + c] = rsc[j];
-  upd[c] = 1;
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+    if (r * kWave + lane < m) coef[(r * kWave + lane) * nrhs + c] = y[r];
 }
 
 // x[r, c] += sum_j coef[j, c] * Z_j[r, c] for columns with upd[c], summed
@@ -1226,22 +1481,6 @@ template <typename V>
 __global__ void k_fill_zero(int64_t m, V* __restrict__ x) {
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < m) x[t] = V(0.0);
-}
-
-// Restart bookkeeping: any column still running?  flag[0] = number of running columns.
-__global__ void k_count_running(int nrhs, const KState* __restrict__ st, int maxits, int* __restrict__ flag) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  int cnt = 0;
-  for (int c = 0; c < nrhs; ++c)
-    if (st[c].status == 0 && st[c].iters < maxits) ++cnt;
-  flag[0] = cnt;
-}
-
-__global__ void k_count_active(int nrhs, const KState* __restrict__ st, int* __restrict__ flag) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  int cnt = 0;
-  for (int c = 0; c < nrhs; ++c) cnt += st[c].active ? 1 : 0;
-  flag[0] = cnt;
 }
 
 // copy v (double) into z (VZ) : identity preconditioner
