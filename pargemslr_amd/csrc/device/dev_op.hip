@@ -510,12 +510,14 @@ void launch_trsv_pipe(int nt, int lpr, const DevTrsv& T, const V* rhs, V* x, int
 constexpr int kRingWidth = 20;
 
 // Steps whose records are in LDS or on the way there: enough that a copy has
-// K - 2 steps to arrive (1 to 2 us), within the 63 copies that can be waited for
+// K - 3 steps to arrive (1 to 2 us), within the 63 copies that can be waited for
 // apart.  8 to 14 stages of 4-byte values and 6 to 10 of 8-byte ones measured
-// within 3 % of each other.
-template <typename V>
+// within 3 % of each other, except for a single column in half steps, the
+// shortest ones (8 -> 12 stages of 8-byte values: 1023x1021 513 -> 485 us, 96^3
+// 323 -> 305).
+template <typename V, bool SHORT>
 constexpr int ring_depth() {
-  return sizeof(V) == 4 ? 10 : sizeof(V) == 8 ? 8 : 6;
+  return SHORT ? (sizeof(V) == 4 ? 16 : sizeof(V) == 8 ? 12 : 10) : sizeof(V) == 4 ? 10 : sizeof(V) == 8 ? 8 : 6;
 }
 
 template <typename V, int K, int CG, int NG, int NH>
@@ -526,7 +528,7 @@ void launch_trsv_ring_k(const DevTrsv& T, const V* rhs, V* x, int nrhs, hipStrea
   const DevMem& step = NH == 1 ? T.step_h : T.step;
   const DevMem& stepU = NH == 1 ? T.stepU_h : T.stepU;
   const DevMem& pos = NH == 1 ? T.pos_h : T.pos;
-  kern<<<grid, 64 * (NH * NG + 2), lds, s>>>(T.nblocks, T.window, T.row0.as<int>(), step.as<int>(), stepU.as<int>(),
+  kern<<<grid, 64 * (NH * NG + NH + 1), lds, s>>>(T.nblocks, T.window, T.row0.as<int>(), step.as<int>(), stepU.as<int>(),
                                              T.ri0.as<int64_t>(), pos.as<int>(), T.rec.as<unsigned char>(),
                                              T.info.as<int2>(), T.dinv.as<V>(), rhs, x, nrhs);
 }
@@ -543,7 +545,6 @@ void launch_trsv_ring(pgs_dev_op_s* op, const DevTrsv& T, const V* rhs, V* x, in
     throw std::runtime_error("diagonal block too large for 32-bit offsets");
   if (nrhs <= 0 || (nrhs & (nrhs - 1)) != 0)
     throw std::runtime_error("the ring solve takes a power-of-two number of columns");
-  constexpr int KB = ring_depth<V>();
   constexpr int CMAX = sizeof(V) == 4 ? 16 : sizeof(V) == 8 ? 8 : 4;
   // A workgroup takes as many columns as its rings and registers hold, since its
   // columns share the records; but below one workgroup per CU the step chain is
@@ -558,6 +559,7 @@ void launch_trsv_ring(pgs_dev_op_s* op, const DevTrsv& T, const V* rhs, V* x, in
   auto go = [&](auto cg, auto ng, auto nh) {
     constexpr int CG = decltype(cg)::value, NG = decltype(ng)::value, NH = decltype(nh)::value;
     using L = RingLds<V, CG, NG, NH>;
+    constexpr int KB = ring_depth<V, CG * NG * NH == 1>();
     const int64_t grid = (int64_t)T.nblocks * (nrhs / (CG * NG));
     auto rounds = [&](int K) {
       const int64_t at_once = (int64_t)op->num_cus * (op->lds_max / L::bytes(T.window, K));
@@ -575,9 +577,9 @@ void launch_trsv_ring(pgs_dev_op_s* op, const DevTrsv& T, const V* rhs, V* x, in
   // Half steps have no idle wave where a level set rarely holds more than 16 rows:
   // the solving waves are then all column groups.  Whole steps shorten the chain
   // where it often does.  Measured, us per launch, half / whole steps: 64^3
-  // (62,914 against 60,888 steps) 8 FP64 columns 206 / 263, 64 FP32 306 / 424;
-  // 96^3 convection-diffusion (153,495 against 110,111) 8 FP64 columns 541 / 634;
-  // 128^3 (319,055 against 202,577) 8 FP32 columns 802 / 613, 8 FP64 940 / 806.
+  // (62,914 against 60,888 steps) 8 FP64 columns 175 / 263, 64 FP32 249 / 424;
+  // 96^3 convection-diffusion (153,495 against 110,111) 8 FP64 columns 476 / 630;
+  // 128^3 (319,055 against 202,577) 8 FP32 columns 740 / 599, 8 FP64 888 / 803.
   const bool half = op->ring_nt == 64 || (op->ring_nt == 0 && 2 * T.max_block_steps_h < 3 * T.max_block_steps);
   if constexpr (CMAX >= 16) {
     if (c == 16 && (half ? go(I4(), I4(), I1()) : go(I8(), I2(), I2()))) return;
@@ -639,7 +641,7 @@ template <typename V>
 void set_trsv_attrs(int lds_max) {
   auto both = [&](auto cg, auto ng, auto nh) {  // both numbers of stages
     constexpr int CG = decltype(cg)::value, NG = decltype(ng)::value, NH = decltype(nh)::value;
-    set_ring_attrs(k_trsv_ring<V, ring_depth<V>(), CG, NG, NH>, lds_max);
+    set_ring_attrs(k_trsv_ring<V, ring_depth<V, CG * NG * NH == 1>(), CG, NG, NH>, lds_max);
     set_ring_attrs(k_trsv_ring<V, 4, CG, NG, NH>, lds_max);
   };
   using I1 = std::integral_constant<int, 1>;

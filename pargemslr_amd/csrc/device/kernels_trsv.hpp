@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace pgs {
 namespace dev {
@@ -356,16 +357,17 @@ __global__ __launch_bounds__(NT) void k_trsv_pipe(int nblocks, const int* __rest
 // each, since a SIMD issues one instruction of a wave at a time.  So the work is
 // split over waves, one per SIMD for one column: NH * NG solving waves (NH = 2:
 // the rows 0-15 and 16-31 of a step, NH = 1: half steps of at most 16 rows; NG
-// groups of CG columns) do nothing but the chain, one wave copies the factor
-// records to LDS and one the row data, both K steps ahead and straight from
+// groups of CG columns) do nothing but the chain, NH waves copy the factor
+// records to LDS and one the right-hand sides, K steps ahead and straight from
 // memory to LDS.  Four lanes solve a row with five entries each; lane q of a row
 // finalizes columns q, q + 4, ...  When every wave did everything (5 entry loads, a
 // row pair, a descriptor and a right-hand side per step: about 51 instructions
 // for one FP32 column, 69 for FP64, against 35 and 42 in a solving wave now),
 // level 0 took, us per launch at 128^3, FP32 / FP64, before -> now: 1 column 652 /
-// 970 -> 517 / 664; 8 columns 740 / 1013 -> 611 / 807; 64 columns 1586 / 3699 ->
-// 1452 / 2869; 64^3, 1 column: 219 / 255 -> 145 / 172; 1023 x 1021, 8 columns: 790 /
-// 1020 -> 592 / 685.
+// 970 -> 495 / 664; 8 columns 740 / 1013 -> 599 / 803; 64 columns 1586 / 3699 ->
+// 1452 / 2887; 64^3, 1 column: 219 / 255 -> 129 / 146; 1023 x 1021, 8 columns: 790 /
+// 1020 -> 506 / 596.  With the loading waves idle the solving waves alone take
+// 415 / 482 (128^3, 1 column) and 112 / 128 (64^3): LDS serves both.
 template <typename V, int CG>
 struct alignas(CG * sizeof(V) < 16 ? CG * sizeof(V) : 16) RingRow {
   V v[CG];
@@ -525,16 +527,39 @@ struct RingLds {
   __host__ __device__ static int bytes(int rows, int K) { return NG * ring(rows) + K * stage; }
 };
 
-// Sweep of the wave that moves the records.  Between the barriers of steps s - 1
-// and s it starts the copy of the records of step s + K into the stage that the
-// solving waves have just taken step s from, and waits until the records of step
-// s + 2 have arrived.
-template <typename V, int K, int CG, int NG, int NH>
-__device__ __forceinline__ void ring_copy_sweep(int nsteps, const int* pos, int rows, __amdgpu_buffer_rsrc_t rs_ent) {
+// Hand-over of the stages.  A stage's reads are issued a step ahead (take).  With
+// two waves per group of columns (NH = 2) a step ends with all LDS work done,
+// since the waves read each other's ring rows; the stage taken in a step is free
+// at its end.  With one wave per group (NH = 1) no other wave reads its ring: LDS
+// serves a wave's accesses in order, so a step ends at once, without waiting for
+// its ring write or for the reads of the next step's stage.  That stage is free
+// a step later, when its values have been used: the loading waves run one step
+// later ("late": K - 1 steps ahead, K - 3 in flight), and the solving waves need
+// K > 4 stages (with 4 only one copy would be in flight: 96^3, 64 columns, 830 ->
+// 1040 us).  One column, FP64: 64^3 171 -> 150 us, 1023x1021 570 -> 520.
+template <int NH, int K>
+constexpr bool ring_late() { return NH == 1 && K > 4; }
+
+// Sweep of a wave that moves records: those of the group of rows HC of each step
+// (the first or the second 16).  Between the barriers of steps s - 1 and s it
+// starts the copy of the records of step s + K (late: s + K - 1) into a stage that
+// the solving waves have done with, and waits until those of step s + 2 have
+// arrived.  The first of these waves also moves the ring slots and row ids, the
+// last the pivots: issuing the copies is what the loading waves spend their time
+// on, and the slowest of them sets the step (one wave for both groups, with all
+// row data on its neighbour: level 0 at 128^3, 1 column, 664 us in FP64 where the
+// solving waves alone take 482).
+template <typename V, int K, int CG, int NG, int NH, int HC, bool UPPER>
+__device__ __forceinline__ void ring_copy_sweep(int nsteps, const int* pos, int rows, int dummy,
+                                                __amdgpu_buffer_rsrc_t rs_ent, __amdgpu_buffer_rsrc_t rs_info,
+                                                __amdgpu_buffer_rsrc_t rs_dinv) {
   constexpr int RB = ring_row_bytes<V>(), PB = ring_stage_bytes<V>(), NP = ring_pieces<V>();
   using L = RingLds<V, CG, NG, NH>;
   static_assert(2 * K + 2 <= 64, "step boundaries of a pass and its look-ahead in one register");
-  constexpr int kWait = K > 2 ? (K - 2) * NH * NP : 0;  // the copies of the K - 2 steps after s + 2
+  constexpr int late = ring_late<NH, K>() ? 1 : 0;
+  // the copies of the K - 2 steps after s + 2 (late: K - 3)
+  constexpr bool kInfo = HC == 0, kPiv = UPPER && HC == NH - 1;
+  constexpr int kWait = K > 2 ? (K - 2 - late) * (NP + (kInfo ? 1 : 0) + (kPiv ? 1 : 0)) : 0;
   static_assert(kWait <= 60, "outstanding copies");
   const int lane = threadIdx.x & 63;
   const unsigned stage0 = (unsigned)(NG * L::ring(rows));
@@ -559,22 +584,36 @@ __device__ __forceinline__ void ring_copy_sweep(int nsteps, const int* pos, int 
     const int p0 = __builtin_amdgcn_readlane(pv, i), n = __builtin_amdgcn_readlane(pv, i + 1) - p0;
     const int n0 = min(n, kRingGroup);
     const unsigned a = stage0 + stage * L::stage;
-    copy_group(a, p0, n0);
-    if constexpr (NH == 2) copy_group(a + PB, p0 + n0, n - n0);
+    if constexpr (HC == 0) copy_group(a, p0, n0);
+    else copy_group(a + PB, p0 + n0, n - n0);
+    // lanes past the step's rows copy the dummy row's pair and no pivot
+    using LP = __attribute__((address_space(3))) void*;
+    if constexpr (kInfo)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_info, (LP)(size_t)(a + L::rec), 4,
+                                               lane < 2 * n ? lane * 4 : dummy - p0 * 8 + (lane & 1) * 4, p0 * 8, 0, 0);
+    if constexpr (kPiv) {
+      if constexpr (sizeof(V) == 16)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_dinv, (LP)(size_t)(a + L::rec + L::info), 16,
+                                                 lane < n ? l16 : kRingOut, p0 * 16, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_dinv, (LP)(size_t)(a + L::rec + L::info), 4,
+                                                 lane < n * ((int)sizeof(V) / 4) ? lane * 4 : kRingOut,
+                                                 p0 * (int)sizeof(V), 0, 0);
+    }
   };
 #pragma unroll
-  for (int k = 0; k < K; ++k) copy_step(k, k);
+  for (int k = 0; k < K - late; ++k) copy_step(k, k);
   __builtin_amdgcn_sched_barrier(0);
   __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   // the solving waves take step 0 here, before its stage is used again
-  __builtin_amdgcn_s_barrier();
+  if constexpr (!late) __builtin_amdgcn_s_barrier();
   __asm__ __volatile__("" ::: "memory");
   for (int base = 0; base < nsteps; base += K) {
     const int pvn = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_pos, min(base + K + lane, nsteps) * 4, 0, 0);
 #pragma unroll
     for (int kk = 0; kk < K; ++kk) {
-      copy_step(kk, kk + K);
+      copy_step((kk + K - late) % K, kk + K - late);
       __builtin_amdgcn_sched_barrier(0);
       __asm__ __volatile__("s_waitcnt vmcnt(%0)" ::"n"(kWait) : "memory");
       __builtin_amdgcn_s_barrier();
@@ -591,19 +630,18 @@ __device__ __forceinline__ void ring_copy_sweep(int nsteps, const int* pos, int 
 // every resource.
 constexpr int kRingDummyRow = 0x3fe00000;
 
-// Sweep of the wave that moves the row data (right-hand sides, pivots, ring slots
-// and row ids), as ring_copy_sweep the records; the row ids that the right-hand
-// sides' addresses need are loaded K steps before them.
-template <typename V, int K, int CG, int NG, int NH, bool UPPER>
-__device__ __forceinline__ void ring_row_sweep(int nsteps, const int* pos, int rows, int nrhs, int c0, int dummy,
-                                               __amdgpu_buffer_rsrc_t rs_info, __amdgpu_buffer_rsrc_t rs_dinv,
-                                               __amdgpu_buffer_rsrc_t rs_src) {
+// Sweep of the wave that moves the right-hand sides, as ring_copy_sweep the
+// records; the row ids that their addresses need are loaded K steps before them.
+template <typename V, int K, int CG, int NG, int NH>
+__device__ __forceinline__ void ring_row_sweep(int nsteps, const int* pos, int rows, int nrhs, int c0,
+                                               __amdgpu_buffer_rsrc_t rs_info, __amdgpu_buffer_rsrc_t rs_src) {
   constexpr int VS = (int)sizeof(V);
   using L = RingLds<V, CG, NG, NH>;
   using R = typename L::R;
   constexpr int ND = R::ND, U = R::U;
-  constexpr int OPS = 2 * ND + (UPPER ? 2 : 1);
-  constexpr int kWait = K > 2 ? (K - 2) * OPS : 0;
+  constexpr int OPS = 2 * ND;
+  constexpr int late = ring_late<NH, K>() ? 1 : 0;
+  constexpr int kWait = K > 2 ? (K - 2 - late) * OPS : 0;
   static_assert(kWait <= 60, "outstanding loads");
   static_assert(3 * K + 2 <= 64, "step boundaries of a pass and its look-ahead in one register");
   const int lane = threadIdx.x & 63;
@@ -627,22 +665,11 @@ __device__ __forceinline__ void ring_row_sweep(int nsteps, const int* pos, int r
     for (int j = 0; j < ND; ++j)
       rowr[k][j] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_info, rl[j] < n ? rl[j] * 8 + 4 : kRingOut, p * 8, 0);
   };
-  // row data of step i of the pass into stage k, its row ids in rowr[k].  Lanes
-  // past the step's rows copy the dummy row's pair and, for the rest, zeros (no
-  // memory traffic).
+  // right-hand sides of step i of the pass into stage k, their row ids in
+  // rowr[k]; lanes past the step's rows copy zeros (no memory traffic)
   auto copy_step = [&](int k, int i) {
     const int p = bnd(i), n = bnd(i + 1) - p;
     const unsigned a = stage0 + k * L::stage + L::rec;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_info, (LP)(size_t)a, 4,
-                                             lane < 2 * n ? lane * 4 : dummy - p * 8 + (lane & 1) * 4, p * 8, 0, 0);
-    if constexpr (UPPER) {
-      if constexpr (VS == 16)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_dinv, (LP)(size_t)(a + L::info), 16, lane < n ? lane * 16 : kRingOut,
-                                                 p * VS, 0, 0);
-      else
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_dinv, (LP)(size_t)(a + L::info), 4,
-                                                 lane < n * (VS / 4) ? lane * 4 : kRingOut, p * VS, 0, 0);
-    }
 #pragma unroll
     for (int j = 0; j < ND; ++j) {
       const int o = (int)((unsigned)rowr[k][j] << csh) * VS + rb[j];
@@ -653,9 +680,9 @@ __device__ __forceinline__ void ring_row_sweep(int nsteps, const int* pos, int r
 #pragma unroll
   for (int k = 0; k < K; ++k) load_row(k, k);
 #pragma unroll
-  for (int k = 0; k < K; ++k) copy_step(k, k);
+  for (int k = 0; k < K - late; ++k) copy_step(k, k);
 #pragma unroll
-  for (int k = 0; k < K; ++k) load_row(k, K + k);
+  for (int k = 0; k < K - late; ++k) load_row(k, K + k);
   // The compiler gives the loop's first steps the load waits of the worst
   // path into them.  Taking the prologue's registers as redefined here (one
   // wait for its loads, once per sweep) leaves the loop the waits of its own
@@ -668,14 +695,14 @@ __device__ __forceinline__ void ring_row_sweep(int nsteps, const int* pos, int r
     for (int j = 0; j < ND; ++j) pin_reg(rowr[k][j]);
   __builtin_amdgcn_s_barrier();
   // the solving waves take step 0 here, before its stage is used again
-  __builtin_amdgcn_s_barrier();
+  if constexpr (!late) __builtin_amdgcn_s_barrier();
   __asm__ __volatile__("" ::: "memory");
   for (int base = 0; base < nsteps; base += K) {
     const int pvn = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_pos, min(base + K + lane, nsteps) * 4, 0, 0);
 #pragma unroll
     for (int kk = 0; kk < K; ++kk) {
-      copy_step(kk, kk + K);
-      load_row(kk, kk + 2 * K);
+      copy_step((kk + K - late) % K, kk + K - late);
+      load_row((kk + K - late) % K, kk + 2 * K - late);
       __builtin_amdgcn_sched_barrier(0);
       __asm__ __volatile__("s_waitcnt vmcnt(%0)" ::"n"(kWait) : "memory");
       __builtin_amdgcn_s_barrier();
@@ -696,6 +723,11 @@ __device__ __forceinline__ void ring_solve_sweep(int h, int g, int nsteps, int r
   using L = RingLds<V, CG, NG, NH>;
   constexpr int NCL = CG == 8 ? 2 : 1;  // columns finalized per lane: adjacent ones, one access for both
   static_assert(CG == 1 || CG == 2 || CG == 4 || (CG == 8 && VS == 4), "columns per group");
+  // Left alone, the compiler moves reads of the next step's stage before the last
+  // gathers and their waits into the sum.  Holding it back: 64^3, 8 / 64 FP32
+  // columns 169 -> 160 and 274 -> 253 us; 128^3, 1 column 516 -> 498; but with
+  // several columns and two waves per group up to 3 % slower.
+  constexpr bool kOrder = NH == 1 || CG == 1;
   const int lane = threadIdx.x & 63;
   const int q = lane % 4;
   const int t = 16 * h + lane / 4;                      // this lane's row of the step
@@ -757,7 +789,7 @@ __device__ __forceinline__ void ring_solve_sweep(int h, int g, int nsteps, int r
 
   __syncthreads();  // the loading waves have filled the first stages
   take(0);
-  __syncthreads();  // step 0 is taken: its stage may be used again
+  if constexpr (!ring_late<NH, K>()) __syncthreads();  // step 0 is taken: its stage may be used again
   for (int base = 0; base < nsteps; base += K) {
 #pragma unroll
     for (int kk = 0; kk < K; ++kk) {
@@ -778,6 +810,7 @@ __device__ __forceinline__ void ring_solve_sweep(int h, int g, int nsteps, int r
       for (int j = 0; j < NCL; ++j) x0[j] = xin[j];
       const V d0 = dv;
       // the next step's records and row data follow the gathers in the LDS queue
+      if constexpr (kOrder) __builtin_amdgcn_sched_barrier(0);
       take((kk + 1) % K);
       V acc[CG];
 #pragma unroll
@@ -787,6 +820,8 @@ __device__ __forceinline__ void ring_solve_sweep(int h, int g, int nsteps, int r
 #pragma unroll
         for (int c = 0; c < CG; ++c) acc[c] += wgt[e] * xv[e].v[c];
       }
+      // nothing that waits for the reads after the gathers comes before this
+      if constexpr (kOrder) __builtin_amdgcn_sched_barrier(0);
       // sum over the row's lanes, scattered so that lane q ends with column q % CG
       // (with 8 columns: columns 2q and 2q + 1)
       V a[NCL];
@@ -831,7 +866,13 @@ __device__ __forceinline__ void ring_solve_sweep(int h, int g, int nsteps, int r
         lds_write(wa, v);
         bstore_val(rs_dst, off, v);
       }
-      __syncthreads();
+      if constexpr (ring_late<NH, K>()) {
+        __asm__ __volatile__("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __asm__ __volatile__("" ::: "memory");
+      } else {
+        __syncthreads();
+      }
     }
   }
 }
@@ -843,7 +884,7 @@ __device__ __forceinline__ void ring_solve_sweep(int h, int g, int nsteps, int r
 // after the last block's; ent: the block's records, from blk_ri0[b] *
 // ring_row_bytes<V>().
 template <typename V, int K, int CG, int NG, int NH>
-__global__ __launch_bounds__(64 * (NH * NG + 2)) void k_trsv_ring(
+__global__ __launch_bounds__(64 * (NH * NG + NH + 1)) void k_trsv_ring(
     int nblocks, int rows, const int* __restrict__ blk_row0, const int* __restrict__ blk_step,
     const int* __restrict__ blk_stepU, const int64_t* __restrict__ blk_ri0, const int* __restrict__ pos,
     const unsigned char* __restrict__ ent, const int2* __restrict__ info, const V* __restrict__ dinv,
@@ -858,10 +899,11 @@ __global__ __launch_bounds__(64 * (NH * NG + 2)) void k_trsv_ring(
   const int64_t vbytes = (int64_t)nb * nrhs * (int64_t)sizeof(V);
   V* xb = x + (int64_t)r0 * nrhs;
   const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(xb, vbytes);
+  const __amdgpu_buffer_rsrc_t rs_info = make_rsrc(info + q0, (nd + 1) * 8);
   // rings, dummy rows and stages start as zeros: a record that is not there reads
   // slot 0 with weight zero
   uint4* lds4 = reinterpret_cast<uint4*>(smem_raw);
-  for (int i = threadIdx.x; i < RingLds<V, CG, NG, NH>::bytes(rows, K) / 16; i += 64 * (NH * NG + 2)) lds4[i] = uint4{0, 0, 0, 0};
+  for (int i = threadIdx.x; i < RingLds<V, CG, NG, NH>::bytes(rows, K) / 16; i += 64 * (NH * NG + NH + 1)) lds4[i] = uint4{0, 0, 0, 0};
   __syncthreads();
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (w < NH * NG) {
@@ -872,19 +914,22 @@ __global__ __launch_bounds__(64 * (NH * NG + 2)) void k_trsv_ring(
     __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     ring_solve_sweep<V, K, CG, NG, NH, true>(h, g, send - sU, rows, nrhs, c0, rs_x);
-  } else if (w == NH * NG) {
+  } else if (w < NH * NG + NH) {
     const __amdgpu_buffer_rsrc_t rs_ent = make_rsrc(ent + q0 * ring_row_bytes<V>(), np * ring_row_bytes<V>());
-    ring_copy_sweep<V, K, CG, NG, NH>(sU - sbeg, pb, rows, rs_ent);
-    __syncthreads();
-    ring_copy_sweep<V, K, CG, NG, NH>(send - sU, pb + (sU - sbeg), rows, rs_ent);
-  } else {
-    const __amdgpu_buffer_rsrc_t rs_info = make_rsrc(info + q0, (nd + 1) * 8);
     const __amdgpu_buffer_rsrc_t rs_dinv = make_rsrc(dinv + q0, np * (int64_t)sizeof(V));
     const int dummy = (int)(nd * 8);
-    ring_row_sweep<V, K, CG, NG, NH, false>(sU - sbeg, pb, rows, nrhs, c0, dummy, rs_info, rs_dinv,
-                                        make_rsrc(rhs + (int64_t)r0 * nrhs, vbytes));
+    auto copies = [&](auto hc) {
+      constexpr int HC = decltype(hc)::value;
+      ring_copy_sweep<V, K, CG, NG, NH, HC, false>(sU - sbeg, pb, rows, dummy, rs_ent, rs_info, rs_dinv);
+      __syncthreads();
+      ring_copy_sweep<V, K, CG, NG, NH, HC, true>(send - sU, pb + (sU - sbeg), rows, dummy, rs_ent, rs_info, rs_dinv);
+    };
+    if (NH == 1 || w == NH * NG) copies(std::integral_constant<int, 0>());
+    else copies(std::integral_constant<int, NH - 1>());
+  } else {
+    ring_row_sweep<V, K, CG, NG, NH>(sU - sbeg, pb, rows, nrhs, c0, rs_info, make_rsrc(rhs + (int64_t)r0 * nrhs, vbytes));
     __syncthreads();
-    ring_row_sweep<V, K, CG, NG, NH, true>(send - sU, pb + (sU - sbeg), rows, nrhs, c0, dummy, rs_info, rs_dinv, rs_x);
+    ring_row_sweep<V, K, CG, NG, NH>(send - sU, pb + (sU - sbeg), rows, nrhs, c0, rs_info, rs_x);
   }
 }
 
