@@ -1590,14 +1590,35 @@ int fgmres_impl(pgs_dev_op_s* op, pgs_ws_s* ws, const S* b, S* x, int nrhs, cons
       }
       hadd = h2;
     } else {
-      // PargemslrMgs (matrixops.cpp:10728-10807): one (dot, axpy) pair per basis vector
+      // PargemslrMgs (matrixops.cpp:10728-10807): launch j takes out v_{j-1} and
+      // has the dot with v_j, the last one the norm; the partials go to two
+      // places in turn, the norm's to the first
       const double vb = (double)n * nrhs * sizeof(S);
-      for (int j = 0; j < i; ++j) {
-        timed(ws, ss, PGS_PROF_ORTH_DOTS, 2.0 * vb, [&] {
-          multidot<S, S, S>(ws, n, nrhs, 1, V + (int64_t)j * ldv, ldv, w, h + (int64_t)j * nrhs, 0, ss);
-        });
-        timed(ws, ss, PGS_PROF_ORTH_UPDATE, 3.0 * vb, [&] {
-          nblk = multi_axpy<S>(ws, n, nrhs, 1, V + (int64_t)j * ldv, ldv, h + (int64_t)j * nrhs, w, j == i - 1, ss);
+      constexpr int E = 16 / (int)sizeof(S);
+      const int64_t want = (n * nrhs + kMgsNT * E - 1) / (kMgsNT * E);
+      nblk = (int)std::max<int64_t>(1, std::min<int64_t>(ws->part_blocks, want));
+      S* part = ws->part.as<S>();
+      const S* prev = nullptr;
+      int nprev = 0;
+      for (int j = 0; j <= i; ++j) {
+        const S* vp = j > 0 ? V + (int64_t)(j - 1) * ldv : nullptr;
+        const S* vn = j < i ? V + (int64_t)j * ldv : nullptr;
+        S* out = part + (int64_t)((i - j) & 1) * nblk * nrhs;
+        S* hj = h + (int64_t)(j - 1) * nrhs;
+        S* hout = nprev > 0 && prev != hj ? hj : nullptr;
+        timed(ws, ss, j == 0 ? PGS_PROF_ORTH_DOTS : PGS_PROF_ORTH_UPDATE, (j == 0 ? 2.0 : j < i ? 4.0 : 3.0) * vb, [&] {
+          if (E == 2 && nrhs == 1)
+            k_mgs_step<S, E == 2><<<nblk, kMgsNT, 0, ss>>>(n, nrhs, nprev, prev, hout, vp, vn, w, out);
+          else
+            k_mgs_step<S, false><<<nblk, kMgsNT, 0, ss>>>(n, nrhs, nprev, prev, hout, vp, vn, w, out);
+          if (j < i && nblk * nrhs > kMgsPartials) {
+            dot_final<S>(nblk, 1, nrhs, out, h + (int64_t)j * nrhs, 0, ss);
+            prev = h + (int64_t)j * nrhs;
+            nprev = 1;
+          } else {
+            prev = out;
+            nprev = nblk;
+          }
         });
       }
     }

@@ -1014,6 +1014,104 @@ __global__ __launch_bounds__(NT) void k_dcgs2_update(int64_t n, int nrhs, int p,
   }
 }
 
+// One launch of modified Gram-Schmidt: w -= vp h with h = vp^H w summed here
+// from nprev partials (a row of nrhs values each; none: w stays), then partials
+// of vn^H w, or, without vn, of ||w||^2 (doubles), one row of nrhs values per
+// workgroup in part.  h is kept in hout (may be null).  A step against i vectors
+// is i + 1 of these, each reading w, vp and vn and writing w, where a dot, its
+// sum and an update took three launches per vector and read w once more: 48^3,
+// one column, 11.2 -> 4.5 us per vector; 128^3, 20 steps,
+// 1 column 7.2 -> 4.8 ms, 16 columns 66 -> 54.  Every workgroup adds up all partials
+// itself, which costs less than a launch up to kMgsPartials values.
+// ONE: a single real column.
+constexpr int kMgsNT = 256;
+constexpr int kMgsPartials = 4096;
+
+template <typename S, bool ONE>
+__global__ __launch_bounds__(kMgsNT) void k_mgs_step(int64_t n, int nrhs, int nprev, const S* __restrict__ prev,
+                                                     S* __restrict__ hout, const S* __restrict__ vp,
+                                                     const S* __restrict__ vn, S* __restrict__ w,
+                                                     S* __restrict__ part) {
+  constexpr int E = 16 / (int)sizeof(S), NW = kMgsNT / kWave;
+  __shared__ S red[NW][64];
+  __shared__ S hs[64];
+  const int tid = threadIdx.x, lane = tid % kWave, wid = tid / kWave;
+  if (nprev > 0) {
+    S t = S(0.0);
+#pragma unroll 4
+    for (int b = row_of(tid, nrhs); b < nprev; b += kMgsNT / nrhs) t += prev[b * nrhs + col_of(tid, nrhs)];
+    t = lane_class_sum(t, nrhs);
+    if (lane < nrhs) red[wid][lane] = t;
+    __syncthreads();
+    if (tid < nrhs) {
+      for (int k = 1; k < NW; ++k) t += red[k][tid];
+      hs[tid] = t;
+      if (hout && blockIdx.x == 0) hout[tid] = t;
+    }
+    __syncthreads();
+  }
+  const int c = ONE ? 0 : (tid * E) % nrhs;  // the lane's first column (the grid stride keeps it)
+  f64x2 h = {0.0, 0.0};
+  if (nprev > 0) {
+    if constexpr (ONE) h = f64x2{hs[0], hs[0]};
+    else h = *reinterpret_cast<const f64x2_a8*>(&hs[c]);
+  }
+  f64x2 acc = {0.0, 0.0};
+  const int64_t total = n * nrhs;
+  const int64_t stride = (int64_t)gridDim.x * kMgsNT * E;
+  int64_t g = ((int64_t)blockIdx.x * kMgsNT + tid) * E;
+  for (; g + E <= total; g += stride) {
+    f64x2 wv = load16(w + g);
+    const f64x2 nv = vn ? load16(vn + g) : f64x2{0.0, 0.0};
+    if (nprev > 0) {
+      const f64x2 pv = load16(vp + g);
+      if constexpr (E == 2) {
+        wv -= pv * h;
+      } else {
+        wv.x -= pv.x * h.x - pv.y * h.y;
+        wv.y -= pv.x * h.y + pv.y * h.x;
+      }
+      *reinterpret_cast<f64x2_a8*>(w + g) = wv;
+    }
+    const f64x2 x = vn ? nv : wv;
+    if constexpr (E == 2) {
+      acc += x * wv;
+    } else {
+      acc.x += x.x * wv.x + x.y * wv.y;
+      acc.y += x.x * wv.y - x.y * wv.x;
+    }
+  }
+  if constexpr (ONE) {
+    if (g < total) {  // the last value of an odd length
+      double wv = w[g];
+      if (nprev > 0) w[g] = wv = wv - vp[g] * hs[0];
+      acc.x += (vn ? vn[g] : wv) * wv;
+    }
+  }
+  __syncthreads();
+  if constexpr (E == 1) {
+    const S t = lane_class_sum(S(acc.x, acc.y), nrhs);
+    if (lane < nrhs) red[wid][lane] = t;
+  } else if constexpr (ONE) {
+    const double t = lane_class_sum(acc.x + acc.y, 1);
+    if (lane == 0) red[wid][0] = t;
+  } else {
+    double a[2] = {acc.x, acc.y};
+    lane_class_sums<2>(a, nrhs / 2);
+    if (lane < nrhs / 2) {
+      red[wid][2 * lane] = a[0];
+      red[wid][2 * lane + 1] = a[1];
+    }
+  }
+  __syncthreads();
+  if (tid < nrhs) {
+    S t = red[0][tid];
+    for (int k = 1; k < NW; ++k) t += red[k][tid];
+    if (vn) part[(int64_t)blockIdx.x * nrhs + tid] = t;
+    else reinterpret_cast<double*>(part)[(int64_t)blockIdx.x * nrhs + tid] = sreal(t);
+  }
+}
+
 // Per column (one workgroup of 64 lanes, blockIdx.x = column), after the
 // dots of step p.  The basis slots hold raw vectors: slot j < p is step j's
 // first projection as k_dcgs2_update left it, and the final (orthonormal)

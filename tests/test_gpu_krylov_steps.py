@@ -60,3 +60,10 @@ def test_fixed_steps(ops, gpu, grid, cx, nr, kdim, maxits, orth):
         assert res[c][1] == ito == maxits
         assert abs(res[c][2] - rro) <= 1e-9 * max(rro, 1e-3)
         assert np.linalg.norm(x[:, c] - xo) <= 1e-9 * np.linalg.norm(xo)
+
+
+@pytest.mark.parametrize("nr", [16, 32, 64])
+def test_mgs_partials(ops, gpu, nr):
+    """MGS where every workgroup adds up the dots' partials itself (up to 4096
+    values: 16 and 32 columns of 32^3 rows) and where a kernel of its own does."""
+    test_fixed_steps(ops, gpu, (32, 32, 32), False, nr, 7, 17, pg.PGS_ORTH_MGS)
