@@ -758,6 +758,12 @@ void launch_lowrank(pgs_ws_s* ws, const DevLevel& L, V* zl, int nrhs, hipStream_
     nblk = (m + rows_per_blk - 1) / rows_per_blk;
     k_lr_dot<V, kNT><<<nblk, kNT, 0, s>>>(m, k, nrhs, L.W.as<V>(), zl, part, rows_per_blk);
   }
+  if ((int64_t)nblk * k * nrhs <= kLrFused && k * nrhs <= kLrFused / 2) {  // t in LDS: at most 32 KB
+    k_lr_update_sum<V, kNT><<<nblocks_for((int64_t)m * nrhs, kNT), kNT, sizeof(V) * (size_t)k * nrhs, s>>>(
+        m, k, nrhs, nblk, L.WH.as<V>(), part, zl);
+    HIPCHK(hipGetLastError());
+    return;
+  }
   k_lr_final<V><<<(k * nrhs + 3) / 4, 256, 0, s>>>(nblk, k, nrhs, part, t);
   k_lr_update<V><<<nblocks_for((int64_t)m * nrhs, kNT), kNT, 0, s>>>(m, k, nrhs, L.WH.as<V>(), t, zl);
   HIPCHK(hipGetLastError());

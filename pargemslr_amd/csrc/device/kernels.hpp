@@ -50,6 +50,20 @@ __device__ __forceinline__ double lane_step(double v) {
     return v + __builtin_bit_cast(double, (unsigned long long)h << 32 | l);
   }
 }
+template <int M>
+__device__ __forceinline__ float lane_step(float v) {
+  const unsigned u = __float_as_uint(v);
+  if constexpr (M == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  } else if constexpr (M == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  } else {
+    constexpr int ctrl = M == 8 ? 0x128 : M == 4 ? 0x124 : M == 2 ? 0x4E : 0xB1;
+    return v + __int_as_float(__builtin_amdgcn_mov_dpp((int)u, ctrl, 0xF, 0xF, true));
+  }
+}
 template <int M, typename R>
 __device__ __forceinline__ cplx<R> lane_step(cplx<R> v) {
   return cplx<R>(lane_step<M>(v.re), lane_step<M>(v.im));
@@ -369,14 +383,10 @@ __global__ __launch_bounds__(NT) void k_lr_dot_reg(int m, int k, int nrhs, const
       if (j < k) acc[j] += sconj(wr[j]) * zv;
   }
   const int wid = tid / 64, lane = tid % 64;
+  lane_class_sums<KM>(acc, nrhs);
 #pragma unroll
-  for (int j = 0; j < KM; ++j) {
-    if (j < k) {
-      V s = acc[j];
-      for (int o = 32; o >= nrhs; o >>= 1) s += shfl_xor_v(s, o);
-      if (lane < nrhs) red[(wid * k + j) * nrhs + lane] = s;
-    }
-  }
+  for (int j = 0; j < KM; ++j)
+    if (j < k && lane < nrhs) red[(wid * k + j) * nrhs + lane] = acc[j];
   __syncthreads();
   for (int t = tid; t < k * nrhs; t += NT) {
     V s = 0;
@@ -396,6 +406,51 @@ __global__ void k_lr_final(int nblk, int k, int nrhs, const V* __restrict__ part
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += shfl_xor_v(s, o);
   if (lane == 0) t[g] = s;
+}
+
+// z += WH t with t summed here from the nblk partials of stage 1, by every
+// workgroup for itself: while the partials are few (kLrFused values) that costs
+// less than the launch that would sum them.  Stage 1 with its lane sums by lane
+// permutes and this: 48^3, one FP64 column, rank 16, 20 -> 10.1 us per term in three
+// launches -> two.  Dynamic LDS: k * nrhs values.
+constexpr int kLrFused = 4096;
+
+template <typename V, int NT>
+__global__ __launch_bounds__(NT) void k_lr_update_sum(int m, int k, int nrhs, int nblk, const V* __restrict__ WH,
+                                                      const V* __restrict__ part, V* __restrict__ z) {
+  extern __shared__ unsigned char lu_smem[];
+  V* t = reinterpret_cast<V*>(lu_smem);
+  __shared__ V red[NT];
+  const int no = k * nrhs, tid = threadIdx.x;
+  if (no >= NT) {
+    for (int o = tid; o < no; o += NT) {
+      V s = part[o];
+#pragma unroll 4
+      for (int b = 1; b < nblk; ++b) s += part[b * no + o];
+      t[o] = s;
+    }
+  } else {
+    const int ng = NT / no, g = tid / no, o = tid % no;
+    V s = 0;
+    if (g < ng) {
+#pragma unroll 4
+      for (int b = g; b < nblk; b += ng) s += part[b * no + o];
+    }
+    red[tid] = s;
+    __syncthreads();
+    if (tid < no) {
+      for (int q = 1; q < ng; ++q) s += red[q * no + tid];
+      t[tid] = s;
+    }
+  }
+  __syncthreads();
+  const int64_t g = (int64_t)blockIdx.x * NT + tid;
+  if (g >= (int64_t)m * nrhs) return;
+  const int64_t i = row_of(g, nrhs);
+  const int c = col_of(g, nrhs);
+  V acc = 0;
+  for (int j = 0; j < k; ++j) acc += WH[i * k + j] * t[j * nrhs + c];
+  z[g] += acc;
 }
 
 template <typename V>
