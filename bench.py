@@ -43,9 +43,9 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes read + written per level-0 ring-solve launch of the 128^3 operator
 # (FP32 apply), by right-hand sides per launch, measured with rocprofv3
 # FETCH_SIZE and WRITE_SIZE passes over `bench.py --probe --nrhs N`, each
-# scaled by what the counter reads for a 1 GiB device copy (8-column groups: of
-# 128 threads on whole steps at 32 columns, one wave on half steps at 64)
-TRAFFIC_LEVEL0 = {32: 1667.6e6, 64: 2742.2e6}
+# scaled by what the counter reads for a 1 GiB device copy (whole steps, 8
+# columns per workgroup at 32 columns, 16 at 64)
+TRAFFIC_LEVEL0 = {32: 1539.0e6, 64: 2538.5e6}
 
 
 def log(*a):

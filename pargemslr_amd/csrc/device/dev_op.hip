@@ -353,6 +353,7 @@ namespace {
 constexpr int kNT = 256;
 constexpr int kTrsvNT = 256;
 constexpr int kPMAX = 128;  // Krylov dimension + 1 limit of the shared-memory coefficient tables
+static_assert(kPMAX <= 128 && PGS_SCHUR_MAXITS_LIMIT < 128, "k_backsolve holds 128 values");
 constexpr int kLrBlocks = 1024;  // most workgroups (partial sums) of the low-rank stage 1
 constexpr int kBasisNT = 256;
 constexpr int kBasisPM = 64;  // most basis vectors k_basis_reg takes
