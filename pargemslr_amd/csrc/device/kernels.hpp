@@ -1167,7 +1167,7 @@ __global__ __launch_bounds__(kMgsNT) void k_mgs_step(int64_t n, int nrhs, int np
   }
 }
 
-// Per column (one workgroup of 64 lanes, blockIdx.x = column), after the
+// Per column (one workgroup, blockIdx.x = column), after the
 // dots of step p.  The basis slots hold raw vectors: slot j < p is step j's
 // first projection as k_dcgs2_update left it, and the final (orthonormal)
 // basis is v_j = sum_{i<=j} slot_i R[i, j], R upper triangular (row-major,
