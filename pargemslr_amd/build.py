@@ -19,7 +19,7 @@ HOST_SRC = ["host/partition.cpp", "host/rcm_ilut.cpp", "host/dense.cpp", "host/g
 HIP_SRC = ["device/dev_op.hip", "device/server.hip"]
 
 # host-only checks built a second time with AddressSanitizer and UBSan (g++,
-# no HIP code): the setup, the level-set packing and its replay, the thread pool
+# no HIP code): the setup, the level-set packing and its replays, the thread pool
 SAN_SRC = ["host/partition.cpp", "host/rcm_ilut.cpp", "host/dense.cpp", "host/gemslr_setup.cpp", "host/gen.cpp",
            "host/trsv_pack.cpp"]
 SAN_FLAGS = ["-O1", "-g", "-std=c++17", "-fsanitize=address,undefined", "-fno-omit-frame-pointer",
@@ -53,10 +53,13 @@ def build(verbose=False):
     root = os.path.dirname(HERE)
     san_dir = os.path.join(OBJ, "san")
     os.makedirs(san_dir, exist_ok=True)
-    san_objs = []
-    for s in SAN_SRC + ["../../tests/cpp/pack_check.cpp"]:
+    san_objs, san_main = [], {}
+    for s in SAN_SRC + ["../../tests/cpp/pack_check.cpp", "../../tests/cpp/ring_check.cpp"]:
         o = os.path.join(san_dir, os.path.basename(s) + ".o")
-        san_objs.append(o)
+        if s in SAN_SRC:
+            san_objs.append(o)
+        else:
+            san_main[os.path.basename(s)[:-4]] = o
         jobs.append(["g++"] + SAN_FLAGS + ["-I", os.path.join(root, "include"), "-c", os.path.join(CSRC, s), "-o", o])
     with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(jobs))) as ex:
         outs = list(ex.map(_run, jobs))
@@ -69,11 +72,12 @@ def build(verbose=False):
     _run([HIPCC, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp] + objs + ["-pthread"])
     os.replace(tmp, LIB)
     cpp = os.path.join(root, "tests", "cpp")
-    _run(["g++"] + SAN_FLAGS + san_objs + ["-o", os.path.join(cpp, "pack_check_san")])
+    for name, o in san_main.items():
+        _run(["g++"] + SAN_FLAGS + san_objs + [o, "-o", os.path.join(cpp, name + "_san")])
     _run(["g++"] + SAN_FLAGS + [os.path.join(cpp, "parallel_for_check.cpp"), "-o",
                                 os.path.join(cpp, "parallel_for_check_san")])
     # C++ driver on the class surface (include/pargemslr_amd.hpp), run by the tests
-    for name in ("driver_laplacian", "driver_gen", "driver_surface", "pack_check"):
+    for name in ("driver_laplacian", "driver_gen", "driver_surface", "pack_check", "ring_check"):
         drv_src = os.path.join(root, "tests", "cpp", name + ".cpp")
         if os.path.exists(drv_src):
             drv = os.path.join(root, "tests", "cpp", name)

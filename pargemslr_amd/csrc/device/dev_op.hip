@@ -200,8 +200,8 @@ void upload_trsv(DevTrsv& d, const TrsvPack<T>& P, int64_t* counter) {
     upload(d.stepU_h, suh, counter);
     upload(d.pos_h, step_bounds(dh, sh), counter);
     // the packed slots are positions modulo a power of two; the device's ring
-    // holds just the window's rows (a fifth less LDS at 128^3: room for more
-    // columns or stages): slot = position modulo the window
+    // holds just the rows needed (a fifth less LDS at 128^3: room for more
+    // columns or stages): slot = position modulo those
     const int W = P.window, wn = std::max(P.window_needed, 1);
     if (wn > 0xffff) throw std::runtime_error("sweep window too large for 16-bit slots");
     d.window = wn;

@@ -141,7 +141,12 @@ TrsvPack<T> trsv_pack(const HostLevel<T>& L, int lev_start, int nloc, int max_ro
     else oU[t / 2] = best_order(F.U, true, max_rows);
   });
   for (int b = 0; b < L.ncomp; ++b)
-    P.window_needed = std::max(P.window_needed, std::max(oL[b].window, oU[b].window));
+    for (const SweepOrder* o : {&oL[b], &oU[b]}) {
+      P.window_needed = std::max(P.window_needed, o->window);
+      // nothing orders the writes of a step's rows: a slot each
+      for (size_t s = 0; s + 1 < o->step.size(); ++s)
+        P.window_needed = std::max(P.window_needed, o->step[s + 1] - o->step[s]);
+    }
   int W = 1;
   while (W < P.window_needed) W <<= 1;
   int row_len = 0;

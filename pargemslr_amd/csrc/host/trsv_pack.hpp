@@ -21,11 +21,15 @@
 // Sweep window.  Number the row pairs of a block in storage order (all L rows,
 // then all U rows); a row's position is its pair index.  The window of a
 // sweep is the largest (end position of a step) - (position of a row that
-// step reads).  When it is at most W (a power of two), a solve can keep x in
-// a ring of W slots, slot = position & (W - 1): no value is overwritten before
-// its last reader has run.  With `max_window` > 0 and every sweep's window
-// within it, the ELL columns hold those slots instead of row ids and
-// `window` is the ring size; otherwise columns are block-local row ids and
+// step reads).  A ring holds x if it has at least that many slots, slot =
+// position modulo the slots, so that no later step overwrites a value before its
+// last reader has run, and at least as many as the longest step has rows, so
+// that the rows of a step, whose writes nothing orders, have a slot each
+// (otherwise the slot of a row that is read later can end with the value of one
+// of its own step that is not).  `window_needed` is the larger of the two.  With
+// `max_window` > 0 and the next power of two W within it, the ELL columns
+// hold the slots position & (W - 1) instead of row ids and
+// `window` is W; otherwise columns are block-local row ids and
 // `window` is 0.  Ring-packed slabs have a fixed width, so a lane that reads
 // slot j of its row never reaches into the next row, and padded slots weigh
 // zero.
@@ -45,7 +49,7 @@ struct TrsvPack {
   int max_block_rows = 0;
   int max_steps = 0;                 // deepest block, L + U steps
   int max_width = 0;                 // widest step
-  int window_needed = 0;             // largest sweep window over all blocks
+  int window_needed = 0;             // slots a ring needs: largest sweep window, longest step
   int window = 0;                    // ring size when columns are ring slots, else 0
   std::vector<int> blk_row0;         // nblocks+1, level-local first row of each block
   std::vector<int> blk_step;         // nblocks+1, step ranges into desc
