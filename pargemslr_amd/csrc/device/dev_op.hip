@@ -14,6 +14,7 @@
 
 #include "../../../include/pargemslr_amd.h"
 #include "../host/gemslr_host.hpp"
+#include "../host/ring_pack.hpp"
 #include "../host/trsv_pack.hpp"
 #include "capi_internal.hpp"
 #include "kernels.hpp"
@@ -145,7 +146,7 @@ struct DevTrsv {
   // levels solved by the pipelined and direct kernels
   DevMem ent0, desc, ent, ri;
   // ring-packed levels: step boundaries, lane records, (slot, row id) pairs and
-  // 1/pivots by position (layouts at k_trsv_ring)
+  // 1/pivots by position (RingPack)
   DevMem pos, rec, info, dinv;
   int64_t positions = 0;
   // half steps: a step of more than 16 rows walked as two consecutive ones (rows
@@ -154,23 +155,6 @@ struct DevTrsv {
   int64_t max_block_steps_h = 0;
   DevMem step_h, stepU_h, pos_h;
 };
-
-// Step boundaries of every block (layout at k_trsv_ring) from the step
-// descriptors (desc: 4 per step, the first position at 0 and the rows at 2).
-std::vector<int> step_bounds(const std::vector<int>& desc, const std::vector<int>& blk_step) {
-  const int nb = (int)blk_step.size() - 1;
-  std::vector<int> pos((size_t)blk_step[nb] + nb);
-  for (int b = 0; b < nb; ++b) {
-    int* q = pos.data() + blk_step[b] + b;
-    int end = 0;
-    for (int s = blk_step[b]; s < blk_step[b + 1]; ++s) {
-      *q++ = desc[4 * s];
-      end = desc[4 * s] + desc[4 * s + 2];
-    }
-    *q = end;
-  }
-  return pos;
-}
 
 template <typename V, typename T>
 void upload_trsv(DevTrsv& d, const TrsvPack<T>& P, int64_t* counter) {
@@ -181,55 +165,23 @@ void upload_trsv(DevTrsv& d, const TrsvPack<T>& P, int64_t* counter) {
   d.max_width = P.max_width;
   d.window = P.window;
   d.nnz_real = P.nnz_real;
-  d.max_block_steps = 0;
-  for (int b = 0; b < P.nblocks; ++b)
-    d.max_block_steps = std::max<int64_t>(d.max_block_steps, P.blk_step[b + 1] - P.blk_step[b]);
   upload(d.row0, P.blk_row0, counter);
   upload(d.step, P.blk_step, counter);
   upload(d.stepU, P.blk_stepU, counter);
   upload(d.ri0, P.blk_ri0, counter);
   const int64_t nr = (int64_t)P.rows.size();
   if (P.window > 0) {
-    upload(d.pos, step_bounds(P.desc, P.blk_step), counter);
-    std::vector<int> dh, sh, suh;
-    half_steps(P.desc, P.blk_step, P.blk_stepU, dh, sh, suh);
-    d.max_block_steps_h = 0;
-    for (int b = 0; b < P.nblocks; ++b)
-      d.max_block_steps_h = std::max<int64_t>(d.max_block_steps_h, sh[b + 1] - sh[b]);
-    upload(d.step_h, sh, counter);
-    upload(d.stepU_h, suh, counter);
-    upload(d.pos_h, step_bounds(dh, sh), counter);
-    // the packed slots are positions modulo a power of two; the device's ring
-    // holds just the rows needed (a fifth less LDS at 128^3: room for more
-    // columns or stages): slot = position modulo those
-    const int W = P.window, wn = std::max(P.window_needed, 1);
-    if (wn > 0xffff) throw std::runtime_error("sweep window too large for 16-bit slots");
-    d.window = wn;
+    const RingPack<V> R = ring_pack<V>(P, [](const T& v) { return hval<V>(v); });
+    d.window = R.rows;
     d.positions = nr;
-    constexpr int RB = ring_row_bytes<V>();
-    std::vector<unsigned char> rec((size_t)nr * RB);
-    std::vector<int2> info((size_t)nr + 1);
-    info[nr] = int2{wn * (int)sizeof(V), kRingDummyRow};
-    parallel_for(P.nblocks, [&](int b) {
-      for (int s = P.blk_step[b]; s < P.blk_step[b + 1]; ++s) {
-        const int* d4 = &P.desc[4 * (size_t)s];
-        const int end = d4[0] + d4[2];  // a row the step reads is at most W positions before it
-        for (int t = 0; t < d4[2]; ++t) {
-          const int64_t q = P.blk_ri0[b] + d4[0] + t;
-          info[q] = int2{(d4[0] + t) % wn * (int)sizeof(V), P.rows[q]};
-          const int t0 = t / kRingGroup * kRingGroup;  // first row of t's group
-          unsigned char* g = rec.data() + (P.blk_ri0[b] + d4[0] + t0) * RB;
-          for (int j = 0; j < d4[3]; ++j) {
-            const int64_t e = P.blk_ent0[b] + d4[1] + (int64_t)t * d4[3] + j;
-            // (padded entries weigh zero, whatever row they name)
-            const int p = std::max(0, end - 1 - ((end - 1 - P.col[e]) & (W - 1)));
-            store_rec<V>(g, std::min(kRingGroup, d4[2] - t0), t - t0, j, hval<V>(P.val[e]), (unsigned)(p % wn));
-          }
-        }
-      }
-    });
-    upload(d.rec, rec, counter);
-    upload(d.info, info, counter);
+    d.max_block_steps = R.max_block_steps;
+    d.max_block_steps_h = R.max_block_steps_h;
+    upload(d.pos, R.pos, counter);
+    upload(d.step_h, R.step_h, counter);
+    upload(d.stepU_h, R.stepU_h, counter);
+    upload(d.pos_h, R.pos_h, counter);
+    upload(d.rec, R.rec, counter);
+    upload(d.info, R.info, counter);
     upload(d.dinv, convert_vec<V>(P.dinv), counter);
     return;
   }
@@ -508,7 +460,6 @@ void launch_trsv_pipe(int nt, int lpr, const DevTrsv& T, const V* rhs, V* x, int
 }
 
 // Ring kernel: rows of at most kRingWidth entries, steps of at most 32 rows.
-constexpr int kRingWidth = 20;
 
 // Steps whose records are in LDS or on the way there: enough that a copy has
 // K - 3 steps to arrive (1 to 2 us), within the 63 copies that can be waited for
@@ -531,7 +482,7 @@ void launch_trsv_ring_k(const DevTrsv& T, const V* rhs, V* x, int nrhs, hipStrea
   const DevMem& pos = NH == 1 ? T.pos_h : T.pos;
   kern<<<grid, 64 * (NH * NG + NH + 1), lds, s>>>(T.nblocks, T.window, T.row0.as<int>(), step.as<int>(), stepU.as<int>(),
                                              T.ri0.as<int64_t>(), pos.as<int>(), T.rec.as<unsigned char>(),
-                                             T.info.as<int2>(), T.dinv.as<V>(), rhs, x, nrhs);
+                                             T.info.as<RingInfo>(), T.dinv.as<V>(), rhs, x, nrhs);
 }
 
 template <typename V>

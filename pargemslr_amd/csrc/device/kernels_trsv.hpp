@@ -20,6 +20,8 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "../host/ring_pack.hpp"
+
 namespace pgs {
 namespace dev {
 
@@ -415,24 +417,8 @@ __device__ __forceinline__ void bstore_val2(__amdgpu_buffer_rsrc_t r, int off, c
 // arrived, and it counts as produced here rather than by its load.
 __device__ __forceinline__ void pin_reg(int& v) { __asm__ __volatile__("" : "+v"(v)); }
 
-// Factor entries of the ring kernel.  A row takes four lanes, a lane five
-// entries: entry j of the row is entry j / 4 of lane j % 4.  A lane's record is
-// its five values and five 16-bit ring slots, cut into pieces of at most 16
-// bytes:
-//   4-byte values   [v0 v1 v2 v3] [v4 s01 s23 s4]
-//   8-byte values   [v0 v1] [v2 v3] [v4 s01 s23] [s4]
-//   16-byte values  [v0] [v1] [v2] [v3] [v4] [s01 s23 s4 -]
-// (s01: slots 0 and 1 in one word).  The rows of a step are cut into groups of
-// 16 (the rows of one wave); a group of n rows at position p starts at byte
-// p * ring_row_bytes<V>() of its block and holds piece 0 of its 4 n lanes, then
-// piece 1, ...: every copy of a wave is one contiguous run of memory at a
-// wave-uniform base, and lands in LDS as the solving lanes read it.
-template <typename V>
-__host__ __device__ constexpr int ring_row_bytes() {
-  return 4 * (5 * (int)sizeof(V) + (sizeof(V) == 16 ? 16 : 12));
-}
-constexpr int kRingGroup = 16;  // rows of a group
-
+// The records of the factor entries are laid out by ring_pack.hpp: a lane's five
+// values and five ring slots, in pieces.
 template <typename V>
 struct LaneRec {
   V val[5];
@@ -441,32 +427,6 @@ struct LaneRec {
 
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-
-// Writes (on the host) entry j of row t of the group of n rows
-// whose bytes start at g.
-template <typename V>
-inline void store_rec(unsigned char* g, int n, int t, int j, const V& v, unsigned slot) {
-  const int lane = 4 * t + j % 4, e = j / 4;
-  auto put = [](unsigned char* q, const void* x, int b) { __builtin_memcpy(q, x, (size_t)b); };
-  const uint16_t s16 = (uint16_t)slot;
-  unsigned char* sl;  // the word of slots 0 and 1; slot 4's word
-  unsigned char* s4;
-  if constexpr (sizeof(V) == 4) {
-    unsigned char* b = g + n * 64 + lane * 16;
-    put(e < 4 ? g + lane * 16 + e * 4 : b, &v, 4);
-    sl = b + 4;
-    s4 = b + 12;
-  } else if constexpr (sizeof(V) == 8) {
-    put(g + (e / 2) * n * 64 + lane * 16 + (e % 2) * 8, &v, 8);
-    sl = g + n * 128 + lane * 16 + 8;
-    s4 = g + n * 192 + lane * 4;
-  } else {
-    put(g + e * n * 64 + lane * 16, &v, 16);
-    sl = g + n * 320 + lane * 16;
-    s4 = sl + 8;
-  }
-  put(e < 4 ? sl + 2 * e : s4, &s16, 2);
-}
 
 // LDS byte address of a ring row: base + slot * RS with the slot in the low or
 // high half of w, one instruction.
@@ -625,10 +585,6 @@ __device__ __forceinline__ void ring_copy_sweep(int nsteps, const int* pos, int 
   // the workgroup ends
   __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory");
 }
-
-// The row id of the dummy row: shifted by 2 to 10 bits it is a byte offset past
-// every resource.
-constexpr int kRingDummyRow = 0x3fe00000;
 
 // Sweep of the wave that moves the right-hand sides, as ring_copy_sweep the
 // records; the row ids that their addresses need are loaded K steps before them.
@@ -887,7 +843,7 @@ template <typename V, int K, int CG, int NG, int NH>
 __global__ __launch_bounds__(64 * (NH * NG + NH + 1)) void k_trsv_ring(
     int nblocks, int rows, const int* __restrict__ blk_row0, const int* __restrict__ blk_step,
     const int* __restrict__ blk_stepU, const int64_t* __restrict__ blk_ri0, const int* __restrict__ pos,
-    const unsigned char* __restrict__ ent, const int2* __restrict__ info, const V* __restrict__ dinv,
+    const unsigned char* __restrict__ ent, const RingInfo* __restrict__ info, const V* __restrict__ dinv,
     const V* __restrict__ rhs, V* __restrict__ x, int nrhs) {
   extern __shared__ unsigned char smem_raw[];
   const int b = blockIdx.x % nblocks;

@@ -1,23 +1,30 @@
-// Host replay of the ring solve's LDS slots.
+// Host replay of the ring solve from the arrays that the upload sends.
 //
-// The ring kernel keeps the value of the row at position p (all L rows of a
-// block in storage order, then all U rows) in slot p % rows of its ring, rows =
-// TrsvPack::window_needed.  Nothing orders the writes of one step: two waves
-// take its rows, and the lanes of a wave write together.  So a step's writes
-// are replayed in both row orders, each step's reads before its writes and
-// (for a wave that is ahead) after the other rows' writes, and every replay must
-// give the plain forward/backward substitution on the block's factors.
+// Every level of a set-up operator is packed as the upload packs it (ring_pack)
+// and solved from those arrays alone, as the ring kernel does: a group of 16
+// rows' records copied to a stage piece by piece, lanes' entries and ring slots
+// read from it, a row's own slot and id from its info pair, steps from their
+// boundaries (whole and half steps), the value of the row at position p in slot
+// p % rows of a ring that holds just the rows the packing asks for.  Nothing orders the
+// writes of one step: two waves take its rows, and the lanes of a wave write
+// together.  So a step's rows are replayed in both orders, with the reads
+// before the writes and row by row, and every replay must give plain
+// forward/backward substitution on the block's factors.
 //
 // usage: ring_check   (exit 0 when every level of every problem agrees)
 #include <algorithm>
 #include <cmath>
 #include <complex>
+#include <cstdint>
 #include <cstdio>
+#include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../pargemslr_amd/csrc/host/gemslr_host.hpp"
 #include "../../pargemslr_amd/csrc/host/gen.hpp"
+#include "../../pargemslr_amd/csrc/host/ring_pack.hpp"
 #include "../../pargemslr_amd/csrc/host/trsv_pack.hpp"
 
 using namespace pgs;
@@ -25,8 +32,10 @@ using namespace pgs;
 namespace {
 
 constexpr int kStepRows = 32;
-constexpr int kSlabWidth = 20;
 constexpr int kMaxWindow = 8192;
+
+template <typename V>
+constexpr bool is_single = std::is_same<V, float>::value || std::is_same<V, std::complex<float>>::value;
 
 template <typename T>
 T value_of(double re, double im) {
@@ -57,34 +66,66 @@ struct Order {
   bool reversed, row_by_row;
 };
 
-template <typename T>
-void ring_solve(const TrsvPack<T>& P, const std::vector<int>& desc, int sbeg, int sU, int send, int b, const T* rhs,
-                T* x, int rows, Order o) {
-  std::vector<T> ring(rows, T(0.0));
-  const int64_t e0 = P.blk_ent0[b], q0 = P.blk_ri0[b];
-  for (int s = sbeg; s < send; ++s) {
-    const bool upper = s >= sU;
-    const int ro = desc[4 * s], eo = desc[4 * s + 1], nr = desc[4 * s + 2], w = desc[4 * s + 3];
-    const int end = ro + nr;
-    std::vector<T> v(nr);
+// The lanes' view of a group's records: copied to a stage as the copying wave
+// does (piece i of 4 n lanes from byte i * 64 n of the group to byte i * 1024 of
+// the stage), read as a solving lane does.
+template <typename V>
+struct Stage {
+  std::vector<unsigned char> bytes = std::vector<unsigned char>(16 * ring_row_bytes<V>(), 0);
+  Stage(const unsigned char* group, int n) {
+    constexpr int full = sizeof(V) == 4 ? 2 : sizeof(V) == 8 ? 3 : 6;  // pieces of 16 bytes a lane
+    for (int i = 0; i < full; ++i) std::memcpy(&bytes[i * 1024], group + i * 64 * n, 64 * n);
+    if (sizeof(V) == 8) std::memcpy(&bytes[3 * 1024], group + 3 * 64 * n, 16 * n);
+  }
+  template <typename X>
+  X get(int at) const {
+    X x;
+    std::memcpy(&x, &bytes[at], sizeof(X));
+    return x;
+  }
+  V value(int lane, int e) const {
+    if (sizeof(V) == 4) return get<V>(e < 4 ? lane * 16 + 4 * e : 1024 + lane * 16);
+    if (sizeof(V) == 8) return get<V>((e / 2) * 1024 + lane * 16 + (e % 2) * 8);
+    return get<V>(e * 1024 + lane * 16);
+  }
+  int slot(int lane, int e) const {
+    const int s01 = sizeof(V) == 4 ? 1024 + lane * 16 + 4 : sizeof(V) == 8 ? 2048 + lane * 16 + 8 : 5 * 1024 + lane * 16;
+    const int s4 = sizeof(V) == 8 ? 3 * 1024 + lane * 4 : s01 + 8;
+    return e < 4 ? get<uint16_t>(s01 + 2 * e) : (int)(get<uint32_t>(s4) & 0xffff);
+  }
+};
+
+// One block: pos its step boundaries, nL of its nsteps steps in the L sweep, q0
+// its first position.
+template <typename V, typename T>
+void ring_solve(const RingPack<V>& R, const int* pos, int nL, int nsteps, int64_t q0, const T* dinv, const T* rhs,
+                T* x, Order o) {
+  std::vector<T> ring(R.rows, T(0.0));
+  for (int s = 0; s < nsteps; ++s) {
+    const bool upper = s >= nL;
+    const int p0 = pos[s], n = pos[s + 1] - p0;
+    std::vector<Stage<V>> st;
+    for (int g = 0; g < n; g += 16)
+      st.emplace_back(R.rec.data() + (q0 + p0 + g) * ring_row_bytes<V>(), std::min(16, n - g));
+    std::vector<T> v(n);
     auto solve = [&](int t) {
-      const int row = P.rows[q0 + ro + t];
       T acc = T(0.0);
-      for (int j = 0; j < w; ++j) {
-        const int64_t e = e0 + eo + (int64_t)t * w + j;
-        if (P.val[e] == T(0.0)) continue;  // padding
-        const int p = end - 1 - ((end - 1 - P.col[e]) & (P.window - 1));
-        acc += P.val[e] * ring[p % rows];
-      }
+      for (int q = 0; q < 4; ++q)
+        for (int e = 0; e < 5; ++e) {
+          const int lane = 4 * (t % 16) + q;
+          acc += T(st[t / 16].value(lane, e)) * ring[st[t / 16].slot(lane, e)];
+        }
+      const int row = R.info[q0 + p0 + t].row;
       v[t] = (upper ? x[row] : rhs[row]) - acc;
-      if (upper) v[t] *= P.dinv[q0 + ro + t];
+      if (upper) v[t] *= dinv[q0 + p0 + t];
     };
     auto write = [&](int t) {
-      ring[(ro + t) % rows] = v[t];
-      x[P.rows[q0 + ro + t]] = v[t];
+      const RingInfo i = R.info[q0 + p0 + t];
+      ring.at(i.slot / sizeof(V)) = v[t];
+      x[i.row] = v[t];
     };
     auto each = [&](auto f) {
-      for (int t = 0; t < nr; ++t) f(o.reversed ? nr - 1 - t : t);
+      for (int t = 0; t < n; ++t) f(o.reversed ? n - 1 - t : t);
     };
     if (o.row_by_row) {
       each([&](int t) {
@@ -98,19 +139,25 @@ void ring_solve(const TrsvPack<T>& P, const std::vector<int>& desc, int sbeg, in
   }
 }
 
-// Replays every level; `shorter` takes rows off the ring (a control).
-template <typename T>
+// Replays every level with the device's values in V; `shorter` takes rows off
+// the ring (a control).
+template <typename V, typename T>
 bool check_op(const std::string& name, const HostOp<T>& op, int shorter) {
   bool ok = true;
+  const double tol = is_single<V> ? 1e-5 : 1e-12;
   for (int l = 0; l < op.nlev; ++l) {
     const HostLevel<T>& L = op.levels[l];
     const int nl = op.nloc(l);
-    TrsvPack<T> P = trsv_pack(L, op.lev_ptr[l], nl, kStepRows, kMaxWindow, kSlabWidth);
-    std::vector<int> dh, sh, suh;
-    half_steps(P.desc, P.blk_step, P.blk_stepU, dh, sh, suh);
+    TrsvPack<T> P = trsv_pack(L, op.lev_ptr[l], nl, kStepRows, kMaxWindow, kRingWidth);
+    if (P.window == 0) {
+      std::printf("%s level %d: not ring-packed MISMATCH\n", name.c_str(), l);
+      ok = false;
+      continue;
+    }
+    P.window_needed -= shorter;
+    const RingPack<V> R = ring_pack<V>(P, [](const T& v) { return V(v); });
     int longest = 0;
     for (size_t i = 2; i < P.desc.size(); i += 4) longest = std::max(longest, P.desc[i]);
-    const int rows = std::max(1, P.window_needed - shorter);
     std::vector<double> g(2 * (size_t)nl);
     rng_normal(1000 + l, 2 * (int64_t)nl, g.data());
     std::vector<T> rhs(nl), ref(nl), x(nl);
@@ -121,11 +168,11 @@ bool check_op(const std::string& name, const HostOp<T>& op, int shorter) {
       block_solve(L.ilu[b], rhs.data() + r0, ref.data() + r0);
       for (int k = 0; k < 8; ++k) {
         const Order o = {(k & 1) != 0, (k & 2) != 0};
-        if (k & 4)
-          ring_solve(P, P.desc, P.blk_step[b], P.blk_stepU[b], P.blk_step[b + 1], b, rhs.data() + r0, x.data() + r0,
-                     rows, o);
-        else
-          ring_solve(P, dh, sh[b], suh[b], sh[b + 1], b, rhs.data() + r0, x.data() + r0, rows, o);
+        const bool half = (k & 4) != 0;
+        const int s0 = half ? R.step_h[b] : P.blk_step[b], s1 = half ? R.step_h[b + 1] : P.blk_step[b + 1];
+        const int sU = half ? R.stepU_h[b] : P.blk_stepU[b];
+        ring_solve<V>(R, (half ? R.pos_h : R.pos).data() + s0 + b, sU - s0, s1 - s0, P.blk_ri0[b],
+                      P.dinv.data(), rhs.data() + r0, x.data() + r0, o);
         for (int i = r0; i < r0 + nb; ++i) {
           nmax = std::max(nmax, std::abs(ref[i]));
           const double e = std::abs(x[i] - ref[i]);
@@ -134,9 +181,10 @@ bool check_op(const std::string& name, const HostOp<T>& op, int shorter) {
       }
     }
     const double rel = nmax > 0.0 ? emax / nmax : emax;
-    const bool good = P.window > 0 && rel <= 1e-12;
-    std::printf("%s level %d: %d blocks, longest step %d rows, ring %d rows%s, rel err %.2e %s\n", name.c_str(), l,
-                L.ncomp, longest, rows, shorter ? " (shortened)" : "", rel, good ? "ok" : "MISMATCH");
+    const bool good = rel <= tol;
+    std::printf("%s, %d-byte values, level %d: %d blocks, longest step %d rows, ring %d rows%s, rel err %.2e %s\n",
+                name.c_str(), (int)sizeof(V), l, L.ncomp, longest, R.rows, shorter ? " (shortened)" : "", rel,
+                good ? "ok" : "MISMATCH");
     ok = ok && good;
   }
   return ok;
@@ -159,7 +207,10 @@ bool run(const std::string& name, const Csr<T>& A, int nlev, int ncomp, double d
     std::printf("%s: setup failed: %s\n", name.c_str(), msg.c_str());
     return false;
   }
-  return check_op(name, op, shorter);
+  bool ok = check_op<T>(name, op, shorter);
+  if constexpr (is_complex<T>::value) ok = check_op<std::complex<float>>(name, op, shorter) && ok;
+  else ok = check_op<float>(name, op, shorter) && ok;
+  return ok;
 }
 
 // n rows: the diagonal, and entries of the last row in the given columns (upper:

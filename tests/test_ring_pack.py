@@ -1,7 +1,7 @@
-"""The ring solve's slots, replayed on the host (tests/cpp/ring_check.cpp, built
-with the library): a step's rows written in either order, ahead of or after the
-other rows' reads, give plain substitution; a ring that is too short does not.
-CPU only."""
+"""The ring solve replayed on the host from the arrays that the upload sends
+(tests/cpp/ring_check.cpp, built with the library): a step's rows written in
+either order, ahead of or after the other rows' reads, give plain substitution; a
+ring that is too short does not.  CPU only."""
 import os
 import subprocess
 
