@@ -148,7 +148,6 @@ struct DevTrsv {
   // ring-packed levels: step boundaries, lane records, (slot, row id) pairs and
   // 1/pivots by position (RingPack)
   DevMem pos, rec, info, dinv;
-  int64_t positions = 0;
   // half steps: a step of more than 16 rows walked as two consecutive ones (rows
   // 0-15, then 16-31).  Rows of a step are independent, and a half step reads
   // and writes a subset of its step's positions, so the window still holds.
@@ -169,11 +168,9 @@ void upload_trsv(DevTrsv& d, const TrsvPack<T>& P, int64_t* counter) {
   upload(d.step, P.blk_step, counter);
   upload(d.stepU, P.blk_stepU, counter);
   upload(d.ri0, P.blk_ri0, counter);
-  const int64_t nr = (int64_t)P.rows.size();
   if (P.window > 0) {
     const RingPack<V> R = ring_pack<V>(P, [](const T& v) { return hval<V>(v); });
     d.window = R.rows;
-    d.positions = nr;
     d.max_block_steps = R.max_block_steps;
     d.max_block_steps_h = R.max_block_steps_h;
     upload(d.pos, R.pos, counter);
@@ -189,7 +186,7 @@ void upload_trsv(DevTrsv& d, const TrsvPack<T>& P, int64_t* counter) {
   upload(d.desc, P.desc, counter);
   std::vector<TPair<V>> ent(P.col.size() + 1), ri(P.rows.size() + 1);
   constexpr int64_t kChunk = 1 << 20;
-  const int64_t ne = (int64_t)P.col.size();
+  const int64_t ne = (int64_t)P.col.size(), nr = (int64_t)P.rows.size();
   parallel_for((int)((ne + kChunk - 1) / kChunk), [&](int c) {
     for (int64_t i = c * kChunk, i1 = std::min(ne, (c + 1) * kChunk); i < i1; ++i) {
       ent[i] = TPair<V>();
@@ -487,14 +484,7 @@ void launch_trsv_ring_k(const DevTrsv& T, const V* rhs, V* x, int nrhs, hipStrea
 
 template <typename V>
 void launch_trsv_ring(pgs_dev_op_s* op, const DevTrsv& T, const V* rhs, V* x, int nrhs, hipStream_t s) {
-  // the kernel addresses a block's rows of all columns, its records (two
-  // positions per row) and its step boundaries with 32-bit byte offsets; lanes
-  // with nothing to load or store aim at offset kRingOut, which must stay past
-  // each of them
-  if ((int64_t)T.max_rows * nrhs * (int64_t)sizeof(V) > (int64_t)kRingOut ||
-      2 * (int64_t)T.max_rows * ring_row_bytes<V>() > (int64_t)kRingOut || (T.positions + 1) * 8 > (int64_t)kRingOut ||
-      (T.max_block_steps + 64) * 4 > (int64_t)kRingOut)
-    throw std::runtime_error("diagonal block too large for 32-bit offsets");
+  if (!ring_offsets_fit<V>(T.max_rows, nrhs)) throw std::runtime_error("diagonal block too large for 32-bit offsets");
   if (nrhs <= 0 || (nrhs & (nrhs - 1)) != 0)
     throw std::runtime_error("the ring solve takes a power-of-two number of columns");
   constexpr int CMAX = sizeof(V) == 4 ? 16 : sizeof(V) == 8 ? 8 : 4;

@@ -450,8 +450,6 @@ __device__ __forceinline__ void lds_write(unsigned addr, const T& v) {
   }
 }
 
-constexpr int kRingOut = 0x7ffffff0;  // a byte offset past every resource of the ring kernel
-
 // Pieces of a lane's record: loads (and direct-to-LDS copies) per wave and step.
 template <typename V>
 constexpr int ring_pieces() {
@@ -836,8 +834,8 @@ __device__ __forceinline__ void ring_solve_sweep(int h, int g, int nsteps, int r
 // pos: per block b the boundaries of its steps (blk_step[b + 1] - blk_step[b] + 1
 // values from blk_step[b] + b; the first of them is 0, sU's the block's
 // rows).  info, dinv: per position the pair (ring slot times sizeof(V),
-// block-local row id) and 1/pivot, from blk_ri0[b], and the dummy row's pair
-// after the last block's; ent: the block's records, from blk_ri0[b] *
+// block-local row id) from blk_ri0[b] + b, the dummy row's pair after the block's
+// own, and 1/pivot from blk_ri0[b]; ent: the block's records, from blk_ri0[b] *
 // ring_row_bytes<V>().
 template <typename V, int K, int CG, int NG, int NH>
 __global__ __launch_bounds__(64 * (NH * NG + NH + 1)) void k_trsv_ring(
@@ -850,12 +848,12 @@ __global__ __launch_bounds__(64 * (NH * NG + NH + 1)) void k_trsv_ring(
   const int c0 = (blockIdx.x / nblocks) * CG * NG;
   const int r0 = blk_row0[b], nb = blk_row0[b + 1] - r0;
   const int sbeg = blk_step[b], send = blk_step[b + 1], sU = blk_stepU[b];
-  const int64_t q0 = blk_ri0[b], np = blk_ri0[b + 1] - q0, nd = blk_ri0[nblocks] - q0;
+  const int64_t q0 = blk_ri0[b], np = blk_ri0[b + 1] - q0;
   const int* pb = pos + sbeg + b;
   const int64_t vbytes = (int64_t)nb * nrhs * (int64_t)sizeof(V);
   V* xb = x + (int64_t)r0 * nrhs;
   const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(xb, vbytes);
-  const __amdgpu_buffer_rsrc_t rs_info = make_rsrc(info + q0, (nd + 1) * 8);
+  const __amdgpu_buffer_rsrc_t rs_info = make_rsrc(info + q0 + b, (np + 1) * 8);
   // rings, dummy rows and stages start as zeros: a record that is not there reads
   // slot 0 with weight zero
   uint4* lds4 = reinterpret_cast<uint4*>(smem_raw);
@@ -873,7 +871,7 @@ __global__ __launch_bounds__(64 * (NH * NG + NH + 1)) void k_trsv_ring(
   } else if (w < NH * NG + NH) {
     const __amdgpu_buffer_rsrc_t rs_ent = make_rsrc(ent + q0 * ring_row_bytes<V>(), np * ring_row_bytes<V>());
     const __amdgpu_buffer_rsrc_t rs_dinv = make_rsrc(dinv + q0, np * (int64_t)sizeof(V));
-    const int dummy = (int)(nd * 8);
+    const int dummy = (int)(np * 8);
     auto copies = [&](auto hc) {
       constexpr int HC = decltype(hc)::value;
       ring_copy_sweep<V, K, CG, NG, NH, HC, false>(sU - sbeg, pb, rows, dummy, rs_ent, rs_info, rs_dinv);

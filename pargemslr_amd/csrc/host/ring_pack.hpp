@@ -37,6 +37,17 @@ constexpr int ring_row_bytes() {
   return 4 * (5 * (int)sizeof(V) + (sizeof(V) == 16 ? 16 : 12));
 }
 
+constexpr int kRingOut = 0x7ffffff0;  // a byte offset past every resource of the ring kernel
+
+// The ring kernel addresses a block's rows of all columns, its records (two
+// positions per row) and, both shorter, its pairs and step boundaries with 32-bit
+// byte offsets; lanes with nothing to load or store aim at offset kRingOut, which
+// must stay past each of them.  A level may hold any number of such blocks.
+template <typename V>
+constexpr bool ring_offsets_fit(int64_t max_block_rows, int nrhs) {
+  return max_block_rows * nrhs * (int64_t)sizeof(V) <= kRingOut && 2 * max_block_rows * ring_row_bytes<V>() <= kRingOut;
+}
+
 // The row id of the dummy row: shifted by 2 to 10 bits it is a byte offset past
 // every resource.
 constexpr int kRingDummyRow = 0x3fe00000;
@@ -78,7 +89,7 @@ struct RingPack {
   std::vector<int> pos_h, step_h, stepU_h;
   int64_t max_block_steps = 0, max_block_steps_h = 0;
   std::vector<unsigned char> rec;       // records, ring_row_bytes<V>() per position
-  std::vector<RingInfo> info;           // per position, and the dummy row's after the last
+  std::vector<RingInfo> info;           // per position, and the dummy row's after a block's last
 };
 
 // Step boundaries of every block from the step descriptors (4 per step, the
@@ -119,15 +130,15 @@ RingPack<V> ring_pack(const TrsvPack<T>& P, F val) {
   constexpr int RB = ring_row_bytes<V>();
   const int64_t nr = (int64_t)P.rows.size();
   R.rec.resize((size_t)nr * RB);
-  R.info.resize((size_t)nr + 1);
-  R.info[nr] = RingInfo{wn * (int)sizeof(V), kRingDummyRow};
+  R.info.resize((size_t)nr + P.nblocks);
   parallel_for(P.nblocks, [&](int b) {
+    R.info[P.blk_ri0[b + 1] + b] = RingInfo{wn * (int)sizeof(V), kRingDummyRow};
     for (int s = P.blk_step[b]; s < P.blk_step[b + 1]; ++s) {
       const int* d4 = &P.desc[4 * (size_t)s];
       const int end = d4[0] + d4[2];  // a row the step reads is at most W positions before it
       for (int t = 0; t < d4[2]; ++t) {
         const int64_t q = P.blk_ri0[b] + d4[0] + t;
-        R.info[q] = RingInfo{(d4[0] + t) % wn * (int)sizeof(V), P.rows[q]};
+        R.info[q + b] = RingInfo{(d4[0] + t) % wn * (int)sizeof(V), P.rows[q]};
         const int t0 = t / kRingGroup * kRingGroup;  // first row of t's group
         unsigned char* g = R.rec.data() + (P.blk_ri0[b] + d4[0] + t0) * RB;
         for (int j = 0; j < d4[3]; ++j) {

@@ -98,8 +98,8 @@ struct Stage {
 // One block: pos its step boundaries, nL of its nsteps steps in the L sweep, q0
 // its first position.
 template <typename V, typename T>
-void ring_solve(const RingPack<V>& R, const int* pos, int nL, int nsteps, int64_t q0, const T* dinv, const T* rhs,
-                T* x, Order o) {
+void ring_solve(const RingPack<V>& R, const int* pos, int nL, int nsteps, int64_t q0, const RingInfo* info,
+                const T* dinv, const T* rhs, T* x, Order o) {
   std::vector<T> ring(R.rows, T(0.0));
   for (int s = 0; s < nsteps; ++s) {
     const bool upper = s >= nL;
@@ -115,12 +115,12 @@ void ring_solve(const RingPack<V>& R, const int* pos, int nL, int nsteps, int64_
           const int lane = 4 * (t % 16) + q;
           acc += T(st[t / 16].value(lane, e)) * ring[st[t / 16].slot(lane, e)];
         }
-      const int row = R.info[q0 + p0 + t].row;
+      const int row = info[p0 + t].row;
       v[t] = (upper ? x[row] : rhs[row]) - acc;
       if (upper) v[t] *= dinv[q0 + p0 + t];
     };
     auto write = [&](int t) {
-      const RingInfo i = R.info[q0 + p0 + t];
+      const RingInfo i = info[p0 + t];
       ring.at(i.slot / sizeof(V)) = v[t];
       x[i.row] = v[t];
     };
@@ -166,12 +166,19 @@ bool check_op(const std::string& name, const HostOp<T>& op, int shorter) {
     for (int b = 0; b < L.ncomp; ++b) {
       const int r0 = P.blk_row0[b], nb = P.blk_row0[b + 1] - r0;
       block_solve(L.ilu[b], rhs.data() + r0, ref.data() + r0);
+      // lanes past a step's rows take the dummy row's pair, right after the block's own
+      const int64_t np = P.blk_ri0[b + 1] - P.blk_ri0[b];
+      const RingInfo* info = R.info.data() + P.blk_ri0[b] + b;
+      if (info[np].slot != R.rows * (int)sizeof(V) || info[np].row != kRingDummyRow) {
+        std::printf("%s, level %d, block %d: no dummy pair MISMATCH\n", name.c_str(), l, b);
+        ok = false;
+      }
       for (int k = 0; k < 8; ++k) {
         const Order o = {(k & 1) != 0, (k & 2) != 0};
         const bool half = (k & 4) != 0;
         const int s0 = half ? R.step_h[b] : P.blk_step[b], s1 = half ? R.step_h[b + 1] : P.blk_step[b + 1];
         const int sU = half ? R.stepU_h[b] : P.blk_stepU[b];
-        ring_solve<V>(R, (half ? R.pos_h : R.pos).data() + s0 + b, sU - s0, s1 - s0, P.blk_ri0[b],
+        ring_solve<V>(R, (half ? R.pos_h : R.pos).data() + s0 + b, sU - s0, s1 - s0, P.blk_ri0[b], info,
                       P.dinv.data(), rhs.data() + r0, x.data() + r0, o);
         for (int i = r0; i < r0 + nb; ++i) {
           nmax = std::max(nmax, std::abs(ref[i]));
@@ -260,6 +267,12 @@ int main() {
   ok = run("convdiff 20^3", convdiff_upwind(20, 20, 20, 0.3), 2, 4, 1e-2, 10) && ok;
   ok = run("complex laplacian 16^3", laplacian<zdouble>(16, 16, 16, zdouble(0.2, 0.02), 0.05, -0.02, 0.01), 3, 4, 1e-3,
            20) && ok;
+  // limits of the 32-bit offsets are a block's, whatever its level holds: the
+  // largest blocks (FP32, FP64, complex128) and one row more, a block's vectors
+  ok = ring_offsets_fit<float>(8388607, 64) && !ring_offsets_fit<float>(8388608, 1) && ok;
+  ok = ring_offsets_fit<double>(5162220, 32) && !ring_offsets_fit<double>(5162221, 1) && ok;
+  ok = ring_offsets_fit<zdouble>(2796202, 32) && !ring_offsets_fit<zdouble>(2796203, 1) && ok;
+  ok = ring_offsets_fit<double>(4194303, 64) && !ring_offsets_fit<double>(4194304, 64) && ok;
   // controls: a ring one row too short must break the replay
   const bool c1 = run("control 24^3", laplacian<double>(24, 24, 24, 0.0, 0.0, 0.0, 0.0), 3, 8, 1e-3, 20, true, 1);
   const bool c2 = run("control one long row", one_long_row(33, {13, 31}, false), 1, 1, 1e-6, 20, false, 13);
