@@ -54,7 +54,8 @@ def build(verbose=False):
     san_dir = os.path.join(OBJ, "san")
     os.makedirs(san_dir, exist_ok=True)
     san_objs, san_main = [], {}
-    for s in SAN_SRC + ["../../tests/cpp/pack_check.cpp", "../../tests/cpp/ring_check.cpp"]:
+    for s in SAN_SRC + ["../../tests/cpp/pack_check.cpp", "../../tests/cpp/ring_check.cpp",
+                        "../../tests/cpp/sweep_check.cpp"]:
         o = os.path.join(san_dir, os.path.basename(s) + ".o")
         if s in SAN_SRC:
             san_objs.append(o)
@@ -77,7 +78,8 @@ def build(verbose=False):
     _run(["g++"] + SAN_FLAGS + [os.path.join(cpp, "parallel_for_check.cpp"), "-o",
                                 os.path.join(cpp, "parallel_for_check_san")])
     # C++ driver on the class surface (include/pargemslr_amd.hpp), run by the tests
-    for name in ("driver_laplacian", "driver_gen", "driver_surface", "pack_check", "ring_check"):
+    for name in ("driver_laplacian", "driver_gen", "driver_surface", "pack_check", "ring_check",
+                 "sweep_check"):
         drv_src = os.path.join(root, "tests", "cpp", name + ".cpp")
         if os.path.exists(drv_src):
             drv = os.path.join(root, "tests", "cpp", name)

@@ -15,6 +15,7 @@
 #include "../../../include/pargemslr_amd.h"
 #include "../host/gemslr_host.hpp"
 #include "../host/ring_pack.hpp"
+#include "../host/sweep_blocks.hpp"
 #include "../host/trsv_pack.hpp"
 #include "capi_internal.hpp"
 #include "kernels.hpp"
@@ -999,10 +1000,6 @@ struct WsSizes {
 // multi-dots and norms use (level temporaries, partial sums, the low-rank
 // term's partials); no Krylov bases, Hessenberg state or inner-iteration
 // buffers.
-// partial sums per workgroup and column: kdim + 1 dots, or the 2 p + 2 of a
-// delayed-CGS2 step (66: the norms of an update by up to 4096 workgroups)
-size_t part_rows(int kdim) { return (size_t)std::max(2 * kdim + 2, 66); }
-
 WsSizes ws_sizes(const pgs_dev_op_s* op, int nr, int kdim, bool lowrank_build = false) {
   WsSizes z;
   const int64_t n = op->n;
@@ -1016,16 +1013,13 @@ WsSizes ws_sizes(const pgs_dev_op_s* op, int nr, int kdim, bool lowrank_build = 
                      : op->pz64.present ? op->pz64.levels : op->pz32.levels;
     maxrank = std::max(maxrank, lv[l]->rank);
   }
-  // dot products use at most 1024 workgroups (four per CU); the partials
-  // are summed by one wave per output
-  const int64_t rows_per_blk = std::max<int64_t>(256, (n + 1023) / 1024);
-  z.part_blocks = (int)std::max<int64_t>(1, (n + rows_per_blk - 1) / rows_per_blk);
+  z.part_blocks = (int)part_blocks(n);
   const size_t ik = (size_t)kdim;
   auto add = [&](DevMem pgs_ws_s::*m, size_t b) { z.bufs.push_back({m, b}); };
   if (lowrank_build) {
     add(&pgs_ws_s::lrpart, (size_t)std::max(1, (kLrBlocks + 1) * maxrank * nr) * es);
     add(&pgs_ws_s::lrt, (size_t)std::max(1, maxrank * nr) * es);
-    add(&pgs_ws_s::part, (size_t)z.part_blocks * part_rows(kdim) * nr * es);
+    add(&pgs_ws_s::part, (size_t)(z.part_blocks * part_rows(kdim)) * nr * es);
     return z;
   }
   add(&pgs_ws_s::r0, vb);
@@ -1034,7 +1028,7 @@ WsSizes ws_sizes(const pgs_dev_op_s* op, int nr, int kdim, bool lowrank_build = 
   add(&pgs_ws_s::lrt, (size_t)std::max(1, maxrank * nr) * es);
   add(&pgs_ws_s::V, (ik + 1) * (vb + kBasisPad * es));
   add(&pgs_ws_s::Z, ik * (vb + kBasisPad * es));
-  add(&pgs_ws_s::part, (size_t)z.part_blocks * part_rows(kdim) * nr * es);
+  add(&pgs_ws_s::part, (size_t)(z.part_blocks * part_rows(kdim)) * nr * es);
   add(&pgs_ws_s::hbuf, (ik + 1) * nr * es);
   add(&pgs_ws_s::h2buf, (ik + 1) * nr * es);
   add(&pgs_ws_s::H, (size_t)nr * (ik + 1) * ik * es);
@@ -1369,6 +1363,13 @@ struct PrecTypes<cplx<double>> {
   using P32 = cplx<float>;
 };
 
+// sweep_blocks for a sweep that leaves `rows` values per workgroup and column in ws->part
+template <typename S>
+int part_sweep(const pgs_ws_s* ws, int64_t want, int nrhs, int rows, int most) {
+  const int64_t fit = (int64_t)(ws->part.bytes / (sizeof(S) * (size_t)rows * nrhs));
+  return (int)sweep_blocks(ws->part_blocks, want, fit, most);
+}
+
 // FGMRES (FlexGmresClass::Solve, fgmres.hpp:300-540) on nrhs columns at once:
 // Krylov scalar S (double or complex<double>), preconditioned basis Z in VZ.
 // Delayed CGS2, dots of step p: the table [s (p rows) | a (p rows) | q.q | q.w]
@@ -1385,13 +1386,12 @@ int dcgs2_dots(pgs_ws_s* ws, int64_t n, int nrhs, int p, const S* V, int64_t ldv
                hipStream_t s) {
   const S* q = V + (int64_t)p * ldv;
   constexpr int E = 16 / (int)sizeof(S);
-  const int64_t nthr = (n * nrhs + kWave * E - 1) / (kWave * E);
-  const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(ws->part_blocks, nthr));
+  const int nout = w != nullptr ? 2 * p + 2 : p + 1;
+  const int nblk = part_sweep<S>(ws, (n * nrhs + kWave * E - 1) / (kWave * E), nrhs, nout, kDotsPieces);
   // equal chunks: a short last one would leave too few loads in flight
   const int nch = std::max(1, (p + kDotsChunk - 1) / kDotsChunk);
   const int chunk = (p + nch - 1) / nch;
   const dim3 grid(nblk, nch);
-  const int nout = w != nullptr ? 2 * p + 2 : p + 1;
   S* part = ws->part.as<S>();
   if (E == 2 && nrhs == 1) k_dcgs2_dots<S, E == 2><<<grid, kDotsNT, 0, s>>>(n, nrhs, p, chunk, V, ldv, q, w, part);
   else k_dcgs2_dots<S, false><<<grid, kDotsNT, 0, s>>>(n, nrhs, p, chunk, V, ldv, q, w, part);
@@ -1543,8 +1543,7 @@ int fgmres_impl(pgs_dev_op_s* op, pgs_ws_s* ws, const S* b, S* x, int nrhs, cons
       // places in turn, the norm's to the first
       const double vb = (double)n * nrhs * sizeof(S);
       constexpr int E = 16 / (int)sizeof(S);
-      const int64_t want = (n * nrhs + kMgsNT * E - 1) / (kMgsNT * E);
-      nblk = (int)std::max<int64_t>(1, std::min<int64_t>(ws->part_blocks, want));
+      nblk = part_sweep<S>(ws, (n * nrhs + kMgsNT * E - 1) / (kMgsNT * E), nrhs, 2, kMgsPieces);
       S* part = ws->part.as<S>();
       const S* prev = nullptr;
       int nprev = 0;

@@ -869,8 +869,18 @@ __device__ __forceinline__ f64x2 stream16(const void* x) {  // as ld_stream
 // were read before).  Tried: 128 threads (4.69 ms, 375 us), 512 with 4 or 8
 // vectors per wave (5.3 and 4.8 ms, 410 us), 4 KB of a vector per workgroup
 // (4.75 ms, 419 us).
+// A workgroup walks at most kDotsPieces pieces of 64 lanes where the partials'
+// buffer holds more workgroups than one per 256 rows (sweep_blocks): with those
+// alone a wide batch of few rows ran on few workgroups, and slower than the
+// kernels before (at ten vectors, two or three loads in flight per wave).  Two
+// cycles of 10 steps, no preconditioner, 64 complex columns, ms before / with
+// one workgroup per 256 rows / now: 16^3 4.56 / 5.90 / 3.02; 28^3 6.00 / 7.31 /
+// 4.65; 64 real columns of 24^3 3.93 / 3.51 / 2.14.  16 pieces: 2 % faster at 64
+// columns, but past kFixPartials workgroups (a launch more) also at 16; 64: as
+// before at 48^3 x 16.
 constexpr int kDotsPM = 8;
 constexpr int kDotsNT = 256;
+constexpr int kDotsPieces = 32;
 constexpr int kDotsChunk = kDotsPM * (kDotsNT / kWave);
 
 template <typename S, bool ONE>
@@ -1078,9 +1088,15 @@ __global__ __launch_bounds__(NT) void k_dcgs2_update(int64_t n, int nrhs, int p,
 // one column, 11.2 -> 4.5 us per vector; 128^3, 20 steps,
 // 1 column 7.2 -> 4.8 ms, 16 columns 66 -> 54.  Every workgroup adds up all partials
 // itself, which costs less than a launch up to kMgsPartials values.
+// A workgroup takes at most kMgsPieces pieces of 256 lanes (sweep_blocks, as the
+// delayed-CGS2 dots): two cycles of 30 steps, 64 complex columns, ms as three
+// launches / with one workgroup per 256 rows / now: 16^3 30.7 / 37.0 / 12.4; 24^3
+// 47.1 / 52.4 / 20.7; 64 real columns of 24^3 33.9 / 21.5 / 12.7.  4 pieces are as
+// fast, 16 and 32 slower (24^3: 24.0 and 33.4).
 // ONE: a single real column.
 constexpr int kMgsNT = 256;
 constexpr int kMgsPartials = 4096;
+constexpr int kMgsPieces = 8;
 
 template <typename S, bool ONE>
 __global__ __launch_bounds__(kMgsNT) void k_mgs_step(int64_t n, int nrhs, int nprev, const S* __restrict__ prev,
