@@ -606,13 +606,14 @@ void set_trsv_attrs(int lds_max) {
     both(I8(), I2(), I2());
     both(I4(), I4(), I1());
   }
-  if constexpr (scalar_traits<V>::is_complex) return;  // no pipelined kernel for complex values
-  constexpr int DL2 = sizeof(V) == 4 ? 5 : 4;  // the pipelined kernel's stage depths (launch_trsv_pipe_nt)
-  constexpr int DP = sizeof(V) == 4 ? 8 : 6;
-  set_lds_limit(k_trsv_pipe<V, true, 64, 2, 10, DL2>, lds_max);
-  set_lds_limit(k_trsv_pipe<V, true, 128, 2, 10, DL2>, lds_max);
-  set_lds_limit(k_trsv_pipe<V, true, 128, 4, 5, DP>, lds_max);
-  set_lds_limit(k_trsv_pipe<V, true, 256, 4, 5, DP>, lds_max);
+  if constexpr (!scalar_traits<V>::is_complex) {  // no pipelined kernel for complex values
+    constexpr int DL2 = sizeof(V) == 4 ? 5 : 4;  // the pipelined kernel's stage depths (launch_trsv_pipe_nt)
+    constexpr int DP = sizeof(V) == 4 ? 8 : 6;
+    set_lds_limit(k_trsv_pipe<V, true, 64, 2, 10, DL2>, lds_max);
+    set_lds_limit(k_trsv_pipe<V, true, 128, 2, 10, DL2>, lds_max);
+    set_lds_limit(k_trsv_pipe<V, true, 128, 4, 5, DP>, lds_max);
+    set_lds_limit(k_trsv_pipe<V, true, 256, 4, 5, DP>, lds_max);
+  }
 }
 
 template <int PM>
@@ -1442,9 +1443,9 @@ int fgmres_impl(pgs_dev_op_s* op, pgs_ws_s* ws, const S* b, S* x, int nrhs, cons
   const int nb = nblocks_for(n * nrhs, kNT);
   const int check = o.check_every > 0 ? o.check_every : 1;
   const int maxits = o.maxits;
-  // delayed CGS2 keeps a step's coefficients in LDS and its basis values in
-  // registers: real bases up to the Krylov limit (two lanes per element past
-  // 32 vectors), complex bases up to 64 vectors (CGS2 beyond)
+  // delayed CGS2: real bases up to the Krylov limit, complex bases up to 64
+  // vectors, CGS2 beyond.  k_dcgs2_fix keeps 39 p + 35 values in LDS, which for
+  // complex ones passes 64 KB at 105 vectors
   const bool dcgs2 = o.orth == PGS_ORTH_DCGS2 && (!scalar_traits<S>::is_complex || m <= 64);
   // ||b||, v0 = b - A x, ||v0||
   colnorm2<S>(ws, n, nrhs, b, ws->nb2.as<double>(), s);

@@ -109,14 +109,10 @@ __device__ __forceinline__ To cvt(From v) { return (To)v; }
 
 // Streaming read of a basis value (non-temporal: each sweep reads a basis
 // vector once, and the basis is far larger than the caches).  At 128^3 x 64
-// the delayed-CGS2 dots went from 0.69 to 0.76 of the HBM peak and the update
-// from 0.58 to 0.59; the same loads of q and w (reused across the dot chunks)
-// and of the preconditioned basis in the solution update gained nothing.
+// the delayed-CGS2 dots, then with 8-byte loads, went from 0.69 to 0.76 of the
+// HBM peak and the update from 0.58 to 0.59; the same loads of q and w and of
+// the preconditioned basis in the solution update gained nothing.
 __device__ __forceinline__ double ld_stream(const double* p) { return __builtin_nontemporal_load(p); }
-template <typename R>
-__device__ __forceinline__ cplx<R> ld_stream(const cplx<R>* p) {
-  return cplx<R>(__builtin_nontemporal_load(&p->re), __builtin_nontemporal_load(&p->im));
-}
 
 // Row and column of element t of a row-interleaved block of nrhs columns.
 // Every entry point admits only power-of-two column counts, so a shift and a

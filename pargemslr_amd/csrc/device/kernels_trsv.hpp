@@ -87,13 +87,13 @@ struct alignas(16) TPair<double> {  // value first: a 12-byte load takes (value,
   int pad;
 };
 template <>
-struct alignas(16) TPair<cplx<float>> {  // one 12-byte load takes (value, column)
+struct alignas(16) TPair<cplx<float>> {
   cplx<float> val;
   int col;
   int pad;
 };
 template <>
-struct alignas(16) TPair<cplx<double>> {  // a 16-byte load takes the value, a 4-byte load the column
+struct alignas(16) TPair<cplx<double>> {
   cplx<double> val;
   int col;
   int pad[3];
@@ -123,21 +123,6 @@ __device__ __forceinline__ TPair<double> bload_pair(__amdgpu_buffer_rsrc_t r, in
   p.val = __hiloint2double((int)v[1], (int)v[0]);
   p.col = (int)v[2];
   p.pad = 0;
-  return p;
-}
-__device__ __forceinline__ TPair<cplx<float>> bload_pair(__amdgpu_buffer_rsrc_t r, int off, cplx<float>) {
-  auto v = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
-  TPair<cplx<float>> p;
-  p.val = cplx<float>(__uint_as_float(v[0]), __uint_as_float(v[1]));
-  p.col = (int)v[2];
-  p.pad = 0;
-  return p;
-}
-__device__ __forceinline__ TPair<cplx<double>> bload_pair(__amdgpu_buffer_rsrc_t r, int off, cplx<double>) {
-  auto v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
-  TPair<cplx<double>> p;
-  p.val = cplx<double>(__hiloint2double((int)v[1], (int)v[0]), __hiloint2double((int)v[3], (int)v[2]));
-  p.col = (int)__builtin_amdgcn_raw_buffer_load_b32(r, off + 16, 0, 0);
   return p;
 }
 // Sum over the 4 lanes of a quad with DPP quad permutations (xor 1, xor 2).
@@ -182,8 +167,6 @@ template <typename R>
 __device__ __forceinline__ cplx<R> dpp_xor2(cplx<R> v) { return cplx<R>(dpp_xor2(v.re), dpp_xor2(v.im)); }
 template <typename R>
 __device__ __forceinline__ cplx<R> quad_sum(cplx<R> v) { return cplx<R>(quad_sum(v.re), quad_sum(v.im)); }
-template <typename R>
-__device__ __forceinline__ cplx<R> pair_sum(cplx<R> v) { return cplx<R>(pair_sum(v.re), pair_sum(v.im)); }
 
 // Direct kernel: any width, nrhs columns (row-interleaved); one thread per
 // (row of the step, column), plain loads.  Used for levels whose rows are too
@@ -667,8 +650,8 @@ __device__ __forceinline__ void ring_row_sweep(int nsteps, const int* pos, int r
   __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-// Sweep of the solving waves: wave g * 2 + h of the group g of CG columns takes
-// rows 16 h .. 16 h + 15 of each step.
+// Sweep of the solving waves: wave g * NH + h of group g of CG columns takes
+// rows 16 h .. 16 h + 15 of each step (NH = 2), or all of a half step's (NH = 1).
 template <typename V, int K, int CG, int NG, int NH, bool UPPER>
 __device__ __forceinline__ void ring_solve_sweep(int h, int g, int nsteps, int rows, int nrhs, int c0,
                                                  __amdgpu_buffer_rsrc_t rs_dst) {
