@@ -408,7 +408,10 @@ __global__ void k_lr_final(int nblk, int k, int nrhs, const V* __restrict__ part
 // workgroup for itself: while the partials are few (kLrFused values) that costs
 // less than the launch that would sum them.  Stage 1 with its lane sums by lane
 // permutes and this: 48^3, one FP64 column, rank 16, 20 -> 10.1 us per term in three
-// launches -> two.  Dynamic LDS: k * nrhs values.
+// launches -> two.  An apply with one term against the same with the third launch,
+// 16^3 to 64^3, 1 to 4 columns: rank 16 up to 3 us less, rank 32 up to 5, rank 3
+// with one column 2 us more (there a lane adds up 85 others' sums); 500 x 401, rank
+// 16, 2 columns: 4 to 6 us more.  Dynamic LDS: k * nrhs values.
 constexpr int kLrFused = 4096;
 
 template <typename V, int NT>
