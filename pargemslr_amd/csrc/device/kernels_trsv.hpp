@@ -817,7 +817,7 @@ __device__ __forceinline__ void ring_solve_sweep(int h, int g, int nsteps, int r
 // pos: per block b the boundaries of its steps (blk_step[b + 1] - blk_step[b] + 1
 // values from blk_step[b] + b; the first of them is 0, sU's the block's
 // rows).  info, dinv: per position the pair (ring slot times sizeof(V),
-// block-local row id) from blk_ri0[b] + b, the dummy row's pair after the block's
+// block-local row id) from ring_info0, the dummy row's pair after the block's
 // own, and 1/pivot from blk_ri0[b]; ent: the block's records, from blk_ri0[b] *
 // ring_row_bytes<V>().
 template <typename V, int K, int CG, int NG, int NH>
@@ -836,7 +836,7 @@ __global__ __launch_bounds__(64 * (NH * NG + NH + 1)) void k_trsv_ring(
   const int64_t vbytes = (int64_t)nb * nrhs * (int64_t)sizeof(V);
   V* xb = x + (int64_t)r0 * nrhs;
   const __amdgpu_buffer_rsrc_t rs_x = make_rsrc(xb, vbytes);
-  const __amdgpu_buffer_rsrc_t rs_info = make_rsrc(info + q0 + b, (np + 1) * 8);
+  const __amdgpu_buffer_rsrc_t rs_info = make_rsrc(info + ring_info0(q0, b), (np + 1) * 8);
   // rings, dummy rows and stages start as zeros: a record that is not there reads
   // slot 0 with weight zero
   uint4* lds4 = reinterpret_cast<uint4*>(smem_raw);

@@ -57,6 +57,12 @@ struct RingInfo {
   int slot, row;
 };
 
+// Index of a block's first pair, ri0 its first position: the blocks' pairs lie two
+// apart.  A block has an even number of positions, so that each block's pairs start
+// at a multiple of 16 bytes (one pair apart, an apply at 1023x1021 x 8 columns took
+// 1436 us, like this 1427 to 1430).
+constexpr int64_t ring_info0(int64_t ri0, int64_t b) { return ri0 + 2 * b; }
+
 // Byte of entry j of row t in a group of n rows: its value's and its slot's.
 template <typename V>
 void ring_entry_bytes(int n, int t, int j, int& value, int& slot) {
@@ -89,7 +95,7 @@ struct RingPack {
   std::vector<int> pos_h, step_h, stepU_h;
   int64_t max_block_steps = 0, max_block_steps_h = 0;
   std::vector<unsigned char> rec;       // records, ring_row_bytes<V>() per position
-  std::vector<RingInfo> info;           // per position, and the dummy row's after a block's last
+  std::vector<RingInfo> info;           // per position, and two of the dummy row after a block's last
 };
 
 // Step boundaries of every block from the step descriptors (4 per step, the
@@ -130,15 +136,14 @@ RingPack<V> ring_pack(const TrsvPack<T>& P, F val) {
   constexpr int RB = ring_row_bytes<V>();
   const int64_t nr = (int64_t)P.rows.size();
   R.rec.resize((size_t)nr * RB);
-  R.info.resize((size_t)nr + P.nblocks);
+  R.info.resize((size_t)ring_info0(nr, P.nblocks), RingInfo{wn * (int)sizeof(V), kRingDummyRow});
   parallel_for(P.nblocks, [&](int b) {
-    R.info[P.blk_ri0[b + 1] + b] = RingInfo{wn * (int)sizeof(V), kRingDummyRow};
     for (int s = P.blk_step[b]; s < P.blk_step[b + 1]; ++s) {
       const int* d4 = &P.desc[4 * (size_t)s];
       const int end = d4[0] + d4[2];  // a row the step reads is at most W positions before it
       for (int t = 0; t < d4[2]; ++t) {
         const int64_t q = P.blk_ri0[b] + d4[0] + t;
-        R.info[q + b] = RingInfo{(d4[0] + t) % wn * (int)sizeof(V), P.rows[q]};
+        R.info[ring_info0(q, b)] = RingInfo{(d4[0] + t) % wn * (int)sizeof(V), P.rows[q]};
         const int t0 = t / kRingGroup * kRingGroup;  // first row of t's group
         unsigned char* g = R.rec.data() + (P.blk_ri0[b] + d4[0] + t0) * RB;
         for (int j = 0; j < d4[3]; ++j) {

@@ -168,9 +168,9 @@ bool check_op(const std::string& name, const HostOp<T>& op, int shorter) {
       block_solve(L.ilu[b], rhs.data() + r0, ref.data() + r0);
       // lanes past a step's rows take the dummy row's pair, right after the block's own
       const int64_t np = P.blk_ri0[b + 1] - P.blk_ri0[b];
-      const RingInfo* info = R.info.data() + P.blk_ri0[b] + b;
-      if (info[np].slot != R.rows * (int)sizeof(V) || info[np].row != kRingDummyRow) {
-        std::printf("%s, level %d, block %d: no dummy pair MISMATCH\n", name.c_str(), l, b);
+      const RingInfo* info = R.info.data() + ring_info0(P.blk_ri0[b], b);
+      if (info[np].slot != R.rows * (int)sizeof(V) || info[np].row != kRingDummyRow || (info - R.info.data()) % 2) {
+        std::printf("%s, level %d, block %d: no dummy pair, or pairs not aligned MISMATCH\n", name.c_str(), l, b);
         ok = false;
       }
       for (int k = 0; k < 8; ++k) {
